@@ -349,8 +349,8 @@ int aar_hip_set_option(const char *name, long value);
 
 /* Per-kernel GPU timing with hipEvents (off by default).  Kernel names:
  * "stencil_matvec", "stencil_aar_true", "stencil_aar_rec", "stencil_resid",
- * "stencil_pgr_rich", "stencil_cg_q", "stencil_cg_resid", "stencil_matvec_res",
- * "gram", "ls", "anchor_update", "fold", "dot", "pgr_update", "cg_update". */
+ * "stencil_pgr_rich", "stencil_cg_q", "stencil_cg_resid",
+ * "gram", "ls", "anchor_update", "fold", "dot", "pgr_update", "cg_dir", "cg_update". */
 int aar_hip_profile(int enable);
 int aar_hip_profile_reset(void);
 int aar_hip_profile_query(const char *name, int *count, double *total_ms, double *bytes);

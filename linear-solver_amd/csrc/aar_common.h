@@ -34,7 +34,7 @@ struct Ctrl {
     int done;          // 1: stop (converged or zero-iteration exit)
     int final_iter;    // iteration count reported when done was set
     int status;        // 0 ok, 1 SVD did not converge, 2 non-finite residual
-    int pad0;
+    int xpend;         // CG: x += alpha d of the last iteration not yet applied
     double rhs_norm;   // ||b||
     double tol_abs;    // tol * ||b||
     double relres;     // last checked ||b - A x|| (absolute)
@@ -54,7 +54,8 @@ enum Fin : int {
     FIN_NORM_B = 3,     // ctrl->rhs_norm = sqrt(sum_0), tol_abs = tol * rhs_norm
     FIN_PGR_RES = 4,    // like FIN_AAR_RES for the post-projection residual of PGR/PL2R
     FIN_CG_ALPHA = 5,   // alpha = delta_new / sum_0
-    FIN_CG_BETA = 6,    // delta_old = delta_new; delta_new = sum_0; relres = sqrt(sum_1); beta; check
+    FIN_CG_BETA = 6,    // delta_old = delta_new; delta_new = sum_0; relres = sqrt(sum_1); beta; check;
+                        // xpend = fin.check (the iteration's x += alpha d is still to come)
 };
 
 struct FinArgs {

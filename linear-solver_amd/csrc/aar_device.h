@@ -187,6 +187,7 @@ __device__ inline void finalize(const FinArgs &f, Ctrl *c, const double *sums, i
         const double rr = sqrt(sums[1]);     // CG.c:137
         c->relres = rr;
         c->beta = c->delta_new / c->delta_old;  // CG.c:148
+        c->xpend = f.check;
         if (f.hist && f.it >= 0 && f.it < f.hist_cap) f.hist[f.it] = rr;
         if (!(rr == rr)) {
             c->status = 2;

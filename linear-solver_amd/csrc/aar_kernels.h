@@ -9,10 +9,9 @@ enum class SMode : int {
     MATVEC = 0,    // y = a*Lap(x) + sigma*x                      (system.c:189-205)
     AAR_TRUE = 1,  // r = b - A x; g = r/diag (T or FP32 out); ||r||^2 (AAR.c:80-82,119-123)
     RESID = 2,     // r = b - A x (+ optional fp32 copy), ||r||^2
-    PGR_RICH = 3,  // u = x + omega (b - Ax)/diag; Au = A u        (PGR.c:92-103)
-    CG_Q = 4,      // d = s + beta d (s = r/diag); q = A d; d.q   (CG.c:94-100,148-150)
+    PGR_STEP = 3,  // Ax = A x; x_next = x + omega (b - Ax)/diag; ||b - Ax||^2 (PGR.c:92-103)
+    CG_Q = 4,      // q = A d; d.q                                (CG.c:94-100)
     CG_RESID = 5,  // r = b - A x; r.s, r.r                        (CG.c:65-84,112-137)
-    MATVEC_RES = 6,  // y = A x and ||b - A x||^2                  (PGR.c:79-81)
     AAR_REC = 7,   // g' = g - (omega/diag) A g: the residual of x + omega g (AAR.c:134-139)
 };
 
@@ -28,40 +27,48 @@ struct SArgs {
     double omega = 0.0;
     int precond = 1;
     int trace = 0;
-    int cg_first = 0;
-    const T *in0 = nullptr, *in1 = nullptr, *in2 = nullptr;   // stencil operand fields
+    const T *in0 = nullptr;           // stencil operand
     const T *bvec = nullptr;          // right-hand side for the epilogue
     // variable-coefficient operator A = a*Lap + c(x) (the VC sweeps only):
-    // MATVEC/AAR_TRUE read c(x); AAR_REC reads h(x) = omega/(diag + c(x))
+    // the sweeps read c(x); AAR_REC reads h(x) = omega/(diag + c(x))
     // with a Jacobi preconditioner, else c(x)
     const T *vf = nullptr;
     T *out0 = nullptr, *out1 = nullptr;
     float *out32 = nullptr;
-    const double *cg_beta = nullptr;
     double *partials = nullptr;       // [nitems * NACC]
-    unsigned *counter = nullptr;
     Ctrl *ctrl = nullptr;
     FinArgs fin = {};
 };
 
-// wy: wavefronts per block stacked in y (4 or 8); py: rows per thread (2 or 4)
+// Launch shape of the sweeps: tile = 0: the z-march (stencil_body.h), a block
+// owning a 64 x (wy*py) column over lz planes; tile > 0: the one-shot boxes of
+// stencil_tile.h, `tile` (1, 2 or 4) planes deep.
+struct Shape {
+    int lz = 0, wy = 8, py = 4;
+    int tile = 0;
+    double us = 0.0;          // measured time of one recurrence sweep (tuned shapes)
+};
+
 template <typename T>
-hipError_t launch_stencil(SMode m, const SArgs<T> &a, int wy, int py, hipStream_t st);
+hipError_t launch_stencil(SMode m, const SArgs<T> &a, const Shape &sh, hipStream_t st);
+// blocks (= partials per sum) of the sweep
 template <typename T>
-int stencil_items(const SArgs<T> &a, int wy, int py);
-// the variable-coefficient sweeps (MATVEC, AAR_TRUE, AAR_REC with a.vf set)
+int stencil_items(const SArgs<T> &a, const Shape &sh);
+// fills the tile geometry of `a` (nxy, ntx, nty, nzc, nitems; lz clamped)
 template <typename T>
-hipError_t launch_stencil_vc(SMode m, const SArgs<T> &a, int wy, int py, hipStream_t st);
+void stencil_geometry(SArgs<T> &a, const Shape &sh);
+// planes of the one-shot boxes on this grid, or 0 where the march is faster
+template <typename T>
+int stencil_tile_planes(int nx, int ny, int nz);
+// the variable-coefficient sweeps (a.vf set)
+template <typename T>
+hipError_t launch_stencil_vc(SMode m, const SArgs<T> &a, const Shape &sh, hipStream_t st);
 // h = omega/(diag + c) (precond) or c, rounded to Tg
 template <typename Tg>
 hipError_t launch_vc_field(long n, const double *c, double diag, double omega, int precond, Tg *h,
                            hipStream_t st);
 // r /= (diag + c), pointwise
 hipError_t launch_div_vc(double *r, double diag, const double *c, long n, hipStream_t st);
-// fills the tile geometry of `a` (nxy, ntx, nty, nzc, nitems; lz clamped)
-template <typename T>
-void stencil_geometry(SArgs<T> &a, int wy, int py);
-
 // ---------------------------------------------------------------------------
 // history sweeps
 // ---------------------------------------------------------------------------
@@ -164,8 +171,9 @@ struct AncArgs {
 template <typename Tx, typename Tg>
 hipError_t launch_anchor_update(const AncArgs<Tx, Tg> &a, hipStream_t st);
 
-// PGR.c:117-130: x += sum DX s; Ax += sum DF s (in place at slot `cur`,
-// the age-0 slot), ||b - Ax||^2 -> FIN_PGR_RES.
+// PGR.c:117-130: x += sum DX s; Ax += sum DF s (in place at the age-0 slot),
+// ||b - Ax||^2 -> FIN_PGR_RES, and the Richardson step from there
+// (PGR.c:92-98): slot `next` of X = x + omega (b - Ax)/diag.
 template <typename T>
 struct PUpdArgs {
     long n = 0;
@@ -174,6 +182,10 @@ struct PUpdArgs {
     const T *b = nullptr;
     long ld = 0;
     int slot[MAXM + 1] = {};
+    int next = -1;            // X slot of the next iterate, or -1
+    double omega = 0.0, diag = 1.0;
+    const T *c = nullptr;     // variable coefficient: divisor diag + c(x)
+    int precond = 1;
     int nvalid = 0;
     int it = 0;
     int nblocks = 0;
@@ -202,24 +214,31 @@ struct DotArgs {
 template <typename T>
 hipError_t launch_dot(const DotArgs<T> &a, hipStream_t st);
 
-// CG.c:106-126: x += alpha d; r -= alpha q; partials r.(r/diag), r.r
-struct CgUpdArgs {
+// The pointwise steps of CG (CG.c:106-150); the divisor of the Jacobi step
+// is diag, or diag + c(x).
+enum class CgStep : int {
+    DIR = 0,     // s = r/diag; d = s + beta d, and first, when x is given, the
+                 // x += alpha d that the previous iteration left pending
+    RES = 1,     // r -= alpha q; partials r.(r/diag), r.r
+    X = 2,       // x += alpha d
+    X_PENDING = 3,   // the same if ctrl says an iteration left it pending
+};
+struct CgArgs {
     long n = 0;
-    double *x = nullptr, *r = nullptr;
-    const double *d = nullptr, *q = nullptr;
+    double *x = nullptr, *r = nullptr, *d = nullptr;
+    const double *q = nullptr;
     double diag = 1.0;
-    const double *c = nullptr;  // variable coefficient: divisor diag + c(x)
+    const double *c = nullptr;
     int precond = 1;
-    int update_r = 1;          // 0 on restart iterations (r recomputed by a stencil pass)
     int nblocks = 0;
     double *partials = nullptr;
     unsigned *counter = nullptr;
     Ctrl *ctrl = nullptr;
     FinArgs fin = {};
 };
-hipError_t launch_cg_update(const CgUpdArgs &a, hipStream_t st);
-// grid (= number of partial pairs) of the CG update on n points
-int cg_update_blocks(long n);
+hipError_t launch_cg(CgStep step, const CgArgs &a, hipStream_t st);
+// grid (= number of partial pairs) of the CG steps on n points
+int cg_blocks(long n);
 
 // ---------------------------------------------------------------------------
 // complex Helmholtz (no MPI_REAL counterpart): A u = a*Lap(u) + (c(x) + i eta) u,

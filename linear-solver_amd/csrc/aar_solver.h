@@ -25,12 +25,6 @@ struct ProfEntry {
     double bytes = 0.0;
 };
 
-// launch shape of the stencil sweeps for one grid and element size
-struct Shape {
-    int lz = 0, wy = 8, py = 4;
-    double us = 0.0;          // measured time of one recurrence sweep (tuned shapes)
-};
-
 struct PendingEv {
     std::string name;
     hipEvent_t a = nullptr, b = nullptr;

@@ -29,7 +29,7 @@ namespace aar {
 
 namespace {
 
-constexpr int BWY = 8, BPY = 4;        // launch shape of the batched stencils
+constexpr int BWY = 8, BPY = 4;        // launch shape of the batched stencils (64 x 32 columns)
 constexpr int CHUNK = 4096;            // elements per block of the streaming kernels
 
 template <typename Tx, typename Tg>
@@ -90,9 +90,7 @@ __global__ __launch_bounds__(64 * BWY) void bstencil_kernel(const BInst<Tx, Tg> 
         }
     }
     __syncthreads();
-    // FP32 with the plain index keeps the sweep within 128 VGPRs (two
-    // blocks per CU with the batch's per-block argument staging)
-    stencil_body<T, BWY, BPY, MODE, sizeof(T) == 4 ? 0 : -1>(sa, wi.idx);
+    stencil_body<T, BWY, BPY / Lane<T>::RPW, MODE>(sa, wi.idx);
 }
 
 // per-instance finish of the true residual: relres check at the Anderson
@@ -413,9 +411,9 @@ int batch_solve(const aar_hip_instance *ins, int count, double omega, double bet
         tr.lz = batch_lz(sizeof(Tx));
         SArgs<Tg> rcg = base_sargs<Tg>(op);
         rcg.lz = batch_lz(sizeof(Tg));
-        const int ntr = stencil_items<Tx>(tr, BWY, BPY), nrc = stencil_items<Tg>(rcg, BWY, BPY);
-        stencil_geometry<Tx>(tr, BWY, BPY);
-        stencil_geometry<Tg>(rcg, BWY, BPY);
+        const int ntr = stencil_items<Tx>(tr, Shape{}), nrc = stencil_items<Tg>(rcg, Shape{});
+        stencil_geometry<Tx>(tr, Shape{});
+        stencil_geometry<Tg>(rcg, Shape{});
         tr.omega = rcg.omega = omega;
         tr.precond = rcg.precond = precond;
         {
@@ -507,13 +505,12 @@ int batch_solve(const aar_hip_instance *ins, int count, double omega, double bet
             Tg *o = I.G + (size_t)(1 % S) * I.ld;
             if constexpr (sizeof(Tx) == sizeof(Tg)) a.out0 = (Tx *)o;
             else a.out32 = (float *)o;
-            a.counter = nullptr;
             a.fin.fin = FIN_AAR_RES;
             a.fin.it = 1;
             a.fin.check = 0;
             a.fin.hist = I.hist;
             a.fin.hist_cap = I.hist_cap;
-            BHC(launch_stencil<Tx>(SMode::AAR_TRUE, a, BWY, BPY, st));
+            BHC(launch_stencil<Tx>(SMode::AAR_TRUE, a, Shape{}, st));
             BHC(launch_finish(a.partials, I.tr_items, 1, a.fin, a.ctrl, st));
         }
         if (p == 1 && max_iter >= 1) {       // iteration 1 is never an Anderson step (AAR.c:109)

@@ -176,7 +176,13 @@ Shape stencil_shape(int nx, int ny, int nz, size_t es)
     Shape sh;
     sh.wy = C.wy;
     sh.py = C.py;
-    sh.lz = C.lz > 0 ? C.lz : auto_lz(op, C.wy, C.py, es);
+    if (!C.tuning_set) {
+        sh.tile = es == 4 ? stencil_tile_planes<float>(nx, ny, nz) : stencil_tile_planes<double>(nx, ny, nz);
+        // FP32 march: 64 x 16 columns of four wavefronts, two blocks a CU
+        // (512^3 recurrence 230 us; 64 x 32 of eight 246, 64 x 64 233)
+        if (es == 4) sh.wy = 4;
+    }
+    sh.lz = C.lz > 0 ? C.lz : auto_lz(op, sh.wy, sh.py, es);
     return sh;
 }
 
@@ -278,29 +284,27 @@ static const char *smode_name(SMode m)
     case SMode::AAR_TRUE: return "stencil_aar_true";
     case SMode::AAR_REC: return "stencil_aar_rec";
     case SMode::RESID: return "stencil_resid";
-    case SMode::PGR_RICH: return "stencil_pgr_rich";
+    case SMode::PGR_STEP: return "stencil_pgr_rich";
     case SMode::CG_Q: return "stencil_cg_q";
     case SMode::CG_RESID: return "stencil_cg_resid";
-    case SMode::MATVEC_RES: return "stencil_matvec_res";
     }
     return "stencil";
 }
 
-// Reductions either finish in the last block of the reducing kernel
-// (counter + device-scope fence) or, in two-pass mode, in a one-block
-// second kernel; the choice is a measured tuning option.
+// The history reductions either finish in the last block of the reducing
+// kernel (counter + device-scope fence) or, in two-pass mode, in a one-block
+// second kernel; the choice is a measured tuning option.  The stencil sweeps
+// always finish in a second kernel.
 template <typename T>
 int run_stencil(SMode mode, SArgs<T> a, double bytes)
 {
     Context &C = ctx();
-    const bool two = C.two_pass && a.partials;
-    if (two) a.counter = nullptr;
     const Shape sh = stencil_shape(a.nx, a.ny, a.nz, sizeof(T));
     prof_begin(smode_name(mode));
-    hipError_t e = launch_stencil<T>(mode, a, sh.wy, sh.py, C.stream);
+    hipError_t e = launch_stencil<T>(mode, a, sh, C.stream);
     prof_end(bytes);
-    if (two && e == hipSuccess)
-        e = launch_finish(a.partials, stencil_items<T>(a, sh.wy, sh.py), mode == SMode::CG_RESID ? 2 : 1, a.fin,
+    if (a.partials && e == hipSuccess)
+        e = launch_finish(a.partials, stencil_items<T>(a, sh), mode == SMode::CG_RESID ? 2 : 1, a.fin,
                           a.ctrl, C.stream);
     if (e != hipSuccess) return fail(AAR_HIP_ERR_HIP, std::string("stencil launch: ") + hipGetErrorString(e));
     C.bytes_acc += bytes;
@@ -335,12 +339,12 @@ static hipError_t run_pgr_update(PUpdArgs<double> u)
     return e;
 }
 
-static hipError_t run_cg_update(CgUpdArgs u)
+static hipError_t run_cg_res(CgArgs u)
 {
     Context &C = ctx();
-    const bool two = C.two_pass && u.update_r;
+    const bool two = C.two_pass;
     if (two) u.counter = nullptr;
-    hipError_t e = launch_cg_update(u, C.stream);
+    hipError_t e = launch_cg(CgStep::RES, u, C.stream);
     if (two && e == hipSuccess) e = launch_finish(u.partials, u.nblocks, 2, u.fin, u.ctrl, C.stream);
     return e;
 }
@@ -350,15 +354,17 @@ int stencil_partials_needed(const Op &op)
 {
     SArgs<T> a = base_sargs<T>(op);
     const Shape sh = stencil_shape(op.nx, op.ny, op.nz, sizeof(T));
-    return stencil_items<T>(a, sh.wy, sh.py) * 2;
+    return stencil_items<T>(a, sh) * 2;
 }
 
 // ---------------------------------------------------------------------------
 // Autotuner: times the recurrence sweep (the dominant kernel of AAR) on the
-// grid over the launch shapes -- wavefronts per block x rows per thread
-// (the tile height; tiles are one wavefront = 64 points wide in x) and the
-// z-slab depth -- and keeps the fastest.  batch_shape restricts the search
-// to the slab depth of the batched 8 x 4 launch.
+// grid over the launch shapes of the march -- wavefronts per block x rows
+// (the tile height; tiles are 64 points wide in x) and the z-slab depth --
+// and keeps the fastest; the one-shot boxes, where the grid may take them,
+// are timed too and kept instead when they beat it (the shape reported stays
+// the best march).  batch_shape restricts the search to the slab depth of the
+// batched 8 x 4 launch.
 // ---------------------------------------------------------------------------
 template <typename T>
 static int autotune_t(int nx, int ny, int nz, bool batch_shape, Shape *out)
@@ -384,6 +390,30 @@ static int autotune_t(int nx, int ny, int nz, bool batch_shape, Shape *out)
     (void)hipEventCreate(&e0);
     (void)hipEventCreate(&e1);
     int rc = 0;
+    auto time_shape = [&](Shape &sh) -> int {
+        SArgs<T> a;
+        a.nx = nx;
+        a.ny = ny;
+        a.nz = nz;
+        a.lz = sh.lz;
+        for (int q = 0; q <= R; q++) {
+            a.w[q] = op.w[q];
+            a.cf[q] = q == 0 ? 0.5 : -1e-3 * op.w[q];
+        }
+        a.in0 = in;
+        a.out0 = o;
+        hipError_t e = launch_stencil<T>(SMode::AAR_REC, a, sh, C.stream);
+        const int reps = 4;
+        e = e == hipSuccess ? hipEventRecord(e0, C.stream) : e;
+        for (int r = 0; r < reps && e == hipSuccess; r++) e = launch_stencil<T>(SMode::AAR_REC, a, sh, C.stream);
+        e = e == hipSuccess ? hipEventRecord(e1, C.stream) : e;
+        e = e == hipSuccess ? hipEventSynchronize(e1) : e;
+        float ms = 0.f;
+        e = e == hipSuccess ? hipEventElapsedTime(&ms, e0, e1) : e;
+        if (e != hipSuccess) return fail(AAR_HIP_ERR_HIP, std::string("autotune: ") + hipGetErrorString(e));
+        sh.us = 1e3 * ms / reps;
+        return 0;
+    };
     for (int si = 0; si < nshape && !rc; si++) {
         const int wy = shapes[si][0], py = shapes[si][1];
         std::vector<int> lzs = {auto_lz(op, wy, py, sizeof(T)), nz, (nz + 1) / 2, (nz + 3) / 4, (nz + 7) / 8};
@@ -391,37 +421,18 @@ static int autotune_t(int nx, int ny, int nz, bool batch_shape, Shape *out)
         lzs.erase(std::unique(lzs.begin(), lzs.end()), lzs.end());
         for (int lz : lzs) {
             if (lz < std::min(nz, 16)) continue;
-            SArgs<T> a;
-            a.nx = nx;
-            a.ny = ny;
-            a.nz = nz;
-            a.lz = lz;
-            for (int q = 0; q <= R; q++) {
-                a.w[q] = op.w[q];
-                a.cf[q] = q == 0 ? 0.5 : -1e-3 * op.w[q];
-            }
-            a.in0 = in;
-            a.out0 = o;
-            hipError_t e = launch_stencil<T>(SMode::AAR_REC, a, wy, py, C.stream);
-            const int reps = 4;
-            e = e == hipSuccess ? hipEventRecord(e0, C.stream) : e;
-            for (int r = 0; r < reps && e == hipSuccess; r++) e = launch_stencil<T>(SMode::AAR_REC, a, wy, py, C.stream);
-            e = e == hipSuccess ? hipEventRecord(e1, C.stream) : e;
-            e = e == hipSuccess ? hipEventSynchronize(e1) : e;
-            float ms = 0.f;
-            e = e == hipSuccess ? hipEventElapsedTime(&ms, e0, e1) : e;
-            if (e != hipSuccess) {
-                rc = fail(AAR_HIP_ERR_HIP, std::string("autotune: ") + hipGetErrorString(e));
-                break;
-            }
-            const double us = 1e3 * ms / reps;
-            if (us < best.us) {
-                best.us = us;
-                best.lz = lz;
-                best.wy = wy;
-                best.py = py;
-            }
+            Shape sh;
+            sh.lz = lz;
+            sh.wy = wy;
+            sh.py = py;
+            if ((rc = time_shape(sh))) break;
+            if (sh.us < best.us) best = sh;
         }
+    }
+    if (!rc && !batch_shape) {
+        Shape sh = best;
+        sh.tile = stencil_tile_planes<T>(nx, ny, nz);
+        if (sh.tile && !(rc = time_shape(sh)) && sh.us < best.us) best.tile = sh.tile;
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
@@ -578,7 +589,6 @@ int aar_rec(const Op &op, Tx *x, const Tx *b, double omega, double beta, int m, 
         if constexpr (sizeof(Tx) == sizeof(Tg)) a.out0 = (Tx *)gptr(k);
         else a.out32 = (float *)gptr(k);
         a.partials = part;
-        a.counter = cnt + 1;
         a.ctrl = ctrl;
         a.fin.fin = FIN_AAR_RES;
         a.fin.it = (int)k;
@@ -637,7 +647,6 @@ int aar_rec(const Op &op, Tx *x, const Tx *b, double omega, double beta, int m, 
             a.out0 = gptr(it + 1);
             a.trace = 1;
             a.partials = part;
-            a.counter = cnt + 1;
             a.ctrl = ctrl;
             a.fin.fin = FIN_AAR_RES;
             a.fin.it = (int)it + 1;
@@ -842,45 +851,34 @@ int pgr_solve(const Op &op, double *x, const double *b, double omega, int m, int
         d.fin.check = 1;
         HC(run_dot<double>(d));
     }
-    // Ax_1 and ||b - A x_1|| (PGR.c:79-81)
-    {
-        SArgs<double> a = base_sargs<double>(op);
-        a.in0 = X + (size_t)slot(1) * ld;
-        a.bvec = b;
-        a.out0 = Y + (size_t)slot(1) * ld;
-        a.partials = part;
-        a.counter = cnt + 1;
-        a.ctrl = ctrl;
-        a.fin.fin = FIN_AAR_RES;
-        a.fin.it = 1;
-        a.fin.check = 0;
-        a.fin.hist = hist;
-        a.fin.hist_cap = max_iter + 4;
-        if (int rc = run_stencil<double>(SMode::MATVEC_RES, a, s_b * 3 + vcb)) return rc;
-    }
-    int cyc = 0;
-    int t = 1;
-    bool stopped = false;
-    for (; t <= max_iter && !stopped; t++) {
+    // Ax_{t+1}, ||b - A x_{t+1}|| and the next iterate x_{t+2} = x_{t+1} +
+    // omega f (PGR.c:92-103): pointwise once A x_{t+1} is known, so the sweep
+    // that makes it reads one field.  No next iterate where a projection will
+    // change x_{t+1} (its update writes the next one) or the solve ends.
+    auto step = [&](int t) -> int {
+        const bool next = t < max_iter && !(t >= 1 && t % p == 0);
         SArgs<double> a = base_sargs<double>(op);
         a.omega = omega;
         a.precond = precond;
-        a.in0 = X + (size_t)slot(t) * ld;
-        a.in1 = b;
-        a.in2 = Y + (size_t)slot(t) * ld;
+        a.in0 = X + (size_t)slot(t + 1) * ld;
         a.bvec = b;
-        a.out0 = X + (size_t)slot(t + 1) * ld;
-        a.out1 = Y + (size_t)slot(t + 1) * ld;
-        a.trace = 1;
+        a.out0 = Y + (size_t)slot(t + 1) * ld;
+        a.out1 = next ? X + (size_t)slot(t + 2) * ld : nullptr;
         a.partials = part;
-        a.counter = cnt + 1;
         a.ctrl = ctrl;
         a.fin.fin = FIN_AAR_RES;
         a.fin.it = t + 1;
         a.fin.check = 0;
         a.fin.hist = hist;
         a.fin.hist_cap = max_iter + 4;
-        if (int rc = run_stencil<double>(SMode::PGR_RICH, a, s_b * 5 + 2 * vcb)) return rc;
+        return run_stencil<double>(SMode::PGR_STEP, a, s_b * (next ? 4 : 3) + vcb);
+    };
+    if (int rc = step(0)) return rc;                                // PGR.c:79-81
+    int cyc = 0;
+    int t = 1;
+    bool stopped = false;
+    for (; t <= max_iter && !stopped; t++) {
+        if (int rc = step(t)) return rc;
         if (t % p == 0) {                                           // PGR.c:111
             // history by age relative to the newest iterate x_{t+1}: the
             // column of age k belongs to iteration t-k (PGR.c:105-109)
@@ -912,6 +910,11 @@ int pgr_solve(const Op &op, double *x, const double *b, double omega, int m, int
             u.Y = Y;
             u.b = b;
             u.ld = ld;
+            u.next = t < max_iter ? slot(t + 2) : -1;
+            u.omega = omega;
+            u.diag = op.diag;
+            u.c = op.c;
+            u.precond = precond;
             u.nblocks = pgr_update_blocks(n, m, nb);
             if ((size_t)u.nblocks > need) return fail(AAR_HIP_ERR_ARG, "PGR: grid too large for the partials");
             u.partials = part;
@@ -923,8 +926,9 @@ int pgr_solve(const Op &op, double *x, const double *b, double omega, int m, int
             u.fin.hist = nullptr;
             prof_begin("pgr_update");
             HC(run_pgr_update(u));
-            prof_end(s_b * (2 * (nv + 1) + 1 + 2));
-            C.bytes_acc += s_b * ((l2 ? 1 : 2) * (nv + 1) + 1) + s_b * (2 * (nv + 1) + 3);
+            const double by = s_b * (2 * (nv + 1) + 3 + (u.next >= 0 ? 1 : 0)) + (u.next >= 0 ? vcb : 0.0);
+            prof_end(by);
+            C.bytes_acc += s_b * ((l2 ? 1 : 2) * (nv + 1) + 1) + by;
             if (int rc = poll_record(ctrl, cyc)) return rc;
             if (poll_check(cyc - 2)) stopped = true;
             cyc++;
@@ -966,14 +970,14 @@ int cg_solve(const Op &op, double *x, const double *b, int max_iter, double tol,
     if (!x || !b) return fail(AAR_HIP_ERR_ARG, "null vector");
     if (max_iter < 0) return fail(AAR_HIP_ERR_ARG, "max_iter must be >= 0");
     const long n = op.n;
-    // r, d[2], q (padded slots, as the rings)
+    // r, d, q (padded slots, as the rings)
     const long ld = ring_ld(n, sizeof(double));
-    HC(ensure(C.ring64x, sizeof(double) * ld * 4));
+    HC(ensure(C.ring64x, sizeof(double) * ld * 3));
     HC(ensure(C.hist0, sizeof(double) * (size_t)(max_iter + 4)));
     const int nb = nblocks_for(n);
     const size_t need = std::max<size_t>((size_t)stencil_partials_needed<double>(op), (size_t)nb * GRAM_NA_MAX);
     HC(ensure(C.part0, sizeof(double) * need));
-    double *r = (double *)C.ring64x.p, *dd[2] = {r + ld, r + 2 * ld}, *q = r + 3 * ld;
+    double *r = (double *)C.ring64x.p, *dv = r + ld, *q = r + 2 * ld;
     double *hist = (double *)C.hist0.p, *part = (double *)C.part0.p;
     Ctrl *ctrl = C.ctrl;
     unsigned *cnt = C.counters;
@@ -1002,9 +1006,8 @@ int cg_solve(const Op &op, double *x, const double *b, int max_iter, double tol,
         a.in0 = x;
         a.bvec = b;
         a.out0 = r;
-        a.out1 = dd[0];
+        a.out1 = dv;
         a.partials = part;
-        a.counter = cnt + 1;
         a.ctrl = ctrl;
         a.fin.fin = FIN_CG_BETA;
         a.fin.it = 0;
@@ -1012,52 +1015,59 @@ int cg_solve(const Op &op, double *x, const double *b, int max_iter, double tol,
         a.fin.hist_cap = max_iter + 4;
         if (int rc = run_stencil<double>(SMode::CG_RESID, a, s_b * 4 + vcb)) return rc;
     }
+    // Iteration k: d = r/diag + beta d (and the x += alpha d of iteration k-1,
+    // CG.c:106-107), q = A d with d.q, r -= alpha q with r.s and r.r.  The x
+    // update rides on the next direction step, which reads d anyway, so the
+    // sweep reads one field and an iteration moves 10 vectors.  Every 50th
+    // iteration (CG.c:109) updates x at once and recomputes r = b - A x.
+    CgArgs u;
+    u.n = n;
+    u.r = r;
+    u.d = dv;
+    u.q = q;
+    u.diag = op.diag;
+    u.c = op.c;
+    u.precond = precond;
+    u.nblocks = cg_blocks(n);
+    if ((size_t)u.nblocks * 2 > need) return fail(AAR_HIP_ERR_ARG, "CG: grid too large for the partials");
+    u.partials = part;
+    u.counter = cnt + 3;
+    u.ctrl = ctrl;
+    u.fin.fin = FIN_CG_BETA;
+    u.fin.hist = hist;
+    u.fin.hist_cap = max_iter + 4;
     int k = 0;
     bool stopped = false;
+    bool pending = false;      // iteration k-1 left its x update to come
     int cyc = 0;
     for (; k < max_iter && !stopped; k++) {
-        const int cur = (k + 1) & 1, old = k & 1;
+        if (k > 0) {
+            u.x = pending ? x : nullptr;
+            const double by = s_b * (pending ? 5 : 3) + vcb;
+            prof_begin("cg_dir");
+            HC(launch_cg(CgStep::DIR, u, C.stream));
+            prof_end(by);
+            C.bytes_acc += by;
+        }
         {
             SArgs<double> a = base_sargs<double>(op);
-            a.precond = precond;
-            a.cg_first = (k == 0);
-            a.cg_beta = &ctrl->beta;
-            a.in0 = r;
-            a.in1 = dd[old];
-            a.out0 = dd[cur];
-            a.out1 = q;
+            a.in0 = dv;
+            a.out0 = q;
             a.partials = part;
-            a.counter = cnt + 2;
             a.ctrl = ctrl;
             a.fin.fin = FIN_CG_ALPHA;
-            if (int rc = run_stencil<double>(SMode::CG_Q, a, s_b * 4 + 2 * vcb)) return rc;
+            if (int rc = run_stencil<double>(SMode::CG_Q, a, s_b * 2 + vcb)) return rc;
         }
         const bool restart = (k % 50) == 0;                          // CG.c:109
-        {
-            CgUpdArgs u;
-            u.n = n;
-            u.x = x;
-            u.r = r;
-            u.d = dd[cur];
-            u.q = q;
-            u.diag = op.diag;
-            u.c = op.c;
-            u.precond = precond;
-            u.update_r = restart ? 0 : 1;
-            u.nblocks = cg_update_blocks(n);
-            if ((size_t)u.nblocks * 2 > need) return fail(AAR_HIP_ERR_ARG, "CG: grid too large for the partials");
-            u.partials = part;
-            u.counter = cnt + 3;
-            u.ctrl = ctrl;
-            u.fin.fin = FIN_CG_BETA;
-            u.fin.it = k + 1;
-            u.fin.hist = hist;
-            u.fin.hist_cap = max_iter + 4;
-            prof_begin("cg_update");
-            HC(run_cg_update(u));
-            prof_end(s_b * (restart ? 3 : 6) + (restart ? 0 : vcb));
-            C.bytes_acc += s_b * (restart ? 3 : 6) + (restart ? 0 : vcb);
-        }
+        pending = !restart;
+        prof_begin("cg_update");
+        u.x = x;
+        u.fin.it = k + 1;
+        u.fin.check = 1;
+        if (restart) HC(launch_cg(CgStep::X, u, C.stream));
+        else HC(run_cg_res(u));
+        prof_end(s_b * 3 + (restart ? 0 : vcb));
+        C.bytes_acc += s_b * 3 + (restart ? 0 : vcb);
         if (restart) {
             SArgs<double> a = base_sargs<double>(op);
             a.precond = precond;
@@ -1065,7 +1075,6 @@ int cg_solve(const Op &op, double *x, const double *b, int max_iter, double tol,
             a.bvec = b;
             a.out0 = r;
             a.partials = part;
-            a.counter = cnt + 1;
             a.ctrl = ctrl;
             a.fin.fin = FIN_CG_BETA;
             a.fin.it = k + 1;
@@ -1079,6 +1088,12 @@ int cg_solve(const Op &op, double *x, const double *b, int max_iter, double tol,
             cyc++;
         }
     }
+    // the last iteration's x += alpha d (runs after done is set too)
+    u.x = x;
+    prof_begin("cg_update");
+    HC(launch_cg(CgStep::X_PENDING, u, C.stream));
+    prof_end(s_b * 3);
+    C.bytes_acc += s_b * 3;
     HC(hipEventRecord(C.t1, C.stream));
     Ctrl &hc = C.ctrl_h[0];
     if (int rc = finish_ctrl(ctrl, &hc)) return rc;
@@ -1465,7 +1480,6 @@ int aar_refined(const Op &op, double *x, const double *b, double omega, double b
         a.bvec = b;
         a.out32 = r32;
         a.partials = part;
-        a.counter = cnt + 1;
         a.ctrl = ctrl;
         a.fin.fin = FIN_SUMS;
         if (int rc = run_stencil<double>(SMode::RESID, a, s_b * 2 + 4.0 * n)) return rc;

@@ -7,20 +7,33 @@
 // w_o = a*coeff_lap[o].  The same operation order is used here with
 // contraction off, so a stencil result is bit-identical to the reference.
 //
-// Design (gfx950): a block of 256 threads = 4 wavefronts owns a 64 x TY
-// column of the grid (64 = one wavefront across x, TY = 4*PY rows, PY
-// rows per thread) over a z-chunk of `lz` planes and marches it in z.
+// Two forms of the sweep share the point formulas (stencil_point.h):
+//
+// The march (stencil_body.h), for grids that fill the chip: a block of WY
+// wavefronts owns a 64 x TY column of the grid over a z-chunk of `lz` planes
+// and marches it in z.
 // * z-neighbours come from a per-thread register queue of 13 planes, so
 //   every plane of the column is read from HBM once per chunk;
 // * x/y-neighbours come from a double-buffered LDS tile of the current
 //   plane with a 6-wide halo (corners are not needed by a star stencil),
-//   one barrier per plane; halo cells are fetched R planes ahead, together
-//   with the queue plane, and parked in a per-thread LDS ring;
+//   one barrier per plane; halo vectors are fetched R planes ahead, together
+//   with the queue plane, and parked in an LDS ring;
 // * block ids are mapped XCD-aware onto tiles so that y-adjacent tiles
 //   (whose halos overlap) run on the same XCD and share its L2.
+// What bounds it: with one point a lane the plane tile was read 8 (FP32: 4)
+// bytes a lane, 21 values a point, and the LDS pipe took 1.5 of the 2.2
+// clocks per point and CU at 512^3 FP64.  With 16 bytes a lane (Lane in
+// stencil_point.h) it takes 0.7, and HBM bounds the sweep.  Recurrence sweep
+// at 512^3: FP64 487 -> 436 us (4.9 TB/s of the two vectors), FP32 285 -> 230
+// us; the true residual 680 -> 580 us.
+//
+// The one-shot boxes (stencil_tile.h), for the smaller grids.
+//
 // The epilogue of each mode fuses the pointwise work of the solver step
 // that consumes A*x, so that step costs one pass over the grid.
-#include "stencil_body.h"
+#include "stencil_launch.h"
+
+#include <algorithm>
 
 namespace aar {
 
@@ -28,66 +41,84 @@ namespace aar {
 // host-side launch
 // ---------------------------------------------------------------------------
 
+// Rows of a one-shot box: four wavefronts, one row per thread.
+template <typename T> constexpr int TILE_ROWS = 4 * Lane<T>::RPW;
+
+// Where the boxes are faster than the march (recurrence sweep, microseconds
+// with the launch, best march shape against the boxes): FP64 48^3 8.4 / 5.2,
+// 96^3 11.7 / 12.7, 128^3 14.0 / 15.8, 160^3 30.8 / 27.9, 200 x 161 x 150
+// 33.8 / 35.2, 200^3 54.8 / 54.2, 256^3 67 / 103; FP32 48^3 7.9 / 4.9, 96^3
+// 9.5 / 8.3, 160^3 17.4 / 16.3, 200^3 29.6 / 28.8, 256^3 41 / 50.  The two
+// meet at about 8 million points; near the tie the boxes need no depth chosen
+// to fit.  Boxes of 4 planes read (4 + 12)/4 values a point; while they are
+// about one a CU or fewer, boxes of 2 planes are shorter (FP32 96^3 8.7 ->
+// 8.3 us, FP64 true residual 64^3 7.9 -> 6.2; 128^3 15.8 -> 16.8), and of one
+// plane while those leave half the CUs idle (48^3 5.2 -> 4.9, FP32 4.9 ->
+// 4.4, 16^3 4.9 -> 4.0; FP64 64^3 8.2 -> 8.5).  32-bit offsets span the grid.
 template <typename T>
-void stencil_geometry(SArgs<T> &a, int wy, int py)
+int stencil_tile_planes(int nx, int ny, int nz)
 {
-    const int ty = wy * py;
+    const long n = (long)nx * ny * nz;
+    if (n > 8500000L) return 0;
+    const long cols = (long)((nx + TX - 1) / TX) * ((ny + TILE_ROWS<T> - 1) / TILE_ROWS<T>);
+    if (cols * ((nz + 1) / 2) <= 150) return 1;
+    return cols * ((nz + 3) / 4) <= 300 ? 2 : 4;
+}
+
+template <typename T>
+void stencil_geometry(SArgs<T> &a, const Shape &sh)
+{
+    const int ty = sh.tile ? TILE_ROWS<T> : sh.wy * sh.py;
     a.nxy = a.nx * a.ny;
     a.ntx = (a.nx + TX - 1) / TX;
     a.nty = (a.ny + ty - 1) / ty;
-    if (a.lz <= 0) a.lz = a.nz;
-    if (a.lz > a.nz) a.lz = a.nz;
+    if (sh.tile) {
+        a.lz = sh.tile;
+    } else {
+        if (a.lz <= 0) a.lz = a.nz;
+        if (a.lz > a.nz) a.lz = a.nz;
+    }
     a.nzc = (a.nz + a.lz - 1) / a.lz;
     a.nitems = a.ntx * a.nty * a.nzc;
 }
 
-template <typename T, SMode M>
-hipError_t launch_stencil_t(SArgs<T> a, int wy, int py, hipStream_t st)
-{
-    stencil_geometry(a, wy, py);
-    dim3 grid(a.nitems), block(64 * wy);
-    const int key = wy * 10 + py;
-    switch (key) {
-    case 42: hipLaunchKernelGGL((stencil_kernel<T, 4, 2, M>), grid, block, 0, st, a); break;
-    case 44: hipLaunchKernelGGL((stencil_kernel<T, 4, 4, M>), grid, block, 0, st, a); break;
-    case 82: hipLaunchKernelGGL((stencil_kernel<T, 8, 2, M>), grid, block, 0, st, a); break;
-    case 84: hipLaunchKernelGGL((stencil_kernel<T, 8, 4, M>), grid, block, 0, st, a); break;
-    case 48: hipLaunchKernelGGL((stencil_kernel<T, 4, 8, M>), grid, block, 0, st, a); break;
-    default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
-}
-
 template <typename T>
-hipError_t launch_stencil(SMode m, const SArgs<T> &a, int wy, int py, hipStream_t st)
+hipError_t launch_stencil(SMode m, const SArgs<T> &a, const Shape &sh, hipStream_t st)
 {
-    if (a.vf) return launch_stencil_vc<T>(m, a, wy, py, st);
+    if (a.vf) return launch_stencil_vc<T>(m, a, sh, st);
     switch (m) {
-    case SMode::MATVEC: return launch_stencil_t<T, SMode::MATVEC>(a, wy, py, st);
-    case SMode::AAR_TRUE: return launch_stencil_t<T, SMode::AAR_TRUE>(a, wy, py, st);
-    case SMode::AAR_REC: return launch_stencil_t<T, SMode::AAR_REC>(a, wy, py, st);
-    case SMode::RESID: return launch_stencil_t<T, SMode::RESID>(a, wy, py, st);
-    case SMode::PGR_RICH: return launch_stencil_t<T, SMode::PGR_RICH>(a, wy, py, st);
-    case SMode::CG_Q: return launch_stencil_t<T, SMode::CG_Q>(a, wy, py, st);
-    case SMode::CG_RESID: return launch_stencil_t<T, SMode::CG_RESID>(a, wy, py, st);
-    case SMode::MATVEC_RES: return launch_stencil_t<T, SMode::MATVEC_RES>(a, wy, py, st);
+    case SMode::MATVEC: return launch_sweep<T, SMode::MATVEC, false>(a, sh, st);
+    case SMode::AAR_TRUE: return launch_sweep<T, SMode::AAR_TRUE, false>(a, sh, st);
+    case SMode::AAR_REC: return launch_sweep<T, SMode::AAR_REC, false>(a, sh, st);
+    default: break;
+    }
+    if constexpr (sizeof(T) == 8) {              // the FP64 solvers' own sweeps
+        switch (m) {
+        case SMode::RESID: return launch_sweep<T, SMode::RESID, false>(a, sh, st);
+        case SMode::PGR_STEP: return launch_sweep<T, SMode::PGR_STEP, false>(a, sh, st);
+        case SMode::CG_Q: return launch_sweep<T, SMode::CG_Q, false>(a, sh, st);
+        case SMode::CG_RESID: return launch_sweep<T, SMode::CG_RESID, false>(a, sh, st);
+        default: break;
+        }
     }
     return hipErrorInvalidValue;
 }
 
 template <typename T>
-int stencil_items(const SArgs<T> &a0, int wy, int py)
+int stencil_items(const SArgs<T> &a0, const Shape &sh)
 {
     SArgs<T> a = a0;
-    stencil_geometry(a, wy, py);
+    stencil_geometry(a, sh);
     return a.nitems;
 }
 
-template hipError_t launch_stencil<double>(SMode, const SArgs<double> &, int, int, hipStream_t);
-template hipError_t launch_stencil<float>(SMode, const SArgs<float> &, int, int, hipStream_t);
-template int stencil_items<double>(const SArgs<double> &, int, int);
-template void stencil_geometry<double>(SArgs<double> &, int, int);
-template void stencil_geometry<float>(SArgs<float> &, int, int);
-template int stencil_items<float>(const SArgs<float> &, int, int);
+template hipError_t launch_stencil<double>(SMode, const SArgs<double> &, const Shape &, hipStream_t);
+template hipError_t launch_stencil<float>(SMode, const SArgs<float> &, const Shape &, hipStream_t);
+template int stencil_items<double>(const SArgs<double> &, const Shape &);
+template int stencil_items<float>(const SArgs<float> &, const Shape &);
+template void stencil_geometry<double>(SArgs<double> &, const Shape &);
+template void stencil_geometry<float>(SArgs<float> &, const Shape &);
+template int stencil_tile_planes<double>(int, int, int);
+template int stencil_tile_planes<float>(int, int, int);
 
 }  // namespace aar

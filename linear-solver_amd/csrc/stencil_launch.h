@@ -1,0 +1,47 @@
+// stencil_launch.h -- host-side launch of one stencil sweep in a given shape.
+#pragma once
+
+#include "stencil_body.h"
+#include "stencil_tile.h"
+
+namespace aar {
+
+// A column of 64 x (wy*py) points.  A wavefront covers RPW rows of the tile
+// (2 in FP64, 4 in FP32), so wy*py rows are wy wavefronts with wy*py/(RPW wy)
+// rows per thread, or fewer wavefronts where that is below one row.
+template <typename T, SMode M, bool VC, int WY, int ROWS>
+hipError_t launch_march(const SArgs<T> &a, hipStream_t st)
+{
+    constexpr int RPW = Lane<T>::RPW;
+    constexpr int W = WY * RPW <= ROWS ? WY : ROWS / RPW;
+    constexpr int PY = ROWS / (W * RPW);
+    static_assert(W * RPW * PY == ROWS, "whole rows");
+    hipLaunchKernelGGL((stencil_kernel<T, W, PY, M, VC>), dim3(a.nitems), dim3(64 * W), 0, st, a);
+    return hipGetLastError();
+}
+
+template <typename T, SMode M, bool VC>
+hipError_t launch_sweep(SArgs<T> a, const Shape &sh, hipStream_t st)
+{
+    stencil_geometry(a, sh);
+    if (sh.tile) {
+        const dim3 grid(a.nitems), block(256);
+        switch (sh.tile) {
+        case 1: hipLaunchKernelGGL((stencil_tile_kernel<T, 4, 1, 1, M, VC>), grid, block, 0, st, a); break;
+        case 2: hipLaunchKernelGGL((stencil_tile_kernel<T, 4, 1, 2, M, VC>), grid, block, 0, st, a); break;
+        case 4: hipLaunchKernelGGL((stencil_tile_kernel<T, 4, 1, 4, M, VC>), grid, block, 0, st, a); break;
+        default: return hipErrorInvalidValue;
+        }
+        return hipGetLastError();
+    }
+    switch (sh.wy * 10 + sh.py) {
+    case 42: return launch_march<T, M, VC, 4, 8>(a, st);
+    case 44: return launch_march<T, M, VC, 4, 16>(a, st);
+    case 82: return launch_march<T, M, VC, 8, 16>(a, st);
+    case 84: return launch_march<T, M, VC, 8, 32>(a, st);
+    case 48: return launch_march<T, M, VC, 4, 32>(a, st);
+    default: return hipErrorInvalidValue;
+    }
+}
+
+}  // namespace aar

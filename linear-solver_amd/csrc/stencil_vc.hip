@@ -9,57 +9,39 @@
 //   MATVEC    y = a*Lap(x) + c x          (the order of the screened term)
 //   AAR_TRUE  r = b - A x; g = r / (diag + c); ||r||^2
 //   AAR_REC   g' = (1 - omega) g - h sum_o w_o S_o,  h = omega / D
-// and, for PGR/PL2R and CG, MATVEC_RES, CG_RESID (s = r / (diag + c)) and
-// PGR_RICH, CG_Q, whose pre-stencil step divides by diag + c at every
-// queue and halo point (c loaded there as one more field)
+// and, for PGR/PL2R and CG, PGR_STEP, CG_Q and CG_RESID (their Jacobi steps
+// divide by diag + c).
 // Kept in their own translation unit so the constant-coefficient kernels
 // compile exactly as before.
-#include "stencil_body.h"
+#include "stencil_launch.h"
 
 #include <algorithm>
 
 namespace aar {
 
-template <typename T, SMode M>
-hipError_t launch_stencil_vc_t(SArgs<T> a, int wy, int py, hipStream_t st)
-{
-    stencil_geometry(a, wy, py);
-    dim3 grid(a.nitems), block(64 * wy);
-    switch (wy * 10 + py) {
-    case 42: hipLaunchKernelGGL((stencil_kernel<T, 4, 2, M, true>), grid, block, 0, st, a); break;
-    case 44: hipLaunchKernelGGL((stencil_kernel<T, 4, 4, M, true>), grid, block, 0, st, a); break;
-    case 82: hipLaunchKernelGGL((stencil_kernel<T, 8, 2, M, true>), grid, block, 0, st, a); break;
-    case 84: hipLaunchKernelGGL((stencil_kernel<T, 8, 4, M, true>), grid, block, 0, st, a); break;
-    case 48: hipLaunchKernelGGL((stencil_kernel<T, 4, 8, M, true>), grid, block, 0, st, a); break;
-    default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
-}
-
 template <typename T>
-hipError_t launch_stencil_vc(SMode m, const SArgs<T> &a, int wy, int py, hipStream_t st)
+hipError_t launch_stencil_vc(SMode m, const SArgs<T> &a, const Shape &sh, hipStream_t st)
 {
     if (!a.vf || a.sigma != 0.0) return hipErrorInvalidValue;
     if constexpr (sizeof(T) == 4) {
         // FP32: the recurrence sweep of the mixed-precision solver only
         if (m != SMode::AAR_REC) return hipErrorInvalidValue;
-        return launch_stencil_vc_t<T, SMode::AAR_REC>(a, wy, py, st);
+        return launch_sweep<T, SMode::AAR_REC, true>(a, sh, st);
     } else {
         switch (m) {
-        case SMode::MATVEC: return launch_stencil_vc_t<T, SMode::MATVEC>(a, wy, py, st);
-        case SMode::AAR_TRUE: return launch_stencil_vc_t<T, SMode::AAR_TRUE>(a, wy, py, st);
-        case SMode::AAR_REC: return launch_stencil_vc_t<T, SMode::AAR_REC>(a, wy, py, st);
-        case SMode::MATVEC_RES: return launch_stencil_vc_t<T, SMode::MATVEC_RES>(a, wy, py, st);
-        case SMode::PGR_RICH: return launch_stencil_vc_t<T, SMode::PGR_RICH>(a, wy, py, st);
-        case SMode::CG_Q: return launch_stencil_vc_t<T, SMode::CG_Q>(a, wy, py, st);
-        case SMode::CG_RESID: return launch_stencil_vc_t<T, SMode::CG_RESID>(a, wy, py, st);
+        case SMode::MATVEC: return launch_sweep<T, SMode::MATVEC, true>(a, sh, st);
+        case SMode::AAR_TRUE: return launch_sweep<T, SMode::AAR_TRUE, true>(a, sh, st);
+        case SMode::AAR_REC: return launch_sweep<T, SMode::AAR_REC, true>(a, sh, st);
+        case SMode::PGR_STEP: return launch_sweep<T, SMode::PGR_STEP, true>(a, sh, st);
+        case SMode::CG_Q: return launch_sweep<T, SMode::CG_Q, true>(a, sh, st);
+        case SMode::CG_RESID: return launch_sweep<T, SMode::CG_RESID, true>(a, sh, st);
         default: return hipErrorInvalidValue;
         }
     }
 }
 
-template hipError_t launch_stencil_vc<double>(SMode, const SArgs<double> &, int, int, hipStream_t);
-template hipError_t launch_stencil_vc<float>(SMode, const SArgs<float> &, int, int, hipStream_t);
+template hipError_t launch_stencil_vc<double>(SMode, const SArgs<double> &, const Shape &, hipStream_t);
+template hipError_t launch_stencil_vc<float>(SMode, const SArgs<float> &, const Shape &, hipStream_t);
 
 // h(x) = omega / (diag + c(x)) with a Jacobi preconditioner, else c(x),
 // rounded to Tg: the pointwise input of the recurrence sweep
