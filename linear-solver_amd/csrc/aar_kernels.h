@@ -103,6 +103,12 @@ struct GramArgs {
     Ctrl *ctrl = nullptr;
 };
 
+// The Gram's products: per-block partials, or with a.counter (and m <= 16)
+// their sums in ctrl->G by the last block.  launch_gram_solve, next on the
+// stream, sums the partials into ctrl->G and solves the m x m system (flags
+// as launch_ls).
+template <typename T>
+hipError_t launch_gram_solve(const GramArgs<T> &a, int flags, hipStream_t st);
 template <typename T>
 hipError_t launch_gram(const GramArgs<T> &a, hipStream_t st);
 
@@ -114,8 +120,6 @@ hipError_t launch_gram(const GramArgs<T> &a, hipStream_t st);
 // (s_j <= 2^-53 s_max dropped) instead of tools.c's (s_j < m s_max eps).
 constexpr int LS_TEXTBOOK = 1, LS_GELSD = 2;
 hipError_t launch_ls(Ctrl *ctrl, int m, int flags, hipStream_t st);
-// the same for `count` independent solves, ctrls a device array of pointers
-hipError_t launch_ls_batch(Ctrl *const *ctrls, int count, int m, hipStream_t st);
 
 // AAR.c:225-231 + 116-117:  x_new = (x_k + beta f_k) - sum_k (DX_k + beta DF_k) s_col(k)
 template <typename T>
@@ -280,10 +284,14 @@ struct HGramArgs {
     int nvalid = 0;
     int it = 0;
     int nblocks = 0;
+    int flags = 0;            // launch_ls's
     double *partials = nullptr;
     Ctrl *ctrl = nullptr;
 };
+// per-block partials; then their sums as the real 2m x 2m system in ctrl->G
+// and its solution
 hipError_t launch_hgram(const HGramArgs &a, hipStream_t st);
+hipError_t launch_hgram_solve(const HGramArgs &a, hipStream_t st);
 
 // complex anchor update: AncArgs with complex gamma = s[t] + i s[m + t]
 struct HAncArgs {

@@ -23,6 +23,7 @@
 #include <vector>
 
 #include "aar_solver.h"
+#include "ls_body.h"
 #include "stencil_body.h"
 
 namespace aar {
@@ -45,7 +46,7 @@ struct BInst {
     double *hist = nullptr;
     int hist_cap = 0;
     double *spart = nullptr;   // stencil partials
-    double *gpart = nullptr;   // Gram partials [nchunks][NA]
+    double *gpart = nullptr;   // Gram partials [NA][nchunks]
     int nchunks = 0;
     int tr_items = 0;
 };
@@ -133,14 +134,14 @@ __global__ __launch_bounds__(BLOCK) void bgram_kernel(const BInst<double, Tg> *i
     Ctrl *ctrl;
     const Tg *G;
     long n, ld;
-    int S;
+    int S, nchunks;
     double *gpart;
     if (instd) {
         const auto &I = instd[wi.inst];
-        ctrl = I.ctrl; G = I.G; n = I.n; ld = I.ld; S = I.S; gpart = I.gpart;
+        ctrl = I.ctrl; G = I.G; n = I.n; ld = I.ld; S = I.S; gpart = I.gpart; nchunks = I.nchunks;
     } else {
         const auto &I = instf[wi.inst];
-        ctrl = I.ctrl; G = I.G; n = I.n; ld = I.ld; S = I.S; gpart = I.gpart;
+        ctrl = I.ctrl; G = I.G; n = I.n; ld = I.ld; S = I.S; gpart = I.gpart; nchunks = I.nchunks;
     }
     if (ctrl->done) return;
     const long k = (long)*clock + jrel;
@@ -171,20 +172,23 @@ __global__ __launch_bounds__(BLOCK) void bgram_kernel(const BInst<double, Tg> *i
             acc[NG + j] += d[j] * v[0];
         }
     }
-    block_reduce_to<NA>(acc, gpart + (size_t)wi.idx * NA, scratch);
+    block_reduce_to_vm<NA>(acc, gpart + wi.idx, nchunks, scratch);
 }
 
-// per instance: fixed-order sum of the chunk partials, laid out as the
-// reference's allredvec (AAR.c:192-212) for the m x m solve
-template <typename Tg, int MM>
-__global__ __launch_bounds__(BLOCK) void bgram_finish_kernel(const BInst<double, Tg> *instd,
-                                                             const BInst<float, Tg> *instf, const int *clock,
-                                                             int jrel, BShared sh)
+// Per instance: fixed-order sums of the chunk partials (one wavefront per
+// value), laid out as the reference's allredvec (AAR.c:192-212) by every
+// thread, and the m x m solve by the first wavefront.
+constexpr int BFIN_NT = 512;
+
+template <typename Tg, int MM, int ML>
+__global__ __launch_bounds__(BFIN_NT) void bgram_solve_kernel(const BInst<double, Tg> *instd,
+                                                              const BInst<float, Tg> *instf, const int *clock,
+                                                              int jrel, BShared sh)
 {
     constexpr int NG = MM * (MM + 1) / 2;
     constexpr int NA = NG + MM;
-    __shared__ double scratch[BLOCK / 64];
     __shared__ double sums[NA];
+    __shared__ LsLds<ML> L;
     Ctrl *ctrl;
     const double *gpart;
     int nchunks;
@@ -196,20 +200,28 @@ __global__ __launch_bounds__(BLOCK) void bgram_finish_kernel(const BInst<double,
         ctrl = I.ctrl; gpart = I.gpart; nchunks = I.nchunks;
     }
     if (ctrl->done) return;
-    final_sum(gpart, nchunks, NA, sums, scratch);
-    if (threadIdx.x != 0) return;
+    final_sum_vm<BFIN_NT>(gpart, nchunks, NA, sums);
     const int k = *clock + jrel, m = sh.m;
     const int nv = min(m, k - 1);
-    double *Gm = ctrl->G;
-    for (int q = 0; q < m * m + m; q++) Gm[q] = 0.0;
-    auto col = [&](int age) { return ((k - 2 - age) % m + m) % m; };     // AAR.c:97
-    for (int j = 0; j < nv; j++)
-        for (int q = 0; q <= j; q++) {
-            const double v = sums[j * (j + 1) / 2 + q];
-            Gm[col(j) * m + col(q)] = v;
-            Gm[col(q) * m + col(j)] = v;
+    auto age = [&](int c) { return ((k - 2 - c) % m + m) % m; };     // AAR.c:97 inverted
+    auto entry = [&](int e) -> double {
+        if (e >= m * m) {
+            const int j = age(e - m * m);
+            return j < nv ? sums[NG + j] : 0.0;
         }
-    for (int j = 0; j < nv; j++) Gm[m * m + col(j)] = sums[NG + j];
+        const int j = age(e / m), q = age(e % m);
+        if (j >= nv || q >= nv) return 0.0;
+        return j > q ? sums[j * (j + 1) / 2 + q] : sums[q * (q + 1) / 2 + j];
+    };
+    for (int e = threadIdx.x; e < m * m + m; e += BFIN_NT) {
+        const double v = entry(e);
+        ctrl->G[e] = v;
+        if (e < m * m) L.A[e % m][e / m] = v;
+    }
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    const int lane = threadIdx.x;
+    ls_solve<ML>(L, lane < m ? entry(m * m + lane) : 0.0, ctrl, m, 0);
 }
 
 // -------------------------------------------------------------------------
@@ -343,12 +355,10 @@ int batch_solve(const aar_hip_instance *ins, int count, double omega, double bet
     std::vector<BInst<Tx, Tg>> hI(count);
     std::vector<Op> ops(count);
     std::vector<WorkItem> wtr, wrc, wch;
-    std::vector<Ctrl *> hctrl(count);
     std::vector<Ctrl> hc(count);
     BInst<Tx, Tg> *dI = nullptr;
     WorkItem *dtr = nullptr, *drc = nullptr, *dch = nullptr;
     Ctrl *ctrls = nullptr;
-    Ctrl **dctrl = nullptr;
     int *clock = nullptr, *ndone = nullptr, *ndone_h = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -373,7 +383,6 @@ int batch_solve(const aar_hip_instance *ins, int count, double omega, double bet
     BHC(hipEventRecord(ev_in, C.stream));
     BHC(hipStreamWaitEvent(st, ev_in, 0));
     BHC(bsp_alloc(&ctrls, count, owned));
-    BHC(bsp_alloc(&dctrl, count, owned));
     BHC(bsp_alloc(&clock, 1, owned));
     BHC(hipHostMalloc((void **)&ndone_h, sizeof(int) * 64, hipHostMallocDefault));
     BHC(bsp_alloc(&ndone, 1, owned));
@@ -392,7 +401,6 @@ int batch_solve(const aar_hip_instance *ins, int count, double omega, double bet
         I.NC = NC;
         I.x = (Tx *)ins[i].x;
         I.ctrl = ctrls + i;
-        hctrl[i] = ctrls + i;
         I.hist_cap = max_iter + 4;
         BHC(bsp_alloc(&I.G, (size_t)I.ld * S, owned));
         if (NC > 0) BHC(bsp_alloc(&I.C, (size_t)I.ld * NC, owned));
@@ -445,7 +453,6 @@ int batch_solve(const aar_hip_instance *ins, int count, double omega, double bet
     BHC(hipMemcpy(dtr, wtr.data(), sizeof(WorkItem) * wtr.size(), hipMemcpyHostToDevice));
     BHC(hipMemcpy(drc, wrc.data(), sizeof(WorkItem) * wrc.size(), hipMemcpyHostToDevice));
     BHC(hipMemcpy(dch, wch.data(), sizeof(WorkItem) * wch.size(), hipMemcpyHostToDevice));
-    BHC(hipMemcpy(dctrl, hctrl.data(), sizeof(Ctrl *) * count, hipMemcpyHostToDevice));
 
     {
         // kernels of the batch, launched on `st` (eagerly or under capture)
@@ -467,13 +474,12 @@ int batch_solve(const aar_hip_instance *ins, int count, double omega, double bet
                 constexpr int M = decltype(mm)::value;
                 hipLaunchKernelGGL((bgram_kernel<Tg, M>), dim3((unsigned)wch.size()), dim3(BLOCK), 0, st, ID, IF, dch,
                                    clock, jrel, sh);
-                hipLaunchKernelGGL((bgram_finish_kernel<Tg, M>), dim3(count), dim3(BLOCK), 0, st, ID, IF, clock, jrel,
-                                   sh);
+                hipLaunchKernelGGL((bgram_solve_kernel<Tg, M, (M <= 8 ? 8 : 16)>), dim3(count), dim3(BFIN_NT), 0, st, ID,
+                                   IF, clock, jrel, sh);
             };
             if (m == 7) gram(std::integral_constant<int, 7>());
             else if (m <= MAXM_FAST) gram(std::integral_constant<int, MAXM_FAST>());
             else gram(std::integral_constant<int, MAXM_BATCH>());
-            (void)launch_ls_batch(dctrl, count, m, st);
             hipLaunchKernelGGL((banchor_kernel<Tx, Tg>), dim3((unsigned)wch.size()), dim3(BLOCK), 0, st, dI, dch, clock,
                                jrel, 0, sh);
             hipLaunchKernelGGL((bstencil_kernel<Tx, Tx, Tg, SMode::AAR_TRUE>), dim3((unsigned)wtr.size()),

@@ -307,7 +307,7 @@ int step_gram_ls(int kind, const StepBufs &sb, int m, int n)
         g.fslot = 0;
     }
     HCR(launch_gram<double>(g, C.stream), AAR_HIP_ERR_HIP);
-    HCR(launch_ls(dc, m, 0, C.stream), AAR_HIP_ERR_HIP);
+    HCR(launch_gram_solve<double>(g, 0, C.stream), AAR_HIP_ERR_HIP);
     return 0;
 }
 

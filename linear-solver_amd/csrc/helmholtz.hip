@@ -18,6 +18,7 @@
 #include "aar_common.h"
 #include "aar_device.h"
 #include "aar_kernels.h"
+#include "ls_body.h"
 
 namespace aar {
 
@@ -267,10 +268,6 @@ hipError_t launch_hstencil(HMode m, const HArgs &a0, hipStream_t st)
 // ---------------------------------------------------------------------------
 // Hermitian Gram of the complex g ring (PETSC_COMPLEX/AAR_Complex.c:213-236)
 // ---------------------------------------------------------------------------
-namespace {
-__device__ inline int href_col(int it, int k, int m) { return ((it - 2 - k) % m + m) % m; }
-}
-
 template <int MM>
 __global__ __launch_bounds__(BLOCK) void hgram_kernel(const HGramArgs a)
 {
@@ -318,63 +315,75 @@ __global__ __launch_bounds__(BLOCK) void hgram_kernel(const HGramArgs a)
             acc[2 * NG + 2 * j + 1] += dr[j] * fi - di[j] * fr;
         }
     }
-    block_reduce_to<NA>(acc, a.partials + (size_t)blockIdx.x * NA, scratch);
+    // value-major partials: each value's per-block sums are contiguous
+    block_reduce_to_vm<NA>(acc, a.partials + blockIdx.x, a.nblocks, scratch);
 }
 
-// one block: fixed-order sum of the partials, then the real 2m x 2m layout
-// read by ls_kernel (a[i][j] = G[j*n + i], rhs G[n*n + i], n = 2m)
-template <int MM>
-__global__ __launch_bounds__(BLOCK) void hgram_finish_kernel(const HGramArgs a)
+// One block: fixed-order sums of the partials (one wavefront per value), the
+// real 2m x 2m system E = [Gr -Gi; Gi Gr] (E[i][j] at G[j*n + i], rhs at
+// G[n*n + i], n = 2m) with every thread laying out its entries, and its solve
+// by the first wavefront.
+template <int M2> constexpr int HFIN_NT = M2 <= 16 ? 512 : 256;
+
+template <int MM, int M2>
+__global__ __launch_bounds__(HFIN_NT<M2>) void hgram_finish_kernel(const HGramArgs a)
 {
     constexpr int NG = MM * (MM + 1) / 2;
     constexpr int NA = 2 * (NG + MM);
-    __shared__ double scratch[BLOCK / 64];
+    static_assert(M2 >= 2 * MM, "the embedded system fits");
     __shared__ double sums[NA];
+    __shared__ LsLds<M2> L;
     if (a.ctrl->done) return;
-    final_sum(a.partials, a.nblocks, NA, sums, scratch);
-    if (threadIdx.x != 0) return;
+    final_sum_vm<HFIN_NT<M2>>(a.partials, a.nblocks, NA, sums);
     const int m = a.m, n2 = 2 * m, nv = a.nvalid;
-    double *G = a.ctrl->G;
-    for (int k = 0; k < n2 * n2 + n2; k++) G[k] = 0.0;
-    auto put = [&](int i, int j, double v) { G[j * n2 + i] = v; };   // E[i][j]
-    for (int j = 0; j < nv; j++)
-        for (int q = 0; q <= j; q++) {
-            const int t = j * (j + 1) / 2 + q;
-            const double re = sums[2 * t], im = sums[2 * t + 1];
-            const int ci = href_col(a.it, q, m), cj = href_col(a.it, j, m);
-            // Gr[ci][cj] = Gr[cj][ci] = re; Gi[ci][cj] = im, Gi[cj][ci] = -im;
-            // E = [Gr -Gi; Gi Gr]
-            put(ci, cj, re);
-            put(cj, ci, re);
-            put(m + ci, m + cj, re);
-            put(m + cj, m + ci, re);
-            put(ci, m + cj, -im);
-            put(cj, m + ci, im);
-            put(m + ci, cj, im);
-            put(m + cj, ci, -im);
+    // age of the reference's column c (ages as in GramArgs)
+    auto age = [&](int c) { return ((a.it - 2 - c) % m + m) % m; };
+    auto entry = [&](int e) -> double {
+        if (e >= n2 * n2) {
+            const int r = e - n2 * n2, k = age(r % m);
+            return k < nv ? sums[2 * NG + 2 * k + r / m] : 0.0;
         }
-    for (int j = 0; j < nv; j++) {
-        const int cj = href_col(a.it, j, m);
-        G[n2 * n2 + cj] = sums[2 * NG + 2 * j];
-        G[n2 * n2 + m + cj] = sums[2 * NG + 2 * j + 1];
+        const int i = e % n2, j = e / n2;                  // E[i][j]
+        const int ki = age(i % m), kj = age(j % m);
+        if (ki >= nv || kj >= nv) return 0.0;
+        // <DF_q, DF_p> of ages q <= p at p(p+1)/2 + q: Gr[i][j] = re, Gi[i][j]
+        // = im for i of age q, the conjugate for the other order
+        const int p = ki > kj ? ki : kj, q = ki > kj ? kj : ki;
+        const double re = sums[2 * (p * (p + 1) / 2 + q)];
+        double im = sums[2 * (p * (p + 1) / 2 + q) + 1];
+        if (ki >= kj) im = -im;
+        const int bi = i / m, bj = j / m;
+        return bi == bj ? re : (bi == 0 ? -im : im);
+    };
+    for (int e = threadIdx.x; e < n2 * n2 + n2; e += HFIN_NT<M2>) {
+        const double v = entry(e);
+        a.ctrl->G[e] = v;
+        if (e < n2 * n2) L.A[e % n2][e / n2] = v;
     }
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    const int lane = threadIdx.x;
+    ls_solve<M2>(L, lane < n2 ? entry(n2 * n2 + lane) : 0.0, a.ctrl, n2, a.flags);
 }
 
 hipError_t launch_hgram(const HGramArgs &a, hipStream_t st)
 {
     if (a.m < 1 || a.m > MAXM_CPLX || 2 * a.m > MAXM_LS || a.nvalid < 0 || a.nvalid > a.m) return hipErrorInvalidValue;
-    if (a.m <= 7) {
-        hipLaunchKernelGGL((hgram_kernel<7>), dim3(a.nblocks), dim3(BLOCK), 0, st, a);
-        hipLaunchKernelGGL((hgram_finish_kernel<7>), dim3(1), dim3(BLOCK), 0, st, a);
-    } else if (a.m <= 8) {
-        hipLaunchKernelGGL((hgram_kernel<8>), dim3(a.nblocks), dim3(BLOCK), 0, st, a);
-        hipLaunchKernelGGL((hgram_finish_kernel<8>), dim3(1), dim3(BLOCK), 0, st, a);
-    } else {
-        // deeper histories (the reference's complex README run uses m = 13):
-        // 304 accumulators, partly spilled; correct, at lower throughput
-        hipLaunchKernelGGL((hgram_kernel<MAXM_CPLX>), dim3(a.nblocks), dim3(BLOCK), 0, st, a);
-        hipLaunchKernelGGL((hgram_finish_kernel<MAXM_CPLX>), dim3(1), dim3(BLOCK), 0, st, a);
-    }
+    const dim3 grid(a.nblocks), block(BLOCK);
+    // deeper histories (the reference's complex README run uses m = 13): 304
+    // accumulators, partly spilled; correct, at lower throughput
+    if (a.m <= 7) hipLaunchKernelGGL((hgram_kernel<7>), grid, block, 0, st, a);
+    else if (a.m <= 8) hipLaunchKernelGGL((hgram_kernel<8>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((hgram_kernel<MAXM_CPLX>), grid, block, 0, st, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_hgram_solve(const HGramArgs &a, hipStream_t st)
+{
+    const dim3 grid(1);
+    if (a.m <= 7) hipLaunchKernelGGL((hgram_finish_kernel<7, 16>), grid, dim3(HFIN_NT<16>), 0, st, a);
+    else if (a.m <= 8) hipLaunchKernelGGL((hgram_finish_kernel<8, 16>), grid, dim3(HFIN_NT<16>), 0, st, a);
+    else hipLaunchKernelGGL((hgram_finish_kernel<MAXM_CPLX, 2 * MAXM_CPLX>), grid, dim3(HFIN_NT<32>), 0, st, a);
     return hipGetLastError();
 }
 

@@ -12,32 +12,46 @@
 #include <type_traits>
 
 #include "history.h"
+#include "ls_body.h"
 
 namespace aar {
 
-// reference allredvec layout (AAR.c:192-212, PGR.c:188-206): [j*m + i] =
-// col_i . col_j, [m*m + j] = col_j . f; missing columns are zero
+// The system built from the sums of a Gram (AAR.c:192-212, PGR.c:188-206):
+// reference allredvec layout, [j*m + i] = col_i . col_j, [m*m + j] = col_j . f;
+// missing columns are zero.  Every thread of the block writes its entries.
+// mm: the columns the sums were made for (products (j, q) at j*mm + q for
+// kind 1, else the lower triangle by rows; then the right-hand sides).
+struct GramFin {
+    int m, mm, kind, nvalid, it, direct;
+    int nblocks;
+    const double *partials;
+    Ctrl *ctrl;
+};
+__device__ __forceinline__ int gram_values(const GramFin &a)
+{
+    return (a.kind == 1 ? a.mm * a.mm : a.mm * (a.mm + 1) / 2) + a.mm;
+}
+// value e < m*m + m of the layout
+__device__ __forceinline__ double gram_entry(const GramFin &a, const double *sums, int e)
+{
+    const int m = a.m, nv = a.nvalid;
+    // age of the reference's column c (ref_col inverted)
+    auto age = [&](int c) { return a.direct ? c : ((a.it - 2 - c) % m + m) % m; };
+    if (e >= m * m) {
+        const int k = age(e - m * m);
+        return k < nv ? sums[gram_values(a) - a.mm + k] : 0.0;
+    }
+    const int j = age(e / m), q = age(e % m);
+    if (j >= nv || q >= nv) return 0.0;
+    if (a.kind == 1) return sums[j * a.mm + q];
+    return j > q ? sums[j * (j + 1) / 2 + q] : sums[q * (q + 1) / 2 + j];
+}
+
 template <typename T, int MM, int KIND>
 __device__ inline void gram_layout(const GramArgs<T> &a, const double *sums)
 {
-    constexpr int NG = (KIND == 1) ? MM * MM : MM * (MM + 1) / 2;
-    const int m = a.m, nv = a.nvalid, dir = a.direct;
-    double *G = a.ctrl->G;
-    for (int k = 0; k < m * m + m; k++) G[k] = 0.0;
-    if constexpr (KIND == 1) {
-        for (int j = 0; j < nv; j++)
-            for (int q = 0; q < nv; q++)
-                G[ref_col(a.it, j, m, dir) * m + ref_col(a.it, q, m, dir)] = sums[j * MM + q];
-    } else {
-        for (int j = 0; j < nv; j++)
-            for (int q = 0; q <= j; q++) {
-                const double v = sums[j * (j + 1) / 2 + q];
-                const int cj = ref_col(a.it, j, m, dir), cq = ref_col(a.it, q, m, dir);
-                G[cj * m + cq] = v;
-                G[cq * m + cj] = v;
-            }
-    }
-    for (int j = 0; j < nv; j++) G[m * m + ref_col(a.it, j, m, dir)] = sums[NG + j];
+    const GramFin f = {a.m, MM, KIND, a.nvalid, a.it, a.direct, a.nblocks, a.partials, a.ctrl};
+    for (int e = threadIdx.x; e < a.m * a.m + a.m; e += blockDim.x) a.ctrl->G[e] = gram_entry(f, sums, e);
 }
 
 // ---------------------------------------------------------------------------
@@ -165,25 +179,61 @@ __global__ __launch_bounds__(BLOCK) void gram_kernel(const GramArgs<T> a)
     if (!a.counter) return;                     // two-pass: gram_finish_kernel follows
     if (last_block_arrive(a.counter, gridDim.x)) {
         final_sum_vm(a.partials, a.nblocks, NA, sums);
-        if (threadIdx.x == 0) {
-            gram_layout<T, MM, KIND>(a, sums);
-            *a.counter = 0u;
-        }
+        gram_layout<T, MM, KIND>(a, sums);
+        if (threadIdx.x == 0) *a.counter = 0u;
     }
 }
 
-// second pass of the normal-equation build: one block sums the per-block
-// partials in a fixed order (one wavefront per value, contiguous reads) and
-// lays the result out for the m x m solve
-template <typename T, int MM, int KIND>
-__global__ __launch_bounds__(BLOCK) void gram_finish_kernel(const GramArgs<T> a)
+// Second pass of the normal-equation build, and the m x m solve: one block
+// sums the per-block partials in a fixed order (one wavefront per value,
+// contiguous reads), every thread lays out its entries, and the first
+// wavefront solves (ls_body.h).  One launch instead of two, and sixteen
+// wavefronts on the sums instead of four: at m = 7 on 512 blocks the finish
+// (17 us, half of it one thread's layout) and the solve (63 us) took 80 us a
+// cycle at 512^3, now 45.  Larger systems leave a wavefront more registers.
+template <int M> constexpr int GFIN_NT = M <= 8 ? 1024 : (M <= 16 ? 512 : 256);
+
+template <int M>
+__global__ __launch_bounds__(GFIN_NT<M>) void gram_finish_kernel(const GramFin a, int flags)
 {
-    constexpr int NG = (KIND == 1) ? MM * MM : MM * (MM + 1) / 2;
-    constexpr int NA = NG + MM;
-    __shared__ double sums[NA];
-    if (a.ctrl->done) return;
-    final_sum_vm(a.partials, a.nblocks, NA, sums);
-    if (threadIdx.x == 0) gram_layout<T, MM, KIND>(a, sums);
+    __shared__ double sums[M * M + M];
+    __shared__ LsLds<M> L;
+    Ctrl *c = a.ctrl;
+    if (c->done) return;
+    final_sum_vm<GFIN_NT<M>>(a.partials, a.nblocks, gram_values(a), sums);
+    const int m = a.m;
+    for (int e = threadIdx.x; e < m * m + m; e += GFIN_NT<M>) {
+        const double v = gram_entry(a, sums, e);
+        c->G[e] = v;
+        // FtF[i][j] = allredvec[j*m + i] (AAR.c:214-221)
+        if (e < m * m) L.A[e % m][e / m] = v;
+    }
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    const int lane = threadIdx.x;
+    ls_solve<M>(L, lane < m ? gram_entry(a, sums, m * m + lane) : 0.0, c, m, flags);
+}
+
+// columns of the instantiation that a history of m runs: the reference's
+// default m = 7 (AAR) has its own, 35 accumulators and 8 loads per point
+// instead of MAXM_FAST's 44 and 9; the READMEs' m = 13 too
+static int gram_columns(int kind, int m)
+{
+    if (kind == 0 && m == 7) return 7;
+    return m <= MAXM_FAST ? MAXM_FAST : (m == 13 ? 13 : (m <= MAXM_MID ? MAXM_MID : MAXM));
+}
+
+template <typename T>
+hipError_t launch_gram_solve(const GramArgs<T> &a, int flags, hipStream_t st)
+{
+    const int mm = gram_columns(a.kind, a.m);
+    if (a.counter && a.m <= MAXM_MID) return launch_ls(a.ctrl, a.m, flags, st);    // ctrl->G is there
+    const GramFin f = {a.m, mm, a.kind, a.nvalid, a.it, a.direct, a.nblocks, a.partials, a.ctrl};
+    const dim3 grid(1);
+    if (mm <= 8) hipLaunchKernelGGL((gram_finish_kernel<8>), grid, dim3(GFIN_NT<8>), 0, st, f, flags);
+    else if (mm <= 16) hipLaunchKernelGGL((gram_finish_kernel<16>), grid, dim3(GFIN_NT<16>), 0, st, f, flags);
+    else hipLaunchKernelGGL((gram_finish_kernel<32>), grid, dim3(GFIN_NT<32>), 0, st, f, flags);
+    return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
@@ -346,10 +396,8 @@ __global__ __launch_bounds__(BLOCK) void gram_split_kernel(const GramArgs<T> a)
     if (NPASS > 1 || !a.counter) return;
     if (last_block_arrive(a.counter, gridDim.x)) {
         final_sum_vm(a.partials, a.nblocks, NA, sums);
-        if (threadIdx.x == 0) {
-            gram_layout<T, MM, KIND>(a, sums);
-            *a.counter = 0u;
-        }
+        gram_layout<T, MM, KIND>(a, sums);
+        if (threadIdx.x == 0) *a.counter = 0u;
     }
 }
 
@@ -472,10 +520,8 @@ __global__ __launch_bounds__(BLOCK) void gram_lds_kernel(const GramArgs<T> a)
     if (!a.counter) return;                     // two-pass: gram_finish_kernel follows
     if (last_block_arrive(a.counter, gridDim.x)) {
         final_sum_vm(a.partials, a.nblocks, NA, sums);
-        if (threadIdx.x == 0) {
-            gram_layout<T, MM, KIND>(a, sums);
-            *a.counter = 0u;
-        }
+        gram_layout<T, MM, KIND>(a, sums);
+        if (threadIdx.x == 0) *a.counter = 0u;
     }
 }
 
@@ -490,54 +536,37 @@ template <typename T>
 hipError_t launch_gram(const GramArgs<T> &a, hipStream_t st)
 {
     if (a.m < 1 || a.m > MAXM || a.nvalid < 0 || a.nvalid > a.m) return hipErrorInvalidValue;
-    dim3 grid(a.nblocks), block(BLOCK);
-    // the reference's default history m = 7 gets its own instantiation: 35
-    // accumulators and 8 loads per point instead of MAXM_FAST's 44 and 9
-    if (a.kind == 0 && a.m == 7) {
-        hipLaunchKernelGGL((gram_kernel<T, 7, 0>), grid, block, 0, st, a);
-        if (!a.counter) hipLaunchKernelGGL((gram_finish_kernel<T, 7, 0>), dim3(1), block, 0, st, a);
-        return hipGetLastError();
-    }
     if (a.kind < 0 || a.kind > 2) return hipErrorInvalidValue;
+    dim3 grid(a.nblocks), block(BLOCK);
     // m <= 8: every accumulator in registers
-    auto go = [&](auto mm) {
-        constexpr int M = decltype(mm)::value;
+    auto go = [&](auto c) {
+        constexpr int M = decltype(c)::value;
         switch (a.kind) {
         case 0: hipLaunchKernelGGL((gram_kernel<T, M, 0>), grid, block, 0, st, a); break;
         case 1: hipLaunchKernelGGL((gram_kernel<T, M, 1>), grid, block, 0, st, a); break;
         default: hipLaunchKernelGGL((gram_kernel<T, M, 2>), grid, block, 0, st, a); break;
         }
-        if (!a.counter) {
-            switch (a.kind) {
-            case 0: hipLaunchKernelGGL((gram_finish_kernel<T, M, 0>), dim3(1), block, 0, st, a); break;
-            case 1: hipLaunchKernelGGL((gram_finish_kernel<T, M, 1>), dim3(1), block, 0, st, a); break;
-            default: hipLaunchKernelGGL((gram_finish_kernel<T, M, 2>), dim3(1), block, 0, st, a); break;
-            }
-        }
     };
-    auto go_lds = [&](auto mm) {
-        constexpr int M = decltype(mm)::value;
+    auto go_lds = [&](auto c) {
+        constexpr int M = decltype(c)::value;
         switch (a.kind) {
         case 0: hipLaunchKernelGGL((gram_lds_kernel<T, M, 0>), grid, block, 0, st, a); break;
         case 1: hipLaunchKernelGGL((gram_lds_kernel<T, M, 1>), grid, block, 0, st, a); break;
         default: hipLaunchKernelGGL((gram_lds_kernel<T, M, 2>), grid, block, 0, st, a); break;
-        }
-        if (!a.counter) {
-            switch (a.kind) {
-            case 0: hipLaunchKernelGGL((gram_finish_kernel<T, M, 0>), dim3(1), block, 0, st, a); break;
-            case 1: hipLaunchKernelGGL((gram_finish_kernel<T, M, 1>), dim3(1), block, 0, st, a); break;
-            default: hipLaunchKernelGGL((gram_finish_kernel<T, M, 2>), dim3(1), block, 0, st, a); break;
-            }
         }
     };
     // 8 < m <= 16: the LDS-staged form, with an exact instantiation for the
     // READMEs' m = 13.  At 512^3, m = 13: AAR 2.63 ms against 2.91 ms with
     // every product in one thread's registers; PGR's square Gram 5.7 ms
     // against 10.9 ms split over wavefronts reading through L2
-    if (a.m <= MAXM_FAST) go(std::integral_constant<int, MAXM_FAST>());
-    else if (a.m <= MAXM_MID) {
-        if (a.m == 13) go_lds(std::integral_constant<int, 13>());
-        else go_lds(std::integral_constant<int, MAXM_MID>());
+    if (a.kind == 0 && a.m == 7) {
+        hipLaunchKernelGGL((gram_kernel<T, 7, 0>), grid, block, 0, st, a);
+    } else if (a.m <= MAXM_FAST) {
+        go(std::integral_constant<int, MAXM_FAST>());
+    } else if (a.m == 13) {
+        go_lds(std::integral_constant<int, 13>());
+    } else if (a.m <= MAXM_MID) {
+        go_lds(std::integral_constant<int, MAXM_MID>());
     } else {
         // 16 < m <= 32: 560 (AAR, PL2R) or 1056 (PGR) products, four and
         // eight passes of four slices, then the fixed-order finish
@@ -546,15 +575,12 @@ hipError_t launch_gram(const GramArgs<T> &a, hipStream_t st)
         case 1: launch_split_passes<T, MAXM, 1, 8>(a, grid, block, st); break;
         default: launch_split_passes<T, MAXM, 2, 4>(a, grid, block, st); break;
         }
-        switch (a.kind) {
-        case 0: hipLaunchKernelGGL((gram_finish_kernel<T, MAXM, 0>), dim3(1), block, 0, st, a); break;
-        case 1: hipLaunchKernelGGL((gram_finish_kernel<T, MAXM, 1>), dim3(1), block, 0, st, a); break;
-        default: hipLaunchKernelGGL((gram_finish_kernel<T, MAXM, 2>), dim3(1), block, 0, st, a); break;
-        }
     }
     return hipGetLastError();
 }
 
+template hipError_t launch_gram_solve<double>(const GramArgs<double> &, int, hipStream_t);
+template hipError_t launch_gram_solve<float>(const GramArgs<float> &, int, hipStream_t);
 template hipError_t launch_gram<double>(const GramArgs<double> &, hipStream_t);
 template hipError_t launch_gram<float>(const GramArgs<float> &, hipStream_t);
 

@@ -1513,7 +1513,7 @@ int aar_petsc_solve(const Op &op, double *x, const double *b, double omega, doub
             g.counter = nullptr;
             g.ctrl = &R.k->c;
             HC(launch_gram<double>(g, C.stream));
-            HC(launch_ls(&R.k->c, m, LS_GELSD, C.stream));   // dgelsd, rcond = -1
+            HC(launch_gram_solve<double>(g, LS_GELSD, C.stream));   // dgelsd, rcond = -1
             if (m <= 8) hipLaunchKernelGGL((k_aa_upd_kernel<8>), dim3(R.nb), dim3(KB), 0, C.stream, n, x,
                                            (const double *)f, (const double *)W, ld, m, beta, (const KCtrl *)R.k);
             else hipLaunchKernelGGL((k_aa_upd_kernel<16>), dim3(R.nb), dim3(KB), 0, C.stream, n, x,
@@ -1654,7 +1654,7 @@ int pgr_petsc_solve(const Op &op, double *x, const double *b, double omega, int 
             g.counter = nullptr;
             g.ctrl = &R.k->c;
             HC(launch_gram<double>(g, C.stream));
-            HC(launch_ls(&R.k->c, m, LS_GELSD, C.stream));   // dgelsd, rcond = -1
+            HC(launch_gram_solve<double>(g, LS_GELSD, C.stream));   // dgelsd, rcond = -1
             if (m <= 8)
                 hipLaunchKernelGGL((k_pg_upd_kernel<8>), dim3(R.nb), dim3(KB), 0, C.stream, n, x,
                                    (const double *)x_old, Ax, (const double *)Ax_prev, res, b, X, Y, ld, m, kk, R.part,

@@ -322,11 +322,19 @@ hipError_t run_dot(DotArgs<T> d)
     return e;
 }
 
+// the Gram and the m x m solve
 template <typename T>
-static hipError_t run_gram(GramArgs<T> g)
+static hipError_t run_gram(GramArgs<T> g, double bytes)
 {
-    if (ctx().two_pass) g.counter = nullptr;
-    return launch_gram<T>(g, ctx().stream);
+    Context &C = ctx();
+    if (C.two_pass) g.counter = nullptr;
+    prof_begin("gram");
+    hipError_t e = launch_gram<T>(g, C.stream);
+    prof_end(bytes);
+    prof_begin("ls");
+    if (e == hipSuccess) e = launch_gram_solve<T>(g, 0, C.stream);
+    prof_end(0);
+    return e;
 }
 
 static hipError_t run_pgr_update(PUpdArgs<double> u)
@@ -693,14 +701,9 @@ int aar_rec(const Op &op, Tx *x, const Tx *b, double omega, double beta, int m, 
             g.partials = part;
             g.counter = cnt + 2;
             g.ctrl = ctrl;
-            prof_begin("gram");
-            HC(run_gram<Tg>(g));
-            prof_end(sg * (nv + 1));
+            HC((run_gram<Tg>(g, sg * (nv + 1))));
             C.bytes_acc += sg * (nv + 1);
         }
-        prof_begin("ls");
-        HC(launch_ls(ctrl, m, 0, C.stream));
-        prof_end(0);
         {
             AncArgs<Tx, Tg> u;
             const long jlo = std::min(first, it - nv);
@@ -900,12 +903,7 @@ int pgr_solve(const Op &op, double *x, const double *b, double omega, int m, int
             g.partials = part;
             g.counter = cnt + 2;
             g.ctrl = ctrl;
-            prof_begin("gram");
-            HC(run_gram<double>(g));
-            prof_end(s_b * ((l2 ? 1 : 2) * (nv + 1) + 1));
-            prof_begin("ls");
-            HC(launch_ls(ctrl, m, 0, C.stream));
-            prof_end(0);
+            HC(run_gram<double>(g, s_b * ((l2 ? 1 : 2) * (nv + 1) + 1)));
             u.X = X;
             u.Y = Y;
             u.b = b;
@@ -1341,14 +1339,15 @@ int helm_solve(const HOp &op, double *u, const double *b, double omega, double b
             g.nblocks = nb;
             g.partials = part;
             g.ctrl = ctrl;
+            g.flags = C.complex_ref_order ? 0 : LS_TEXTBOOK;
             prof_begin("helm_gram");
             HC(launch_hgram(g, C.stream));
             prof_end(sv * (nv + 1));
             C.bytes_acc += sv * (nv + 1);
+            prof_begin("ls");
+            HC(launch_hgram_solve(g, C.stream));
+            prof_end(0);
         }
-        prof_begin("ls");
-        HC(launch_ls(ctrl, 2 * m, C.complex_ref_order ? 0 : LS_TEXTBOOK, C.stream));
-        prof_end(0);
         {
             HAncArgs hu;
             const long jlo = std::min(first, it - nv);
