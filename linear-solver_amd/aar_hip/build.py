@@ -21,7 +21,7 @@ LIB = os.path.join(PKG_ROOT, "libaar_hip.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("AAR_HIP_ARCH", "gfx950")
 
-SOURCES = ["stencil.hip", "stencil_vc.hip", "history.hip", "ls.hip", "update.hip", "helmholtz.hip", "batch.hip", "solver.hip", "krylov.hip",
+SOURCES = ["stencil.hip", "stencil_vc.hip", "history.hip", "ls.hip", "update.hip", "helmholtz.hip", "batch.hip", "solver.hip", "krylov.hip", "ilu.hip",
            "capi.hip", "stream.hip", "noalloc.hip"]
 
 # -ffp-contract=off: the stencil, the Richardson/Anderson updates and the

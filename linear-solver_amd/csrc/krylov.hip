@@ -33,6 +33,7 @@
 // enqueues and polls.
 #include "aar_device.h"
 #include "aar_solver.h"
+#include "ilu.h"
 
 #include <algorithm>
 #include <cstring>
@@ -849,222 +850,13 @@ __global__ __launch_bounds__(KB) void k_final_kernel(KCtrl *k, const double *par
     k->c.relres = k->relres;
 }
 
-// ---------------------------------------------------------------------------
-// ILU(0) of the periodic FD12 star matrix (the PETSc variant's pc = 1:
-// PCBJACOBI -> PCILU on one block, PETSC_REAL/main.c:88-91; PCICC of
-// AAR_Real.c:58-60 is the same preconditioner in exact arithmetic on this
-// symmetric matrix).  Every dependency of a row (x, y, z) in the
-// elimination and in the forward solve has a smaller x + y + z (periodic
-// wrap included), so each level x + y + z = L is one launch; the backward
-// solves run the levels downwards.  Rows are eliminated in PETSc's IKJ
-// order and solved in ascending column order, with no sums across rows:
-// the factors and solves are bit-identical to the oracle's sequential ones.
-//
-// Factor layout: IFS doubles per row (37 used): [0] = 1/u_ii, [1 + 12*axis
-// + k] the entry at periodic offset d along axis (k = d + 6 for d < 0,
-// d + 5 for d > 0): l_ij below the row, u_ij above.
-// ---------------------------------------------------------------------------
-constexpr int IFS = 40;
-
-__host__ __device__ constexpr int islot(int ax, int d) { return 1 + 12 * ax + (d < 0 ? d + 6 : d + 5); }
-
-template <typename T>
-struct IluArgsT {
-    int nx, ny, nz;
-    int level, x0, y0, wx, wy;   // the level and its (x, y) box
-    double w[R + 1];             // a * coeff[o]
-    double diag;                 // real part of the diagonal without c(x): a * 3 * coeff[0] (+ sigma, + c0)
-    double eta;                  // its imaginary part (complex matrix)
-    const double *c;             // + c(x) on the diagonal, or null
-    T *F;
-    const int *skip;             // nonzero: no work (solver stopped / step gated)
-};
-using IluArgs = IluArgsT<double>;
-
-// scalar operations of the real and complex factorizations (complex:
-// explicit formulas, as the oracle's)
-__device__ __forceinline__ double s_mul(double a, double b) { return a * b; }
-__device__ __forceinline__ double2 s_mul(double2 a, double2 b)
+// Grid of the vector passes: four elements a thread, at most 1024 blocks
+// (64^3: 256 blocks where sixteen elements a thread left three CUs in four
+// idle; the 30-vector passes of GMRES there 82 -> 27 us).
+static int k_blocks(long n)
 {
-    return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
-}
-__device__ __forceinline__ double s_sub(double a, double b) { return a - b; }
-__device__ __forceinline__ double2 s_sub(double2 a, double2 b) { return make_double2(a.x - b.x, a.y - b.y); }
-__device__ __forceinline__ double s_inv(double a) { return 1.0 / a; }
-__device__ __forceinline__ double2 s_inv(double2 b)
-{
-    const double den = b.x * b.x + b.y * b.y;
-    return make_double2((1.0 * b.x + 0.0 * b.y) / den, (0.0 * b.x - 1.0 * b.y) / den);
-}
-template <typename T> __device__ __forceinline__ T s_make(double re, double im);
-template <> __device__ __forceinline__ double s_make<double>(double re, double) { return re; }
-template <> __device__ __forceinline__ double2 s_make<double2>(double re, double im) { return make_double2(re, im); }
-
-// Threads per block of the per-level kernels.  A level's points lie on the
-// plane x + y + z = L, so neighbouring lanes are 1 - nx*ny elements apart
-// and every load of a wave touches 64 cache lines; one-wave blocks spread a
-// level over as many CUs as it has waves instead of stacking four per CU.
-constexpr int ILU_WG = 64;
-
-// the point of this thread on the level, or false
-template <typename T>
-__device__ __forceinline__ bool ilu_point(const IluArgsT<T> &a, int &x, int &y, int &z)
-{
-    const int t = blockIdx.x * ILU_WG + threadIdx.x;
-    if (t >= a.wx * a.wy) return false;
-    x = a.x0 + t % a.wx;
-    y = a.y0 + t / a.wx;
-    z = a.level - x - y;
-    return z >= 0 && z < a.nz;
-}
-
-// periodic offsets of a row's columns along one axis in ascending column
-// order: q = 0..5 -> d = 1..6 (below the row only when wrapped), q = 6..11
-// -> d = -6..-1 (below unless wrapped)
-__device__ __forceinline__ constexpr int qoff(int q) { return q < 6 ? q + 1 : q - 12; }
-
-template <typename T>
-__device__ __forceinline__ void ilu_factor_point(const IluArgsT<T> &a, int x, int y, int z)
-{
-    const int cr[3] = {x, y, z}, dims[3] = {a.nx, a.ny, a.nz};
-    const long strides[3] = {1, a.nx, (long)a.nx * a.ny};
-    const long i = x + (long)y * a.nx + (long)z * a.nx * a.ny;
-    T v[37];
-    v[0] = s_make<T>(a.c ? a.diag + a.c[i] : a.diag, a.eta);
-#pragma unroll
-    for (int ax = 0; ax < 3; ax++)
-#pragma unroll
-        for (int d = 1; d <= R; d++) {
-            v[islot(ax, -d)] = s_make<T>(a.w[d], 0.0);
-            v[islot(ax, d)] = s_make<T>(a.w[d], 0.0);
-        }
-#pragma unroll
-    for (int ax = 2; ax >= 0; ax--) {            // z, y, x: ascending column index
-        const int c = cr[ax], n = dims[ax];
-        const long st = strides[ax];
-#pragma unroll
-        for (int q = 0; q < 12; q++) {
-            const int dk = qoff(q);
-            const bool lower = dk > 0 ? (c + dk >= n) : (c + dk >= 0);
-            if (!lower) continue;
-            const int ck = dk > 0 ? c + dk - n : c + dk;
-            const T *Fk = a.F + (size_t)(i + (long)(ck - c) * st) * IFS;
-            const T l = s_mul(v[islot(ax, dk)], Fk[0]);
-            v[islot(ax, dk)] = l;
-            // row k's columns above k that are in row i's pattern: on this axis
-#pragma unroll
-            for (int dij = -R; dij <= R; dij++) {
-                if (dij == dk) continue;
-                int cj = c + dij;
-                cj = cj < 0 ? cj + n : (cj >= n ? cj - n : cj);
-                if (cj <= ck) continue;
-                int dkj = dij - dk;
-                if (dkj > R) dkj -= n;
-                else if (dkj < -R) dkj += n;
-                if (dkj < -R || dkj > R) continue;
-                const int si = dij == 0 ? 0 : islot(ax, dij);
-                v[si] = s_sub(v[si], s_mul(l, Fk[islot(ax, dkj)]));
-            }
-        }
-    }
-    T *Fi = a.F + (size_t)i * IFS;
-    Fi[0] = s_inv(v[0]);
-#pragma unroll
-    for (int s = 1; s < 37; s++) Fi[s] = v[s];
-}
-
-template <typename T>
-__global__ __launch_bounds__(ILU_WG) void ilu_factor_kernel(IluArgsT<T> a)
-{
-    int x, y, z;
-    if (!ilu_point(a, x, y, z)) return;
-    ilu_factor_point(a, x, y, z);
-}
-
-// One level of a triangular solve, in place on io (in -> io when in != io
-// at the first solve of an apply).  lowerpass: the columns below the row
-// (forward levels); trans: the transposed factor (entries of the other
-// row); diagmul: multiply by 1/u_ii at the end.
-template <typename T, bool LOWER, bool TRANS, bool DIAG>
-__device__ __forceinline__ void ilu_solve_point(const IluArgsT<T> &a, const T *in, T *io, int x, int y, int z)
-{
-    const int cr[3] = {x, y, z}, dims[3] = {a.nx, a.ny, a.nz};
-    const long strides[3] = {1, a.nx, (long)a.nx * a.ny};
-    const long i = x + (long)y * a.nx + (long)z * a.nx * a.ny;
-    const T *Fi = a.F + (size_t)i * IFS;
-    T s = in[i];
-#pragma unroll
-    for (int t = 0; t < 3; t++) {
-        const int ax = LOWER ? 2 - t : t;        // ascending column index
-        const int c = cr[ax], n = dims[ax];
-        const long st = strides[ax];
-#pragma unroll
-        for (int q = 0; q < 12; q++) {
-            const int d = qoff(q);
-            const bool below = d > 0 ? (c + d >= n) : (c + d >= 0);
-            if (below != LOWER) continue;
-            const int cj = d > 0 ? (below ? c + d - n : c + d) : (below ? c + d : c + d + n);
-            const long j = i + (long)(cj - c) * st;
-            const T f = TRANS ? a.F[(size_t)j * IFS + islot(ax, -d)] : Fi[islot(ax, d)];
-            s = s_sub(s, s_mul(f, io[j]));
-        }
-    }
-    io[i] = DIAG ? s_mul(s, Fi[0]) : s;
-}
-
-template <typename T, bool LOWER, bool TRANS, bool DIAG>
-__global__ __launch_bounds__(ILU_WG) void ilu_solve_kernel(IluArgsT<T> a, const T *in, T *io)
-{
-    if (*a.skip) return;
-    int x, y, z;
-    if (!ilu_point(a, x, y, z)) return;
-    ilu_solve_point<T, LOWER, TRANS, DIAG>(a, in, io, x, y, z);
-}
-
-// The levels L0, L0 + step, ..., L1 (each with at most ILU_SMALL_PTS points
-// in its (x, y) box) in one workgroup, a barrier between levels: the same
-// per-point work as ilu_solve_kernel without a launch per level.
-constexpr int ILU_SMALL_WG = 1024, ILU_SMALL_PTS = 1024;
-
-template <typename T>
-__device__ __forceinline__ void ilu_level_box(const IluArgsT<T> &a, int L, int &x0, int &y0, int &wx, int &wy)
-{
-    x0 = max(0, L - (a.ny - 1) - (a.nz - 1));
-    y0 = max(0, L - (a.nx - 1) - (a.nz - 1));
-    wx = min(a.nx - 1, L) - x0 + 1;
-    wy = min(a.ny - 1, L) - y0 + 1;
-}
-
-template <typename T, bool LOWER, bool TRANS, bool DIAG>
-__global__ __launch_bounds__(ILU_SMALL_WG) void ilu_solve_small_kernel(IluArgsT<T> a, const T *in, T *io, int L0,
-                                                                      int L1, int step)
-{
-    if (*a.skip) return;
-    for (int L = L0;; L += step) {
-        int x0, y0, wx, wy;
-        ilu_level_box(a, L, x0, y0, wx, wy);
-        for (int t = threadIdx.x; t < wx * wy; t += ILU_SMALL_WG) {
-            const int x = x0 + t % wx, y = y0 + t / wx, z = L - x - y;
-            if (z >= 0 && z < a.nz) ilu_solve_point<T, LOWER, TRANS, DIAG>(a, in, io, x, y, z);
-        }
-        if (L == L1) break;
-        __syncthreads();
-    }
-}
-
-template <typename T>
-__global__ __launch_bounds__(ILU_SMALL_WG) void ilu_factor_small_kernel(IluArgsT<T> a, int L0, int L1)
-{
-    for (int L = L0;; L++) {
-        int x0, y0, wx, wy;
-        ilu_level_box(a, L, x0, y0, wx, wy);
-        for (int t = threadIdx.x; t < wx * wy; t += ILU_SMALL_WG) {
-            const int x = x0 + t % wx, y = y0 + t / wx, z = L - x - y;
-            if (z >= 0 && z < a.nz) ilu_factor_point(a, x, y, z);
-        }
-        if (L == L1) break;
-        __syncthreads();
-    }
+    if (ctx().hist_blocks > 0) return std::min(nblocks_for(n), 1024);
+    return (int)std::max(1L, std::min((n + 4 * KB - 1) / (4 * KB), 1024L));
 }
 
 // ---------------------------------------------------------------------------
@@ -1088,19 +880,6 @@ int check_ilu_grid(const Op &op)
     return 0;
 }
 
-// the (x, y) box of level L: x + y + z = L inside the grid
-template <typename T>
-void ilu_box(IluArgsT<T> &a, int L)
-{
-    const int x0 = std::max(0, L - (a.ny - 1) - (a.nz - 1)), x1 = std::min(a.nx - 1, L);
-    const int y0 = std::max(0, L - (a.nx - 1) - (a.nz - 1)), y1 = std::min(a.ny - 1, L);
-    a.level = L;
-    a.x0 = x0;
-    a.y0 = y0;
-    a.wx = x1 - x0 + 1;
-    a.wy = y1 - y0 + 1;
-}
-
 IluArgs ilu_args(const Op &op, double *F)
 {
     IluArgs a{};
@@ -1115,95 +894,6 @@ IluArgs ilu_args(const Op &op, double *F)
     return a;
 }
 
-template <typename T>
-int ilu_nlev(const IluArgsT<T> &a) { return a.nx + a.ny + a.nz - 2; }
-
-// a level whose (x, y) box has at most ILU_SMALL_PTS points
-template <typename T>
-bool ilu_small(IluArgsT<T> a, int L)
-{
-    ilu_box(a, L);
-    return (long)a.wx * a.wy <= ILU_SMALL_PTS;
-}
-
-// Launch the levels from..to (step +1 or -1): runs of small levels go to
-// `small(L0, L1)` in one launch, the others to `big(L)` one launch each.
-template <typename T, typename Small, typename Big>
-void ilu_levels(const IluArgsT<T> &a, int from, int to, int step, Small small, Big big)
-{
-    for (int L = from; L != to + step;) {
-        if (ilu_small(a, L)) {
-            int L1 = L;
-            while (L1 != to && ilu_small(a, L1 + step)) L1 += step;
-            small(L, L1);
-            L = L1 + step;
-        } else {
-            big(L);
-            L += step;
-        }
-    }
-}
-
-template <typename T>
-hipError_t ilu_factor(IluArgsT<T> a, hipStream_t st)
-{
-    ilu_levels(
-        a, 0, ilu_nlev(a) - 1, 1,
-        [&](int L0, int L1) {
-            hipLaunchKernelGGL((ilu_factor_small_kernel<T>), dim3(1), dim3(ILU_SMALL_WG), 0, st, a, L0, L1);
-        },
-        [&](int L) {
-            IluArgsT<T> b = a;
-            ilu_box(b, L);
-            hipLaunchKernelGGL((ilu_factor_kernel<T>), dim3((b.wx * b.wy + ILU_WG - 1) / ILU_WG), dim3(ILU_WG), 0, st, b);
-        });
-    return hipGetLastError();
-}
-
-// out = M^{-1} in (trans: M^{-T} in); out may be in
-template <typename T>
-hipError_t ilu_apply(IluArgsT<T> a, const T *in, T *out, bool trans, const int *skip, hipStream_t st)
-{
-    a.skip = skip;
-    const int nl = ilu_nlev(a);
-    const dim3 sw(ILU_SMALL_WG);
-    // forward: L (or U^T) over ascending levels, reading `in`
-    ilu_levels(
-        a, 0, nl - 1, 1,
-        [&](int L0, int L1) {
-            if (trans) hipLaunchKernelGGL((ilu_solve_small_kernel<T, true, true, true>), dim3(1), sw, 0, st, a, in, out,
-                                          L0, L1, 1);
-            else hipLaunchKernelGGL((ilu_solve_small_kernel<T, true, false, false>), dim3(1), sw, 0, st, a, in, out,
-                                    L0, L1, 1);
-        },
-        [&](int L) {
-            IluArgsT<T> b = a;
-            ilu_box(b, L);
-            const dim3 g((b.wx * b.wy + ILU_WG - 1) / ILU_WG), wg(ILU_WG);
-            if (trans) hipLaunchKernelGGL((ilu_solve_kernel<T, true, true, true>), g, wg, 0, st, b, in, out);
-            else hipLaunchKernelGGL((ilu_solve_kernel<T, true, false, false>), g, wg, 0, st, b, in, out);
-        });
-    // backward: U (or L^T) over descending levels, in place
-    ilu_levels(
-        a, nl - 1, 0, -1,
-        [&](int L0, int L1) {
-            if (trans) hipLaunchKernelGGL((ilu_solve_small_kernel<T, false, true, false>), dim3(1), sw, 0, st, a,
-                                          (const T *)out, out, L0, L1, -1);
-            else hipLaunchKernelGGL((ilu_solve_small_kernel<T, false, false, true>), dim3(1), sw, 0, st, a,
-                                    (const T *)out, out, L0, L1, -1);
-        },
-        [&](int L) {
-            IluArgsT<T> b = a;
-            ilu_box(b, L);
-            const dim3 g((b.wx * b.wy + ILU_WG - 1) / ILU_WG), wg(ILU_WG);
-            if (trans) hipLaunchKernelGGL((ilu_solve_kernel<T, false, true, false>), g, wg, 0, st, b,
-                                          (const T *)out, out);
-            else hipLaunchKernelGGL((ilu_solve_kernel<T, false, false, true>), g, wg, 0, st, b, (const T *)out,
-                                    out);
-        });
-    return hipGetLastError();
-}
-
 // algorithmic bytes of one ILU(0) apply: each row's 37 factor entries, the
 // input and both passes' output
 constexpr double ILU_APPLY_BYTES = (37 + 4) * 8.0;
@@ -1213,7 +903,7 @@ int k_setup(const Op &op, int precond, double tol, int max_it, int restart, int 
 {
     Context &C = ctx();
     R.n = op.n;
-    R.nb = std::min(nblocks_for(op.n), 1024);
+    R.nb = k_blocks(op.n);
     R.hcap = hcap;
     HC(ensure(C.kctl, sizeof(KCtrl)));
     HC(ensure(C.hist0, sizeof(double) * (size_t)hcap));
@@ -1339,7 +1029,7 @@ int gmres_solve(const Op &op, double *x, const double *b, int restart, int max_i
     double *V = (double *)C.kvec.p, *t = V + (size_t)ld * (restart + 1);
     double *F = nullptr;
     if (ilu) {
-        HC(ensure(C.kilu, sizeof(double) * (size_t)n * IFS));
+        HC(ensure(C.kilu, sizeof(double) * ilu_values(op.nx, op.ny, op.nz)));
         F = (double *)C.kilu.p;
     }
     const int hcap = max_it + max_it / restart + 8;
@@ -1414,7 +1104,7 @@ int ilu0_apply(const Op &op, const double *r, double *z, int trans)
     if (int rc = context_init()) return rc;
     if (!r || !z) return fail(AAR_HIP_ERR_ARG, "null vector");
     if (int rc = check_ilu_grid(op)) return rc;
-    HC(ensure(C.kilu, sizeof(double) * (size_t)op.n * IFS));
+    HC(ensure(C.kilu, sizeof(double) * ilu_values(op.nx, op.ny, op.nz)));
     HC(ensure(C.kctl, sizeof(KCtrl)));
     KCtrl *k = (KCtrl *)C.kctl.p;
     hipLaunchKernelGGL(k_zero_kernel, dim3(64), dim3(KB), 0, C.stream, (unsigned *)k,
@@ -1460,7 +1150,7 @@ int aar_petsc_solve(const Op &op, double *x, const double *b, double omega, doub
     double *r = W + (size_t)(2 * m + 3) * ld;
     double *F = nullptr;
     if (ilu) {
-        HC(ensure(C.kilu, sizeof(double) * (size_t)n * IFS));
+        HC(ensure(C.kilu, sizeof(double) * ilu_values(op.nx, op.ny, op.nz)));
         F = (double *)C.kilu.p;
     }
     const int gnb = nblocks_for(n);
@@ -1594,7 +1284,7 @@ int pgr_petsc_solve(const Op &op, double *x, const double *b, double omega, int 
     double *x_old = X + (size_t)(m + 1) * ld, *Ax_prev = x_old + ld, *res = Ax_prev + ld;
     double *F = nullptr;
     if (ilu) {
-        HC(ensure(C.kilu, sizeof(double) * (size_t)n * IFS));
+        HC(ensure(C.kilu, sizeof(double) * ilu_values(op.nx, op.ny, op.nz)));
         F = (double *)C.kilu.p;
     }
     const int gnb = nblocks_for(n);
@@ -1710,7 +1400,7 @@ static int bicg_ilu_solve(const Op &op, double *x, const double *b, int max_it, 
     const long n = op.n;
     const long ld = ring_ld(n, sizeof(double));
     HC(ensure(C.kvec, sizeof(double) * (size_t)ld * 8));
-    HC(ensure(C.kilu, sizeof(double) * (size_t)n * IFS));
+    HC(ensure(C.kilu, sizeof(double) * ilu_values(op.nx, op.ny, op.nz)));
     double *r = (double *)C.kvec.p, *rl = r + ld, *z = r + 2 * ld, *zl = r + 3 * ld;
     double *p = r + 4 * ld, *pl = r + 5 * ld, *q = r + 6 * ld, *ql = r + 7 * ld;
     const int hcap = max_it + 8;
@@ -1830,7 +1520,7 @@ int kspcg_solve(const Op &op, double *x, const double *b, int max_it, double tol
     const long n = op.n;
     const long ld = ring_ld(n, sizeof(double));
     HC(ensure(C.kvec, sizeof(double) * (size_t)ld * 4));
-    if (ilu) HC(ensure(C.kilu, sizeof(double) * (size_t)n * IFS));
+    if (ilu) HC(ensure(C.kilu, sizeof(double) * ilu_values(op.nx, op.ny, op.nz)));
     double *r = (double *)C.kvec.p, *z = r + ld, *p = r + 2 * ld, *q = r + 3 * ld;
     const int hcap = max_it + 8;
     C.bytes_acc = 0.0;
@@ -2594,7 +2284,7 @@ int helm_ilu0_apply(const HOp &op, const double *r, double *z, int trans)
     if (op.nx < 13 || op.ny < 13 || op.nz < 13)
         return fail(AAR_HIP_ERR_ARG, "the ILU(0) preconditioner needs every grid side >= 13");
     const long n = op.n;
-    HC(ensure(C.kilu, sizeof(double2) * (size_t)n * IFS));
+    HC(ensure(C.kilu, sizeof(double2) * ilu_values(op.nx, op.ny, op.nz)));
     HC(ensure(C.kctl, sizeof(KCtrlZ)));
     KCtrlZ *k = (KCtrlZ *)C.kctl.p;
     hipLaunchKernelGGL(k_zero_kernel, dim3(64), dim3(KB), 0, C.stream, (unsigned *)k,
@@ -2602,7 +2292,7 @@ int helm_ilu0_apply(const HOp &op, const double *r, double *z, int trans)
     IluArgsT<double2> a = helm_ilu_args(op, (double2 *)C.kilu.p);
     HC(ilu_factor(a, C.stream));
     double2 *zz = (double2 *)z;
-    const int nb = std::min(nblocks_for(n), 1024);
+    const int nb = k_blocks(n);
     HC(hipMemcpyAsync(zz, r, sizeof(double2) * n, hipMemcpyDeviceToDevice, C.stream));
     if (trans == 2) hipLaunchKernelGGL(kz_conj_kernel, dim3(nb), dim3(KB), 0, C.stream, n, zz, (const int *)&k->zero);
     HC(ilu_apply(a, (const double2 *)zz, zz, trans != 0, &k->zero, C.stream));
@@ -2649,7 +2339,7 @@ static int helm_gmres_impl(const HOp &op, double *u, const double *b, int restar
     double2 *Zs = t + ld, *AZs = Zs + (size_t)ld * nslot;
     int ord[ZAUG_MAX + 1] = {0}, aug_ct = 0;   // ord[slot]: 1 = newest, 0 = free
     const int ita = restart - aug;             // Arnoldi steps per cycle
-    const int nb = std::min(nblocks_for(n), 1024);
+    const int nb = k_blocks(n);
     const int hcap = max_it + max_it / ita + 8;
     HC(ensure(C.kctl, sizeof(KCtrlZ)));
     HC(ensure(C.hist0, sizeof(double) * (size_t)hcap));
@@ -2673,7 +2363,7 @@ static int helm_gmres_impl(const HOp &op, double *u, const double *b, int restar
     const double s = 16.0 * n, cb = op.c ? 8.0 * n : 0.0;
     IluArgsT<double2> za{};
     if (ilu) {
-        HC(ensure(C.kilu, sizeof(double2) * (size_t)n * IFS));
+        HC(ensure(C.kilu, sizeof(double2) * ilu_values(op.nx, op.ny, op.nz)));
         za = helm_ilu_args(op, (double2 *)C.kilu.p);
         HC(ilu_factor(za, C.stream));
         HC(ilu_apply(za, bz, t, false, &k->zero, C.stream));
@@ -2836,7 +2526,7 @@ int helm_bicg_solve(const HOp &op, double *u, const double *b, int max_it, doubl
     HC(ensure(C.kvec, sizeof(double2) * (size_t)ld * 8));
     double2 *r = (double2 *)C.kvec.p, *rl = r + ld, *z = r + 2 * ld, *zl = r + 3 * ld;
     double2 *p = r + 4 * ld, *pl = r + 5 * ld, *q = r + 6 * ld, *ql = r + 7 * ld;
-    const int nb = std::min(nblocks_for(n), 1024);
+    const int nb = k_blocks(n);
     const int hcap = max_it + 8;
     HC(ensure(C.kctl, sizeof(KCtrlZ)));
     HC(ensure(C.hist0, sizeof(double) * (size_t)hcap));
@@ -2872,7 +2562,7 @@ int helm_bicg_solve(const HOp &op, double *u, const double *b, int max_it, doubl
         return 0;
     };
     if (ilu) {
-        HC(ensure(C.kilu, sizeof(double2) * (size_t)n * IFS));
+        HC(ensure(C.kilu, sizeof(double2) * ilu_values(op.nx, op.ny, op.nz)));
         za = helm_ilu_args(op, (double2 *)C.kilu.p);
         HC(ilu_factor(za, C.stream));
         HC(ilu_apply(za, bz, z, false, &k->zero, C.stream));
