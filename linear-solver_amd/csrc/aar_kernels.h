@@ -256,7 +256,7 @@ enum class HMode : int {
 
 struct HArgs {
     int nx = 0, ny = 0, nz = 0, nxy = 0;
-    int lz = 0;
+    int lz = 0, box = 0;              // box: planes of a one-shot box, 0 the march
     int ntx = 0, nty = 0, nzc = 0, nitems = 0;
     double w[R + 1] = {};
     double dlap = 0.0;                // a * 3 * coeff[0]

@@ -14,7 +14,7 @@
 // The stencil keeps the design of stencil.hip (z-march with a register
 // queue, LDS plane tile, XCD-aware tiles) on 16-byte points; its plane tile
 // is twice as large, so halos are loaded per plane (no halo ring) and a
-// thread owns two rows.
+// thread owns two rows.  Small grids run one-shot boxes.
 #include "aar_common.h"
 #include "aar_device.h"
 #include "aar_kernels.h"
@@ -47,6 +47,33 @@ __device__ inline double2 cdiv_d(double2 f, double dr, double di)
     const double re = __dadd_rn(__dmul_rn(f.x, dr), __dmul_rn(f.y, di)) / den;
     const double im = __dsub_rn(__dmul_rn(f.y, dr), __dmul_rn(f.x, di)) / den;
     return make_double2(re, im);
+}
+
+// What a sweep does with the Laplacian part lap of A u at one point (element
+// g; ck = c(x), b the right-hand side): its output, and its norm term into acc.
+template <HMode MODE>
+__device__ __forceinline__ void helm_point(const HArgs &a, double2 lap, double2 u, double2 b, double ck, bool ok, int g,
+                                           double &acc)
+{
+    const double eta = a.eta, om = a.omega;
+    const double2 au = helm_diag_add(lap, u, ck, eta);
+    const double dr = __dadd_rn(a.dlap, ck);
+    if constexpr (MODE == HMode::MATVEC) {
+        if (ok) a.out0[g] = au;
+    } else if constexpr (MODE == HMode::TRUE_RES) {
+        const double2 f = make_double2(__dsub_rn(b.x, au.x), __dsub_rn(b.y, au.y));
+        acc += ok ? (f.x * f.x + f.y * f.y) : 0.0;
+        if (ok) a.out0[g] = cdiv_d(f, dr, eta);
+    } else {
+        // g' = g - omega (A g)/D; |D g'|^2 = ||b - A x'||^2 at the point
+        const double2 t = cdiv_d(au, dr, eta);
+        const double2 gn = make_double2(__dsub_rn(u.x, __dmul_rn(om, t.x)), __dsub_rn(u.y, __dmul_rn(om, t.y)));
+        if (ok) a.out0[g] = gn;
+        if (a.trace) {
+            const double den = dr * dr + eta * eta;
+            acc += ok ? den * (gn.x * gn.x + gn.y * gn.y) : 0.0;
+        }
+    }
 }
 
 }  // namespace
@@ -115,7 +142,6 @@ __global__ __launch_bounds__(64 * HWY) void hstencil_kernel(const HArgs a)
     double wt[R + 1];
 #pragma unroll
     for (int o = 0; o <= R; o++) wt[o] = a.w[o];
-    const double eta = a.eta, om = a.omega, dlap = a.dlap;
 
     double2 q[PY][QN];
     struct Pre {
@@ -186,27 +212,8 @@ __global__ __launch_bounds__(64 * HWY) void hstencil_kernel(const HArgs a)
                 nb = cadd(nb, q[p][R + o]);
                 y = cadd(y, cscale(nb, wt[o]));
             }
-            const double ck = cur.cc[p];
-            const double2 au = helm_diag_add(y, u, ck, eta);
-            const bool ok = c_ok[p];
-            const int g = c_off[p] + zoff;
-            const double dr = __dadd_rn(dlap, ck);
-            if constexpr (MODE == HMode::MATVEC) {
-                if (ok) a.out0[g] = au;
-            } else if constexpr (MODE == HMode::TRUE_RES) {
-                const double2 f = make_double2(__dsub_rn(cur.bb[p].x, au.x), __dsub_rn(cur.bb[p].y, au.y));
-                acc += ok ? (f.x * f.x + f.y * f.y) : 0.0;
-                if (ok) a.out0[g] = cdiv_d(f, dr, eta);
-            } else {
-                // g' = g - omega (A g)/D; |D g'|^2 = ||b - A x'||^2 at the point
-                const double2 t = cdiv_d(au, dr, eta);
-                const double2 gn = make_double2(__dsub_rn(u.x, __dmul_rn(om, t.x)), __dsub_rn(u.y, __dmul_rn(om, t.y)));
-                if (ok) a.out0[g] = gn;
-                if (a.trace) {
-                    const double den = dr * dr + eta * eta;
-                    acc += ok ? den * (gn.x * gn.x + gn.y * gn.y) : 0.0;
-                }
-            }
+            const double2 b = NEED_B ? cur.bb[p] : make_double2(0.0, 0.0);
+            helm_point<MODE>(a, y, u, b, cur.cc[p], c_ok[p], c_off[p] + zoff, acc);
         }
 #pragma unroll
         for (int p = 0; p < PY; p++)
@@ -228,9 +235,141 @@ __global__ __launch_bounds__(64 * HWY) void hstencil_kernel(const HArgs a)
     }
 }
 
+// ---------------------------------------------------------------------------
+// One-shot boxes for the smaller grids (see stencil_tile.h): 32 x 16 x LZ
+// points a block, one column of LZ points a thread, all planes staged at once
+// behind one barrier.  Bound by the chain of loads, one barrier and the 37
+// ordered additions a block; at 96^3 (884736 points, 864 blocks of 8 waves)
+// the recurrence sweep takes 15.5 us, the march 40 (its reads from HBM alone take
+// 6).  A narrower 32 x 8 box
+// loads 1.9 halo values a point against 1.1 (96^3 36.7 us with its update
+// against 32.7).
+// ---------------------------------------------------------------------------
+constexpr int HBX = 32, HBY = 16, HBN = HBX * HBY;   // two rows a wavefront
+
+template <HMode MODE, int LZ>
+__global__ __launch_bounds__(HBN) void hstencil_box_kernel(const HArgs a)
+{
+    constexpr int NT = HBN, TY = HBY;
+    constexpr int LH = TY + 2 * R, LW = HBX + 2 * R;
+    constexpr int NYC = 2 * R * HBX, NXC = 2 * R * TY;
+    constexpr int NHC = LZ * (NYC + NXC), NH = (NHC + NT - 1) / NT;
+    constexpr int NQ = LZ + 2 * R;
+    constexpr bool NEED_B = MODE == HMode::TRUE_RES;
+
+    __shared__ double2 lds[LZ * LH][LW];
+    __shared__ double red_scratch[NT / 64];
+
+    if (a.ctrl && a.ctrl->done) return;
+
+    const int item = xcd_item(blockIdx.x, a.nitems);
+    const int itx = item % a.ntx;
+    const int rest = item / a.ntx;
+    const int x0 = itx * HBX, y0 = rest % a.nty * TY, z0 = rest / a.nty * LZ;
+    const int tid = threadIdx.x, tx = tid % HBX, ty = tid / HBX;
+    const int nx = a.nx, ny = a.ny, nz = a.nz, nxy = a.nxy;
+
+    const unsigned c_off = (unsigned)(hmodp(x0 + tx, nx) + hmodp(y0 + ty, ny) * nx);
+    const bool c_ok = (x0 + tx < nx) && (y0 + ty < ny);
+    size_t zo[NQ];                                   // planes z0-R .. z0+LZ-1+R (wrapped; uniform)
+    {
+        int z = hmodp(z0 - R, nz);
+#pragma unroll
+        for (int s = 0; s < NQ; s++) {
+            zo[s] = (size_t)z * nxy;
+            z = z + 1 == nz ? 0 : z + 1;
+        }
+    }
+    double2 q[NQ];
+#pragma unroll
+    for (int s = 0; s < NQ; s++) q[s] = (a.in0 + zo[s])[c_off];
+    // halo cell c of the box: plane, then 2R rows of HBX, then TY rows of R
+    // left and R right
+    double2 h[NH];
+    int h_row[NH], h_col[NH];
+#pragma unroll
+    for (int j = 0; j < NH; j++) {
+        const int c0 = tid + NT * j;
+        const int cc = c0 < NHC ? c0 : 0;
+        const int s = cc / (NYC + NXC), c = cc % (NYC + NXC);
+        int gx, gy;
+        if (c < NYC) {
+            const int r = c / HBX, w = c % HBX;
+            gx = x0 + w;
+            gy = r < R ? y0 - R + r : y0 + TY + (r - R);
+            h_row[j] = s * LH + (r < R ? r : TY + r);
+            h_col[j] = R + w;
+        } else {
+            const int r = (c - NYC) / (2 * R), w = (c - NYC) % (2 * R);
+            gx = w < R ? x0 - R + w : x0 + HBX + (w - R);
+            gy = y0 + r;
+            h_row[j] = s * LH + R + r;
+            h_col[j] = w < R ? w : HBX + w;
+        }
+        h[j] = a.in0[(unsigned)(hmodp(gx, nx) + hmodp(gy, ny) * nx) + (unsigned)hmodp(z0 + s, nz) * (unsigned)nxy];
+    }
+    double2 bb[LZ];
+    double ck[LZ];
+#pragma unroll
+    for (int s = 0; s < LZ; s++) {
+        if constexpr (NEED_B) bb[s] = (a.bvec + zo[R + s])[c_off];
+        ck[s] = a.c ? (a.c + zo[R + s])[c_off] : a.c0;
+    }
+#pragma unroll
+    for (int s = 0; s < LZ; s++) lds[s * LH + R + ty][R + tx] = q[R + s];
+#pragma unroll
+    for (int j = 0; j < NH; j++)
+        if (tid + NT * j < NHC) lds[h_row[j]][h_col[j]] = h[j];
+    __syncthreads();
+
+    double acc = 0.0;
+#pragma unroll
+    for (int s = 0; s < LZ; s++) {
+        if (z0 + s < nz) {                           // uniform: planes past the grid
+            const int lr = s * LH + R + ty, lc = R + tx;
+            const double2 u = q[R + s];
+            // system.c:195-201 order on each component
+            double2 y = cscale(cscale(u, 3.0), a.w[0]);
+#pragma unroll
+            for (int o = 1; o <= R; o++) {
+                double2 nb = cadd(lds[lr][lc - o], lds[lr][lc + o]);
+                nb = cadd(nb, lds[lr - o][lc]);
+                nb = cadd(nb, lds[lr + o][lc]);
+                nb = cadd(nb, q[R + s - o]);
+                nb = cadd(nb, q[R + s + o]);
+                y = cadd(y, cscale(nb, a.w[o]));
+            }
+            const double2 b = NEED_B ? bb[s] : make_double2(0.0, 0.0);
+            helm_point<MODE>(a, y, u, b, ck[s], c_ok, (int)(c_off + zo[R + s]), acc);
+        }
+    }
+    if (a.partials) {
+        double accv[1] = {acc};
+        block_reduce_to<1, NT>(accv, a.partials + (size_t)item, red_scratch);
+    }
+}
+
+// Where the boxes are faster than the march (recurrence sweep, its norm's
+// finish and a one-vector update, microseconds, march / boxes): 24^3 44.1 /
+// 12.8, 48^3 46.3 / 14.5, 64^3 48.2 / 15.9, 96^3 57.6 / 32.7, 128^3 72.6 /
+// 62.2, 144^3 84.6 / 89.6, 160^3 106 / 114, 256^3 379 / 435: the march's deep
+// columns leave most CUs idle on the small grids, the boxes' (LZ + 12)/LZ
+// reads a point cost more on the large ones.  Boxes of 2 planes while those of
+// 4 are one a CU or fewer (64^3 18.2 -> 15.9, 96^3 32.7 -> 34.3).
 static void hgeometry(HArgs &a)
 {
     a.nxy = a.nx * a.ny;
+    a.box = 0;
+    if (a.lz <= 0 && (long)a.nxy * a.nz <= 2500000L) {
+        const int tx = (a.nx + HBX - 1) / HBX, ty = (a.ny + HBY - 1) / HBY;
+        a.box = (long)tx * ty * ((a.nz + 3) / 4) <= 256 ? 2 : 4;
+        a.lz = a.box;
+        a.ntx = tx;
+        a.nty = ty;
+        a.nzc = (a.nz + a.lz - 1) / a.lz;
+        a.nitems = a.ntx * a.nty * a.nzc;
+        return;
+    }
     a.ntx = (a.nx + TX - 1) / TX;
     a.nty = (a.ny + HWY * HPY - 1) / (HWY * HPY);
     if (a.lz <= 0) {
@@ -251,15 +390,22 @@ int hstencil_items(const HArgs &a0)
     return a.nitems;
 }
 
+template <HMode M> static void launch_hsweep(const HArgs &a, hipStream_t st)
+{
+    const dim3 grid(a.nitems);
+    if (a.box == 2) hipLaunchKernelGGL((hstencil_box_kernel<M, 2>), grid, dim3(HBN), 0, st, a);
+    else if (a.box == 4) hipLaunchKernelGGL((hstencil_box_kernel<M, 4>), grid, dim3(HBN), 0, st, a);
+    else hipLaunchKernelGGL((hstencil_kernel<M>), grid, dim3(64 * HWY), 0, st, a);
+}
+
 hipError_t launch_hstencil(HMode m, const HArgs &a0, hipStream_t st)
 {
     HArgs a = a0;
     hgeometry(a);
-    dim3 grid(a.nitems), block(64 * HWY);
     switch (m) {
-    case HMode::MATVEC: hipLaunchKernelGGL((hstencil_kernel<HMode::MATVEC>), grid, block, 0, st, a); break;
-    case HMode::TRUE_RES: hipLaunchKernelGGL((hstencil_kernel<HMode::TRUE_RES>), grid, block, 0, st, a); break;
-    case HMode::REC: hipLaunchKernelGGL((hstencil_kernel<HMode::REC>), grid, block, 0, st, a); break;
+    case HMode::MATVEC: launch_hsweep<HMode::MATVEC>(a, st); break;
+    case HMode::TRUE_RES: launch_hsweep<HMode::TRUE_RES>(a, st); break;
+    case HMode::REC: launch_hsweep<HMode::REC>(a, st); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
