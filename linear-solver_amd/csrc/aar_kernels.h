@@ -322,8 +322,19 @@ hipError_t launch_helm_grad_c(long n, const double2 *lambda, const double2 *u, d
 // counter, or only write per-block partials when counter == nullptr; then
 // launch_finish (or, for the Gram, launch_gram itself) runs a one-block
 // second pass.
+//
+// A residual norm that is only recorded needs no finish of its own: the sweeps
+// between two checks leave their partials in consecutive sets, and the finish
+// of the next check sums them too, one more block each: hist[it0-1+j] =
+// sqrt(sum of set j), j < count.  partials == nullptr: the record alone.
+struct TraceFin {
+    const double *partials = nullptr;
+    int nitems = 0, count = 0, it0 = 0;
+    double *hist = nullptr;
+    int hist_cap = 0;
+};
 hipError_t launch_finish(const double *partials, int nitems, int nacc, const FinArgs &fin, Ctrl *ctrl,
-                         hipStream_t st);
+                         hipStream_t st, const TraceFin &trace = TraceFin());
 
 // small pointwise helpers
 hipError_t launch_copy_f64(double *dst, const double *src, long n, const Ctrl *ctrl, hipStream_t st);

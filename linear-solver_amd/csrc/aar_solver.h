@@ -125,8 +125,36 @@ int aar_petsc_solve(const Op &op, double *x, const double *b, double omega, doub
                     int max_iter, double tol, int precond, aar_hip_stats *st);
 int pgr_petsc_solve(const Op &op, double *x, const double *b, double omega, int m, int p, int max_iter, double tol,
                     int precond, int l2, aar_hip_stats *st);
+// Residual norms of the sweeps between two checks, recorded by the finish of
+// the next check (TraceFin); `cap` sets of `items` partials from `part` on.
+struct Trace {
+    TraceFin f;
+    double *part = nullptr;
+    int cap = 0;
+    Trace(double *part_, int items, int cap_, double *hist, int hist_cap) : part(part_), cap(cap_)
+    {
+        f.partials = part;
+        f.nitems = items;
+        f.hist = hist;
+        f.hist_cap = hist_cap;
+    }
+    bool full() const { return f.count == cap; }
+    // the partials of the sweep that makes iterate it
+    double *add(int it)
+    {
+        if (f.count == 0) f.it0 = it;
+        return part + (size_t)f.count++ * f.nitems;
+    }
+    TraceFin take()
+    {
+        const TraceFin t = f;
+        f.count = 0;
+        return t;
+    }
+};
+constexpr int TRACE_CAP = 64;          // sets kept at most (longer cycles are recorded in parts)
 template <typename T>
-int run_stencil(SMode mode, SArgs<T> a, double bytes);
+int run_stencil(SMode mode, SArgs<T> a, double bytes, Trace *tr = nullptr);
 template <typename T>
 int matvec(const Op &op, const T *x, T *y);
 int aar_refined(const Op &op, double *x, const double *b, double omega, double beta, int m, int p,

@@ -295,17 +295,35 @@ static const char *smode_name(SMode m)
 // kernel (counter + device-scope fence) or, in two-pass mode, in a one-block
 // second kernel; the choice is a measured tuning option.  The stencil sweeps
 // always finish in a second kernel.
+//
+// The sums of a sweep whose norm is only recorded (AAR_REC, PGR_STEP) wait in
+// `tr` for the next finish.
+static hipError_t flush_trace(Trace &tr)
+{
+    if (tr.f.count == 0) return hipSuccess;
+    return launch_finish(nullptr, 0, 1, FinArgs{}, nullptr, ctx().stream, tr.take());
+}
+
+static hipError_t finish_or_defer(const double *partials, int nitems, int nacc, const FinArgs &fin, Ctrl *ctrl,
+                                  bool deferred, Trace *tr)
+{
+    if (deferred) return tr->full() ? flush_trace(*tr) : hipSuccess;
+    return launch_finish(partials, nitems, nacc, fin, ctrl, ctx().stream, tr ? tr->take() : TraceFin());
+}
+
 template <typename T>
-int run_stencil(SMode mode, SArgs<T> a, double bytes)
+int run_stencil(SMode mode, SArgs<T> a, double bytes, Trace *tr)
 {
     Context &C = ctx();
     const Shape sh = stencil_shape(a.nx, a.ny, a.nz, sizeof(T));
+    const bool defer = tr && (mode == SMode::AAR_REC || mode == SMode::PGR_STEP);
+    if (defer) a.partials = tr->add(a.fin.it);
     prof_begin(smode_name(mode));
     hipError_t e = launch_stencil<T>(mode, a, sh, C.stream);
     prof_end(bytes);
     if (a.partials && e == hipSuccess)
-        e = launch_finish(a.partials, stencil_items<T>(a, sh), mode == SMode::CG_RESID ? 2 : 1, a.fin,
-                          a.ctrl, C.stream);
+        e = finish_or_defer(a.partials, stencil_items<T>(a, sh), mode == SMode::CG_RESID ? 2 : 1, a.fin, a.ctrl,
+                            defer, tr);
     if (e != hipSuccess) return fail(AAR_HIP_ERR_HIP, std::string("stencil launch: ") + hipGetErrorString(e));
     C.bytes_acc += bytes;
     return 0;
@@ -337,13 +355,14 @@ static hipError_t run_gram(GramArgs<T> g, double bytes)
     return e;
 }
 
-static hipError_t run_pgr_update(PUpdArgs<double> u)
+static hipError_t run_pgr_update(PUpdArgs<double> u, Trace &tr)
 {
     Context &C = ctx();
     const bool two = C.two_pass;
     if (two) u.counter = nullptr;
     hipError_t e = launch_pgr_update<double>(u, C.stream);
-    if (two && e == hipSuccess) e = launch_finish(u.partials, u.nblocks, 1, u.fin, u.ctrl, C.stream);
+    if (e == hipSuccess)
+        e = two ? launch_finish(u.partials, u.nblocks, 1, u.fin, u.ctrl, C.stream, tr.take()) : flush_trace(tr);
     return e;
 }
 
@@ -566,10 +585,12 @@ int aar_rec(const Op &op, Tx *x, const Tx *b, double omega, double beta, int m, 
     const size_t need = std::max<size_t>(
         std::max((size_t)stencil_partials_needed<Tg>(op), (size_t)stencil_partials_needed<Tx>(op)), (size_t)nb * GRAM_NA_MAX);
     DevBuf &PB = ci == 0 ? C.part0 : C.part1;
-    HC(ensure(PB, sizeof(double) * need));
+    const int titems = stencil_partials_needed<Tg>(op) / 2, tcap = std::min(p, TRACE_CAP);
+    HC(ensure(PB, sizeof(double) * (need + (size_t)titems * tcap)));
     Tg *G = (Tg *)RG.p;
     Tg *CR = NC > 0 ? (Tg *)RC.p : nullptr;
     double *hist = (double *)HB.p, *part = (double *)PB.p;
+    Trace tr(part + need, titems, tcap, hist, max_iter + 4);
     Ctrl *ctrl = C.ctrl + ci;
     unsigned *cnt = C.counters + 8 * ci;
     auto gs = [&](long k) { return (int)(k % S); };
@@ -603,7 +624,7 @@ int aar_rec(const Op &op, Tx *x, const Tx *b, double omega, double beta, int m, 
         a.fin.check = check;
         a.fin.hist = hist;
         a.fin.hist_cap = max_iter + 4;
-        return run_stencil<Tx>(SMode::AAR_TRUE, a, 2 * sx + sg + sv_true);
+        return run_stencil<Tx>(SMode::AAR_TRUE, a, 2 * sx + sg + sv_true, &tr);
     };
 
     HC(launch_zero_ctrl(ctrl, C.stream));
@@ -654,14 +675,9 @@ int aar_rec(const Op &op, Tx *x, const Tx *b, double omega, double beta, int m, 
             a.in0 = gptr(it);
             a.out0 = gptr(it + 1);
             a.trace = 1;
-            a.partials = part;
             a.ctrl = ctrl;
-            a.fin.fin = FIN_AAR_RES;
             a.fin.it = (int)it + 1;
-            a.fin.check = 0;
-            a.fin.hist = hist;
-            a.fin.hist_cap = max_iter + 4;
-            if (int rc = run_stencil<Tg>(SMode::AAR_REC, a, 2 * sg + sv_rec)) return rc;
+            if (int rc = run_stencil<Tg>(SMode::AAR_REC, a, 2 * sg + sv_rec, &tr)) return rc;
             // a residual that no Anderson window will read again is folded
             // into the anchor before its slot is reused (only when p > m+1)
             if (it < next_and(it) - m) {
@@ -763,6 +779,7 @@ int aar_rec(const Op &op, Tx *x, const Tx *b, double omega, double beta, int m, 
         prof_end(2 * sx + sg * u.ng);
         C.bytes_acc += 2 * sx + sg * u.ng;
     }
+    HC(flush_trace(tr));
     HC(hipEventRecord(C.t1, C.stream));
     Ctrl &hc = C.ctrl_h[ci];
     if (int rc = finish_ctrl(ctrl, &hc)) return rc;
@@ -804,7 +821,7 @@ template int aar_solve<double>(const Op &, double *, const double *, double, dou
 template SArgs<double> base_sargs<double>(const Op &);
 template SArgs<float> base_sargs<float>(const Op &);
 template hipError_t run_dot<double>(DotArgs<double>);
-template int run_stencil<double>(SMode, SArgs<double>, double);
+template int run_stencil<double>(SMode, SArgs<double>, double, Trace *);
 template int aar_solve<float>(const Op &, float *, const float *, double, double, int, int, int, double,
                               int, int, aar_hip_stats *, int, int);
 
@@ -828,9 +845,11 @@ int pgr_solve(const Op &op, double *x, const double *b, double omega, int m, int
     HC(ensure(C.hist0, sizeof(double) * (size_t)(max_iter + 4)));
     const int nb = nblocks_for(n);
     const size_t need = std::max<size_t>((size_t)stencil_partials_needed<double>(op), (size_t)nb * GRAM_NA_MAX);
-    HC(ensure(C.part0, sizeof(double) * need));
+    const int titems = stencil_partials_needed<double>(op) / 2, tcap = std::min(p, TRACE_CAP - 2) + 2;
+    HC(ensure(C.part0, sizeof(double) * (need + (size_t)titems * tcap)));
     double *X = (double *)C.ring64x.p, *Y = (double *)C.ring64f.p;
     double *hist = (double *)C.hist0.p, *part = (double *)C.part0.p;
+    Trace tr(part + need, titems, tcap, hist, max_iter + 4);
     Ctrl *ctrl = C.ctrl;
     unsigned *cnt = C.counters;
     auto slot = [&](long t) { return (int)(t % ns); };
@@ -867,14 +886,9 @@ int pgr_solve(const Op &op, double *x, const double *b, double omega, int m, int
         a.bvec = b;
         a.out0 = Y + (size_t)slot(t + 1) * ld;
         a.out1 = next ? X + (size_t)slot(t + 2) * ld : nullptr;
-        a.partials = part;
         a.ctrl = ctrl;
-        a.fin.fin = FIN_AAR_RES;
         a.fin.it = t + 1;
-        a.fin.check = 0;
-        a.fin.hist = hist;
-        a.fin.hist_cap = max_iter + 4;
-        return run_stencil<double>(SMode::PGR_STEP, a, s_b * (next ? 4 : 3) + vcb);
+        return run_stencil<double>(SMode::PGR_STEP, a, s_b * (next ? 4 : 3) + vcb, &tr);
     };
     if (int rc = step(0)) return rc;                                // PGR.c:79-81
     int cyc = 0;
@@ -923,7 +937,7 @@ int pgr_solve(const Op &op, double *x, const double *b, double omega, int m, int
             u.fin.check = 1;
             u.fin.hist = nullptr;
             prof_begin("pgr_update");
-            HC(run_pgr_update(u));
+            HC(run_pgr_update(u, tr));
             const double by = s_b * (2 * (nv + 1) + 3 + (u.next >= 0 ? 1 : 0)) + (u.next >= 0 ? vcb : 0.0);
             prof_end(by);
             C.bytes_acc += s_b * ((l2 ? 1 : 2) * (nv + 1) + 1) + by;
@@ -932,6 +946,7 @@ int pgr_solve(const Op &op, double *x, const double *b, double omega, int m, int
             cyc++;
         }
     }
+    HC(flush_trace(tr));
     HC(hipEventRecord(C.t1, C.stream));
     Ctrl &hc = C.ctrl_h[0];
     if (int rc = finish_ctrl(ctrl, &hc)) return rc;
@@ -1178,14 +1193,16 @@ static const char *hmode_name(HMode m)
     return "helm";
 }
 
-static int run_hstencil(HMode mode, const HArgs &a, double bytes)
+static int run_hstencil(HMode mode, HArgs a, double bytes, Trace *tr = nullptr)
 {
     Context &C = ctx();
+    const bool defer = tr && mode == HMode::REC;
+    if (defer) a.partials = tr->add(a.fin.it);
     prof_begin(hmode_name(mode));
     hipError_t e = launch_hstencil(mode, a, C.stream);
     prof_end(bytes);
     if (e == hipSuccess && a.partials)
-        e = launch_finish(a.partials, hstencil_items(a), 1, a.fin, a.ctrl, C.stream);
+        e = finish_or_defer(a.partials, hstencil_items(a), 1, a.fin, a.ctrl, defer, tr);
     if (e != hipSuccess) return fail(AAR_HIP_ERR_HIP, std::string("helmholtz stencil launch: ") + hipGetErrorString(e));
     C.bytes_acc += bytes;
     return 0;
@@ -1233,13 +1250,15 @@ int helm_solve(const HOp &op, double *u, const double *b, double omega, double b
     HC(ensure(C.hist0, sizeof(double) * (size_t)(max_iter + 4)));
     const int nb = nblocks_for(n);
     HArgs probe = base_hargs(op);
-    const size_t need = std::max<size_t>((size_t)hstencil_items(probe), (size_t)nb * HGRAM_NA_MAX);
-    HC(ensure(C.part0, sizeof(double) * need));
+    const int titems = hstencil_items(probe), tcap = std::min(p, TRACE_CAP);
+    const size_t need = std::max<size_t>((size_t)titems, (size_t)nb * HGRAM_NA_MAX);
+    HC(ensure(C.part0, sizeof(double) * (need + (size_t)titems * tcap)));
     double2 *G = (double2 *)C.ringc.p;
     double2 *CR = NC > 0 ? (double2 *)C.corrc.p : nullptr;
     double2 *x = (double2 *)u;
     const double2 *bb = (const double2 *)b;
     double *hist = (double *)C.hist0.p, *part = (double *)C.part0.p;
+    Trace tr(part + need, titems, tcap, hist, max_iter + 4);
     Ctrl *ctrl = C.ctrl;
     unsigned *cnt = C.counters;
     auto gs = [&](long k) { return (int)(k % S); };
@@ -1261,7 +1280,7 @@ int helm_solve(const HOp &op, double *u, const double *b, double omega, double b
         a.fin.check = check;
         a.fin.hist = hist;
         a.fin.hist_cap = max_iter + 4;
-        return run_hstencil(HMode::TRUE_RES, a, 3 * sv + sc);
+        return run_hstencil(HMode::TRUE_RES, a, 3 * sv + sc, &tr);
     };
     auto anchor = [&](HAncArgs &hu, double bytes) -> int {
         prof_begin("helm_anchor_update");
@@ -1300,14 +1319,9 @@ int helm_solve(const HOp &op, double *u, const double *b, double omega, double b
             a.in0 = gptr(it);
             a.out0 = gptr(it + 1);
             a.trace = 1;
-            a.partials = part;
             a.ctrl = ctrl;
-            a.fin.fin = FIN_AAR_RES;
             a.fin.it = (int)it + 1;
-            a.fin.check = 0;
-            a.fin.hist = hist;
-            a.fin.hist_cap = max_iter + 4;
-            if (int rc = run_hstencil(HMode::REC, a, 2 * sv + sc)) return rc;
+            if (int rc = run_hstencil(HMode::REC, a, 2 * sv + sc, &tr)) return rc;
             if (it < next_and(it) - m) {
                 HAncArgs hu;
                 hu.n = n;
@@ -1401,6 +1415,7 @@ int helm_solve(const HOp &op, double *u, const double *b, double omega, double b
         hu.ctrl = ctrl;
         if (int rc = anchor(hu, sv * (2 + hu.ng))) return rc;
     }
+    HC(flush_trace(tr));
     HC(hipEventRecord(C.t1, C.stream));
     Ctrl &hc = C.ctrl_h[0];
     if (int rc = finish_ctrl(ctrl, &hc)) return rc;

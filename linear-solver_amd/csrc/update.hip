@@ -640,23 +640,67 @@ hipError_t launch_cg(CgStep step, const CgArgs &a, hipStream_t st)
 // ---------------------------------------------------------------------------
 // second pass of a reduction: one block sums per-block partials in a fixed
 // order and runs the finaliser (no device-scope fence or atomic needed: the
-// kernel boundary orders it after the partials)
+// kernel boundary orders it after the partials); further blocks sum the
+// recorded norms (TraceFin).  A launch is a chain of latencies, 2.8-4.6 us
+// whatever it sums: one per check instead of one per sweep takes AAR at
+// 48^3 from 6.48 to 5.74 ms, complex AAR with gradients at 96^3 28.8 -> 27.4.
+// A record does not wait for `done`: block 0 may set it meanwhile, and what a
+// sweep skipped after convergence leaves lies past the history that is read.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(BLOCK) void finish_kernel(const double *partials, int nitems, int nacc, FinArgs fin,
-                                                      Ctrl *ctrl)
+template <int NT, int NACC>
+__global__ __launch_bounds__(NT) void finish_kernel(const double *partials, int nitems, FinArgs fin, Ctrl *ctrl,
+                                                    const TraceFin tr)
 {
-    __shared__ double scratch[BLOCK / 64];
-    __shared__ double sums[8];
-    if (ctrl->done) return;
-    final_sum(partials, nitems, nacc, sums, scratch);
-    if (threadIdx.x == 0) finalize(fin, ctrl, sums, nacc);
+    __shared__ double scratch[NACC * (NT / 64)];
+    __shared__ double sums[NACC];
+    if (blockIdx.x > 0) {
+        const int j = blockIdx.x - 1, i = tr.it0 - 1 + j;
+        final_sum<NT>(tr.partials + (size_t)j * tr.nitems, tr.nitems, 1, sums, scratch);
+        if (threadIdx.x == 0 && i >= 0 && i < tr.hist_cap) tr.hist[i] = sqrt(sums[0]);
+        return;
+    }
+    if (!partials || ctrl->done) return;
+    // every value's sum in one pass, in final_sum's order
+    double acc[NACC];
+#pragma unroll
+    for (int k = 0; k < NACC; k++) acc[k] = 0.0;
+#pragma unroll 4
+    for (int i = threadIdx.x; i < nitems; i += NT)
+#pragma unroll
+        for (int k = 0; k < NACC; k++) acc[k] += partials[(size_t)i * NACC + k];
+#pragma unroll
+    for (int k = 0; k < NACC; k++) {
+        acc[k] = wave_sum(acc[k]);
+        if ((threadIdx.x & 63) == 0) scratch[k * (NT / 64) + (threadIdx.x >> 6)] = acc[k];
+    }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+#pragma unroll
+    for (int k = 0; k < NACC; k++) {
+        double t = 0.0;
+        for (int w = 0; w < NT / 64; w++) t += scratch[k * (NT / 64) + w];
+        sums[k] = t;
+    }
+    finalize(fin, ctrl, sums, NACC);
 }
 
 hipError_t launch_finish(const double *partials, int nitems, int nacc, const FinArgs &fin, Ctrl *ctrl,
-                         hipStream_t st)
+                         hipStream_t st, const TraceFin &tr)
 {
-    if (nacc < 1 || nacc > 8) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(finish_kernel, dim3(1), dim3(BLOCK), 0, st, partials, nitems, nacc, fin, ctrl);
+    if (nacc < 1 || nacc > 2) return hipErrorInvalidValue;
+    const dim3 grid(1 + tr.count);
+    // sixteen wavefronts once four would walk more than a few dozen partials
+    // each (CG at 250 x 256 x 243, 7594 pairs a residual: 369 -> 356 ms)
+    auto go = [&](auto nt, auto na) {
+        constexpr int NT = decltype(nt)::value, NA = decltype(na)::value;
+        hipLaunchKernelGGL((finish_kernel<NT, NA>), grid, dim3(NT), 0, st, partials, nitems, fin, ctrl, tr);
+    };
+    using std::integral_constant;
+    const bool big = nitems > 2048;
+    if (nacc == 1 && !big) go(integral_constant<int, BLOCK>{}, integral_constant<int, 1>{});
+    else if (nacc == 1) go(integral_constant<int, 1024>{}, integral_constant<int, 1>{});
+    else if (!big) go(integral_constant<int, BLOCK>{}, integral_constant<int, 2>{});
+    else go(integral_constant<int, 1024>{}, integral_constant<int, 2>{});
     return hipGetLastError();
 }
 
