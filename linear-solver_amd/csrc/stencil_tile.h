@@ -153,8 +153,12 @@ __device__ __forceinline__ void stencil_box(const SArgs<T> &a, const int item, t
                 };
                 auto zn = [&](int d) -> Vec { return q[p][R + s + d]; };
                 const Vec y = stencil_value<T, MODE, VC>(a, k, xw, vv[p][s], yn, zn);
+                // PGR's two outputs wait a projection cycle: non-temporal
+                // (128^3 103.2 -> 100.5 ms a solve; the other modes' output
+                // is the next sweep's input, and they lose 0.3%)
+                constexpr bool NT_OUT = MODE == SMode::PGR_STEP;
                 auto put = [&](auto *base, const auto &o) {
-                    st_vec<std::remove_pointer_t<decltype(base)>, false, T, EDGE>(base + zo[R + s], c_off[p], o,
+                    st_vec<std::remove_pointer_t<decltype(base)>, NT_OUT, T, EDGE>(base + zo[R + s], c_off[p], o,
                                                                                   c_ok[p], true);
                 };
                 stencil_epilogue<T, MODE, VC, EDGE>(a, k, y, u, en[p][s], vv[p][s], c_ok[p], put, acc);
