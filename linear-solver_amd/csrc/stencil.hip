@@ -41,36 +41,39 @@ namespace aar {
 // host-side launch
 // ---------------------------------------------------------------------------
 
-// Rows of a one-shot box: four wavefronts, one row per thread.
-template <typename T> constexpr int TILE_ROWS = 4 * Lane<T>::RPW;
+// Rows of a one-shot box: four wavefronts, one vector per thread.
+template <typename T> static int tile_rows(int lz) { return 256 * Lane<T>::V / tile_x<T>(lz); }
 
-// Where the boxes are faster than the march (recurrence sweep, microseconds
-// with the launch, best march shape against the boxes): FP64 48^3 8.4 / 5.2,
-// 96^3 11.7 / 12.7, 128^3 14.0 / 15.8, 160^3 30.8 / 27.9, 200 x 161 x 150
-// 33.8 / 35.2, 200^3 54.8 / 54.2, 256^3 67 / 103; FP32 48^3 7.9 / 4.9, 96^3
-// 9.5 / 8.3, 160^3 17.4 / 16.3, 200^3 29.6 / 28.8, 256^3 41 / 50.  The two
-// meet at about 8 million points; near the tie the boxes need no depth chosen
-// to fit.  Boxes of 4 planes read (4 + 12)/4 values a point; while they are
-// about one a CU or fewer, boxes of 2 planes are shorter (FP32 96^3 8.7 ->
-// 8.3 us, FP64 true residual 64^3 7.9 -> 6.2; 128^3 15.8 -> 16.8), and of one
-// plane while those leave half the CUs idle (48^3 5.2 -> 4.9, FP32 4.9 ->
-// 4.4, 16^3 4.9 -> 4.0; FP64 64^3 8.2 -> 8.5).  32-bit offsets span the grid.
+// Where the boxes are faster than the march (recurrence sweep; FP64 with a
+// one-vector update, microseconds, march of 64 x 16 columns against boxes):
+// FP64 48^3 20.1 / 9.5, 96^3 24.4 / 15.4, 128^3 30.3 / 26.3, 160^3 43.9 / 44.3,
+// 200 x 161 x 150 56.2 / 57.4, 200^3 86.3 / 88.6, 256^3 (sweep alone) 67 / 103;
+// FP32 (sweep alone) 48^3 7.9 / 4.9, 96^3 9.5 / 8.3, 160^3 17.4 / 16.3, 200^3
+// 29.6 / 28.8, 256^3 41 / 50.  The two meet at about 8 million points; near the
+// tie the boxes need no depth chosen to fit.  Boxes of 4 planes read (4 + 12)/4
+// values a point; while they are about one a CU or fewer, boxes of 2 planes are
+// shorter (FP32 96^3 8.7 -> 8.3 us, FP64 true residual 64^3 7.9 -> 6.2; 128^3
+// 15.8 -> 16.8), and of one plane while those leave half the CUs idle (48^3
+// 5.2 -> 4.9, FP32 4.9 -> 4.4, 16^3 4.9 -> 4.0; FP64 64^3 8.2 -> 8.5).  32-bit
+// offsets span the grid.
 template <typename T>
 int stencil_tile_planes(int nx, int ny, int nz)
 {
     const long n = (long)nx * ny * nz;
     if (n > 8500000L) return 0;
-    const long cols = (long)((nx + TX - 1) / TX) * ((ny + TILE_ROWS<T> - 1) / TILE_ROWS<T>);
-    if (cols * ((nz + 1) / 2) <= 150) return 1;
-    return cols * ((nz + 3) / 4) <= 300 ? 2 : 4;
+    auto cols = [&](int lz) {
+        return (long)((nx + tile_x<T>(lz) - 1) / tile_x<T>(lz)) * ((ny + tile_rows<T>(lz) - 1) / tile_rows<T>(lz));
+    };
+    if (cols(1) * ((nz + 1) / 2) <= 150) return 1;
+    return cols(4) * ((nz + 3) / 4) <= 300 ? 2 : 4;
 }
 
 template <typename T>
 void stencil_geometry(SArgs<T> &a, const Shape &sh)
 {
-    const int ty = sh.tile ? TILE_ROWS<T> : sh.wy * sh.py;
+    const int tx = sh.tile ? tile_x<T>(sh.tile) : TX, ty = sh.tile ? tile_rows<T>(sh.tile) : sh.wy * sh.py;
     a.nxy = a.nx * a.ny;
-    a.ntx = (a.nx + TX - 1) / TX;
+    a.ntx = (a.nx + tx - 1) / tx;
     a.nty = (a.ny + ty - 1) / ty;
     if (sh.tile) {
         a.lz = sh.tile;

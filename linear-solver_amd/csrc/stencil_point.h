@@ -54,6 +54,14 @@ template <typename T> struct Lane {
     typedef T VecU __attribute__((ext_vector_type(V), aligned(sizeof(T))));
 };
 
+// Width of a one-shot box of lz planes.  FP64 boxes of 2 and 4 planes are 32 x
+// 16 points: 1.1 halo values a point against 1.7 of 64 x 8, and less of a tile
+// past an x-side (recurrence sweep with a one-vector update, 64 wide / 32: 96^3
+// 16.9 / 15.4 us, 160^3 48.3 / 44.3, 200^3 93.2 / 88.6; PGR at 128^3 103.5 ->
+// 99.8 ms).  One plane: 64 x 8 (AAR at 48^3 5.80 ms, 32 wide 5.87).  FP32 64 x
+// 16 (32 x 32: 200 x 161 x 150 32.1 -> 32.9 us, 96^3 14.4 -> 13.7).
+template <typename T> __host__ __device__ constexpr int tile_x(int lz) { return sizeof(T) == 8 && lz > 1 ? 32 : 64; }
+
 // base[off] with a uniform (per-plane) base pointer and a 32-bit in-plane
 // offset: the access compiles to the scalar-base + vector-offset form, with
 // no per-access 64-bit address arithmetic (in-plane byte offsets are below
@@ -99,10 +107,10 @@ __device__ __forceinline__ typename Lane<T>::Vec ld_vec(const T *base, const VOf
 
 // An edge tile's x-window reaches past nx while nx is not a whole number of
 // vectors: its vectors may wrap inside and are accessed point by point.
-template <typename T> __device__ __forceinline__ bool edge_tile(const SArgs<T> &a, int item)
+template <typename T, int W = TX> __device__ __forceinline__ bool edge_tile(const SArgs<T> &a, int item)
 {
     using L = Lane<T>;
-    return a.nx % L::V != 0 && (item % a.ntx) * TX + TX + L::HXV * L::V > a.nx;
+    return a.nx % L::V != 0 && (item % a.ntx) * W + W + L::HXV * L::V > a.nx;
 }
 
 // S: the stored type (T, or float for the FP32 copy of an FP64 sweep).

@@ -3,7 +3,7 @@
 //
 // The march of stencil_body.h wants one deep column per CU: on a grid of a
 // few million points it leaves most CUs idle and walks its planes one
-// barrier at a time.  Here a block of WY wavefronts takes a 64 x TY x LZ box
+// barrier at a time.  Here a block of WY wavefronts takes a BX x TY x LZ box
 // and stages all its planes at once: every thread issues the loads of its PY
 // columns of vectors (LZ + 2R planes, kept in registers for the
 // z-neighbours) and of its share of the x/y halo vectors, parks the box
@@ -19,13 +19,15 @@ namespace aar {
 template <typename T, int WY, int PY, int LZ> struct Tile {
     using L = Lane<T>;
     static constexpr int NT = 64 * WY;
-    static constexpr int TY = WY * L::RPW * PY;
+    static constexpr int BX = tile_x<T>(LZ), LPR = BX / L::V, RPW = 64 / LPR;
+    static constexpr int LW = BX + 2 * L::HXV * L::V;
+    static constexpr int TY = WY * RPW * PY;
     static constexpr int LH = TY + 2 * R;
-    static constexpr int NYC = 2 * R * L::LPR, NXC = TY * 2 * L::HXV;
+    static constexpr int NYC = 2 * R * LPR, NXC = TY * 2 * L::HXV;
     static constexpr int NHC = LZ * (NYC + NXC);                   // halo vectors of the box
     static constexpr int NH = (NHC + NT - 1) / NT;
     struct Lds {
-        typename L::Vec tile[LZ * LH][L::LW / L::V];
+        typename L::Vec tile[LZ * LH][LW / L::V];
         double red[2 * WY];
     };
 };
@@ -37,7 +39,7 @@ __device__ __forceinline__ void stencil_box(const SArgs<T> &a, const int item, t
     using L = Lane<T>;
     using Vec = typename L::Vec;
     using Off = VOff<T, EDGE>;
-    constexpr int V = L::V, LPR = L::LPR, HXV = L::HXV;
+    constexpr int V = L::V, LPR = B::LPR, HXV = L::HXV, BX = B::BX;
     constexpr int NT = B::NT, TY = B::TY, NHC = B::NHC, NH = B::NH;
     constexpr int NE = ModeInfo<MODE>::NE;
     constexpr int NACC = ModeInfo<MODE>::NACC;
@@ -47,10 +49,10 @@ __device__ __forceinline__ void stencil_box(const SArgs<T> &a, const int item, t
     const int rest = item / a.ntx;
     const int ity = rest % a.nty;
     const int izc = rest / a.nty;
-    const int x0 = itx * TX, y0 = ity * TY, z0 = izc * LZ;
+    const int x0 = itx * BX, y0 = ity * TY, z0 = izc * LZ;
     const int tid = threadIdx.x, lane = tid & 63;
     const int xv = lane % LPR;
-    const int r0 = ((tid >> 6) * L::RPW + lane / LPR) * PY;
+    const int r0 = ((tid >> 6) * B::RPW + lane / LPR) * PY;
     const int nx = a.nx, ny = a.ny, nz = a.nz, nxy = a.nxy;
 
     const PointK<T> k(a);
@@ -95,7 +97,7 @@ __device__ __forceinline__ void stencil_box(const SArgs<T> &a, const int item, t
             h_col[j] = HXV + w;
         } else {
             const int r = (c - B::NYC) / (2 * HXV), w = (c - B::NYC) % (2 * HXV);
-            off.set(w < HXV ? x0 - (HXV - w) * V : x0 + TX + (w - HXV) * V, y0 + r, nx, ny);
+            off.set(w < HXV ? x0 - (HXV - w) * V : x0 + BX + (w - HXV) * V, y0 + r, nx, ny);
             h_row[j] = s * B::LH + R + r;
             h_col[j] = w < HXV ? w : LPR + w;
         }
@@ -172,7 +174,7 @@ template <typename T, int WY, int PY, int LZ, SMode MODE, bool VC = false>
 __device__ __forceinline__ void stencil_tile_body(const SArgs<T> &a, const int item)
 {
     __shared__ typename Tile<T, WY, PY, LZ>::Lds S;
-    if (edge_tile(a, item)) stencil_box<T, WY, PY, LZ, MODE, VC, true>(a, item, S);
+    if (edge_tile<T, tile_x<T>(LZ)>(a, item)) stencil_box<T, WY, PY, LZ, MODE, VC, true>(a, item, S);
     else stencil_box<T, WY, PY, LZ, MODE, VC, false>(a, item, S);
 }
 
