@@ -94,11 +94,11 @@ __global__ __launch_bounds__(64 * BWY) void bstencil_kernel(const BInst<Tx, Tg> 
     stencil_body<T, BWY, BPY / Lane<T>::RPW, MODE>(sa, wi.idx);
 }
 
-// per-instance finish of the true residual: relres check at the Anderson
-// iteration it = *clock + jrel (FIN_AAR_RES of iterate it+1)
+// per-instance finish of the true residual: relres check (or, at the start, the
+// record alone) at the Anderson iteration it = *clock + jrel (FIN_AAR_RES of iterate it+1)
 template <typename Tx, typename Tg>
 __global__ __launch_bounds__(BLOCK) void bfinish_kernel(const BInst<Tx, Tg> *inst, const int *clock, int jrel,
-                                                        int max_iter, int *ndone)
+                                                        int check, int max_iter, int *ndone)
 {
     __shared__ double scratch[BLOCK / 64];
     __shared__ double out[1];
@@ -109,7 +109,7 @@ __global__ __launch_bounds__(BLOCK) void bfinish_kernel(const BInst<Tx, Tg> *ins
         FinArgs f = {};
         f.fin = FIN_AAR_RES;
         f.it = *clock + jrel + 1;
-        f.check = 1;
+        f.check = check;
         f.max_iter = max_iter;
         f.hist = I.hist;
         f.hist_cap = I.hist_cap;
@@ -321,13 +321,23 @@ __global__ __launch_bounds__(BLOCK) void banchor_kernel(const BInst<Tx, Tg> *ins
 __global__ void bclock_kernel(int *clock, int p) { if (threadIdx.x == 0 && blockIdx.x == 0) *clock += p; }
 __global__ void bset_kernel(int *v, int value) { if (threadIdx.x == 0 && blockIdx.x == 0) *v = value; }
 
-template <typename T>
-hipError_t bsp_alloc(T **p, size_t count, std::vector<void *> &owned)
-{
-    hipError_t e = hipMalloc((void **)p, sizeof(T) * std::max<size_t>(count, 1));
-    if (e == hipSuccess) owned.push_back(*p);
-    return e;
-}
+// A batch's buffers are cut from one allocation, laid out twice: first from
+// address zero for its size, then in place.
+struct Arena {
+    char *base = nullptr;
+    size_t used = 0;
+    template <typename T> T *take(size_t count)
+    {
+        T *p = reinterpret_cast<T *>(base + used);
+        used += (sizeof(T) * std::max<size_t>(count, 1) + 511) / 512 * 512;
+        return p;
+    }
+};
+
+// The allocation is kept for the next batch up to this size (40 systems of
+// sides 24 to 128 take 1.4 GB; allocating and freeing 240 buffers a call took
+// 15 ms of 64.7).
+constexpr size_t BATCH_KEEP = (size_t)4 << 30;
 
 }  // namespace
 
@@ -351,7 +361,6 @@ int batch_solve(const aar_hip_instance *ins, int count, double omega, double bet
     if (p < 1) return fail(AAR_HIP_ERR_ARG, "p must be >= 1");
     if (max_iter < 0) return fail(AAR_HIP_ERR_ARG, "max_iter must be >= 0");
     int rc = 0;
-    std::vector<void *> owned;
     std::vector<BInst<Tx, Tg>> hI(count);
     std::vector<Op> ops(count);
     std::vector<WorkItem> wtr, wrc, wch;
@@ -359,7 +368,7 @@ int batch_solve(const aar_hip_instance *ins, int count, double omega, double bet
     BInst<Tx, Tg> *dI = nullptr;
     WorkItem *dtr = nullptr, *drc = nullptr, *dch = nullptr;
     Ctrl *ctrls = nullptr;
-    int *clock = nullptr, *ndone = nullptr, *ndone_h = nullptr;
+    int *clock = nullptr, *ndone = nullptr, *const ndone_h = C.poll_h;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     const int S = m + 2;
@@ -382,73 +391,80 @@ int batch_solve(const aar_hip_instance *ins, int count, double omega, double bet
     BHC(hipEventCreateWithFlags(&ev_out, hipEventDisableTiming));
     BHC(hipEventRecord(ev_in, C.stream));
     BHC(hipStreamWaitEvent(st, ev_in, 0));
-    BHC(bsp_alloc(&ctrls, count, owned));
-    BHC(bsp_alloc(&clock, 1, owned));
-    BHC(hipHostMalloc((void **)&ndone_h, sizeof(int) * 64, hipHostMallocDefault));
-    BHC(bsp_alloc(&ndone, 1, owned));
-    for (int i = 0; i < count; i++) {
-        aar_hip_grid g = {ins[i].nx, ins[i].ny, ins[i].nz, 6, ins[i].a, ins[i].sigma};
-        if ((rc = make_op(&g, nullptr, ops[i]))) goto done;
-        if (!ins[i].x || !ins[i].b) {
-            rc = fail(AAR_HIP_ERR_ARG, "null vector in batch");
-            goto done;
+    for (int pass = 0; pass < 2; pass++) {
+        Arena ar;
+        if (pass == 1) ar.base = (char *)C.batch.p;
+        ctrls = ar.take<Ctrl>(count);
+        clock = ar.take<int>(1);
+        ndone = ar.take<int>(1);
+        wtr.clear();
+        wrc.clear();
+        wch.clear();
+        for (int i = 0; i < count; i++) {
+            aar_hip_grid g = {ins[i].nx, ins[i].ny, ins[i].nz, 6, ins[i].a, ins[i].sigma};
+            if ((rc = make_op(&g, nullptr, ops[i]))) goto done;
+            if (!ins[i].x || !ins[i].b) {
+                rc = fail(AAR_HIP_ERR_ARG, "null vector in batch");
+                goto done;
+            }
+            const Op &op = ops[i];
+            BInst<Tx, Tg> &I = hI[i];
+            I.n = op.n;
+            I.ld = ring_ld(op.n, sizeof(Tg));
+            I.S = S;
+            I.NC = NC;
+            I.x = (Tx *)ins[i].x;
+            I.ctrl = ctrls + i;
+            I.hist_cap = max_iter + 4;
+            I.G = ar.take<Tg>((size_t)I.ld * S);
+            if (NC > 0) I.C = ar.take<Tg>((size_t)I.ld * NC);
+            I.hist = ar.take<double>((size_t)I.hist_cap);
+            // stencil args (auto z-chunk for this grid and the batch launch shape)
+            // slab depth: the one fixed by aar_hip_set_tuning (its wy, py do not
+            // apply: the batch launch shape is 8 x 4), else tuned for the batched
+            // launch where available, else automatic; stencil_geometry clamps
+            // it to the instance's nz
+            auto batch_lz = [&](size_t es) {
+                if (C.tuning_set && C.lz > 0) return C.lz;
+                auto t = C.tuned_batch.find({op.nx, op.ny, op.nz, (int)es});
+                return t != C.tuned_batch.end() ? t->second.lz : auto_lz(op, BWY, BPY, es);
+            };
+            SArgs<Tx> tr = base_sargs<Tx>(op);
+            tr.lz = batch_lz(sizeof(Tx));
+            SArgs<Tg> rcg = base_sargs<Tg>(op);
+            rcg.lz = batch_lz(sizeof(Tg));
+            const int ntr = stencil_items<Tx>(tr, Shape{}), nrc = stencil_items<Tg>(rcg, Shape{});
+            stencil_geometry<Tx>(tr, Shape{});
+            stencil_geometry<Tg>(rcg, Shape{});
+            tr.omega = rcg.omega = omega;
+            tr.precond = rcg.precond = precond;
+            {
+                const double c = precond ? omega / op.diag : omega;
+                rcg.cf[0] = 1.0 - c * (3.0 * op.w[0] + op.sigma);
+                for (int o = 1; o <= R; o++) rcg.cf[o] = -c * op.w[o];
+            }
+            tr.in0 = I.x;
+            tr.bvec = (const Tx *)ins[i].b;
+            tr.ctrl = I.ctrl;
+            rcg.ctrl = I.ctrl;
+            I.nchunks = (int)((op.n + CHUNK - 1) / CHUNK);
+            const int nbd = nblocks_for(op.n);
+            I.spart = ar.take<double>((size_t)std::max({ntr, nrc, nbd}) * 2);
+            I.gpart = ar.take<double>((size_t)I.nchunks * NA);
+            tr.partials = I.spart;
+            I.tr = tr;
+            I.rc = rcg;
+            I.tr_items = ntr;
+            for (int t = 0; t < ntr; t++) wtr.push_back({i, t});
+            for (int t = 0; t < nrc; t++) wrc.push_back({i, t});
+            for (int t = 0; t < I.nchunks; t++) wch.push_back({i, t});
         }
-        const Op &op = ops[i];
-        BInst<Tx, Tg> &I = hI[i];
-        I.n = op.n;
-        I.ld = ring_ld(op.n, sizeof(Tg));
-        I.S = S;
-        I.NC = NC;
-        I.x = (Tx *)ins[i].x;
-        I.ctrl = ctrls + i;
-        I.hist_cap = max_iter + 4;
-        BHC(bsp_alloc(&I.G, (size_t)I.ld * S, owned));
-        if (NC > 0) BHC(bsp_alloc(&I.C, (size_t)I.ld * NC, owned));
-        BHC(bsp_alloc(&I.hist, (size_t)I.hist_cap, owned));
-        // stencil args (auto z-chunk for this grid and the batch launch shape)
-        // slab depth: the one fixed by aar_hip_set_tuning (its wy, py do not
-        // apply: the batch launch shape is 8 x 4), else tuned for the batched
-        // launch where available, else automatic; stencil_geometry clamps
-        // it to the instance's nz
-        auto batch_lz = [&](size_t es) {
-            if (C.tuning_set && C.lz > 0) return C.lz;
-            auto t = C.tuned_batch.find({op.nx, op.ny, op.nz, (int)es});
-            return t != C.tuned_batch.end() ? t->second.lz : auto_lz(op, BWY, BPY, es);
-        };
-        SArgs<Tx> tr = base_sargs<Tx>(op);
-        tr.lz = batch_lz(sizeof(Tx));
-        SArgs<Tg> rcg = base_sargs<Tg>(op);
-        rcg.lz = batch_lz(sizeof(Tg));
-        const int ntr = stencil_items<Tx>(tr, Shape{}), nrc = stencil_items<Tg>(rcg, Shape{});
-        stencil_geometry<Tx>(tr, Shape{});
-        stencil_geometry<Tg>(rcg, Shape{});
-        tr.omega = rcg.omega = omega;
-        tr.precond = rcg.precond = precond;
-        {
-            const double c = precond ? omega / op.diag : omega;
-            rcg.cf[0] = 1.0 - c * (3.0 * op.w[0] + op.sigma);
-            for (int o = 1; o <= R; o++) rcg.cf[o] = -c * op.w[o];
-        }
-        tr.in0 = I.x;
-        tr.bvec = (const Tx *)ins[i].b;
-        tr.ctrl = I.ctrl;
-        rcg.ctrl = I.ctrl;
-        I.nchunks = (int)((op.n + CHUNK - 1) / CHUNK);
-        const int nbd = nblocks_for(op.n);
-        BHC(bsp_alloc(&I.spart, (size_t)std::max({ntr, nrc, nbd}) * 2, owned));
-        BHC(bsp_alloc(&I.gpart, (size_t)I.nchunks * NA, owned));
-        tr.partials = I.spart;
-        I.tr = tr;
-        I.rc = rcg;
-        I.tr_items = ntr;
-        for (int t = 0; t < ntr; t++) wtr.push_back({i, t});
-        for (int t = 0; t < nrc; t++) wrc.push_back({i, t});
-        for (int t = 0; t < I.nchunks; t++) wch.push_back({i, t});
+        dI = ar.take<BInst<Tx, Tg>>(count);
+        dtr = ar.take<WorkItem>(wtr.size());
+        drc = ar.take<WorkItem>(wrc.size());
+        dch = ar.take<WorkItem>(wch.size());
+        if (pass == 0) BHC(ensure(C.batch, ar.used));
     }
-    BHC(bsp_alloc(&dI, count, owned));
-    BHC(bsp_alloc(&dtr, wtr.size(), owned));
-    BHC(bsp_alloc(&drc, wrc.size(), owned));
-    BHC(bsp_alloc(&dch, wch.size(), owned));
     BHC(hipMemcpy(dI, hI.data(), sizeof(BInst<Tx, Tg>) * count, hipMemcpyHostToDevice));
     BHC(hipMemcpy(dtr, wtr.data(), sizeof(WorkItem) * wtr.size(), hipMemcpyHostToDevice));
     BHC(hipMemcpy(drc, wrc.data(), sizeof(WorkItem) * wrc.size(), hipMemcpyHostToDevice));
@@ -469,6 +485,12 @@ int batch_solve(const aar_hip_instance *ins, int count, double omega, double bet
                 hipLaunchKernelGGL((banchor_kernel<Tx, Tg>), dim3((unsigned)wch.size()), dim3(BLOCK), 0, st, dI, dch,
                                    clock, jrel, 2, sh);
         };
+        auto true_res = [&](int jrel, int check) {
+            hipLaunchKernelGGL((bstencil_kernel<Tx, Tx, Tg, SMode::AAR_TRUE>), dim3((unsigned)wtr.size()),
+                               dim3(64 * BWY), 0, st, dI, dtr, (int)wtr.size(), clock, jrel);
+            hipLaunchKernelGGL((bfinish_kernel<Tx, Tg>), dim3(count), dim3(BLOCK), 0, st, dI, clock, jrel, check,
+                               max_iter, ndone);
+        };
         auto anderson = [&](int jrel) {
             auto gram = [&](auto mm) {
                 constexpr int M = decltype(mm)::value;
@@ -482,14 +504,11 @@ int batch_solve(const aar_hip_instance *ins, int count, double omega, double bet
             else gram(std::integral_constant<int, MAXM_BATCH>());
             hipLaunchKernelGGL((banchor_kernel<Tx, Tg>), dim3((unsigned)wch.size()), dim3(BLOCK), 0, st, dI, dch, clock,
                                jrel, 0, sh);
-            hipLaunchKernelGGL((bstencil_kernel<Tx, Tx, Tg, SMode::AAR_TRUE>), dim3((unsigned)wtr.size()),
-                               dim3(64 * BWY), 0, st, dI, dtr, (int)wtr.size(), clock, jrel);
-            hipLaunchKernelGGL((bfinish_kernel<Tx, Tg>), dim3(count), dim3(BLOCK), 0, st, dI, clock, jrel, max_iter,
-                               ndone);
+            true_res(jrel, 1);
         };
 
-        // prologue, per instance: ||b||, the tolerance rule of AAR.c:76-79
-        // and the true residual of x0 (single-solve kernels)
+        // prologue: ||b|| and the tolerance rule of AAR.c:76-79 per instance
+        // (single-solve kernels), then the true residual of x0
         for (int i = 0; i < count; i++) BHC(launch_zero_ctrl(ctrls + i, st));
         hipLaunchKernelGGL(bset_kernel, dim3(1), dim3(64), 0, st, ndone, 0);
         hipLaunchKernelGGL(bset_kernel, dim3(1), dim3(64), 0, st, clock, 0);
@@ -506,19 +525,10 @@ int batch_solve(const aar_hip_instance *ins, int count, double omega, double bet
             d.fin.fin = FIN_NORM_B;
             d.fin.tol = tol;
             d.fin.check = 1;
-            BHC(run_dot<Tx>(d));
-            SArgs<Tx> a = I.tr;
-            Tg *o = I.G + (size_t)(1 % S) * I.ld;
-            if constexpr (sizeof(Tx) == sizeof(Tg)) a.out0 = (Tx *)o;
-            else a.out32 = (float *)o;
-            a.fin.fin = FIN_AAR_RES;
-            a.fin.it = 1;
-            a.fin.check = 0;
-            a.fin.hist = I.hist;
-            a.fin.hist_cap = I.hist_cap;
-            BHC(launch_stencil<Tx>(SMode::AAR_TRUE, a, Shape{}, st));
-            BHC(launch_finish(a.partials, I.tr_items, 1, a.fin, a.ctrl, st));
+            BHC(launch_dot<Tx>(d, st));
+            BHC(launch_finish(d.partials, d.nblocks, 1, d.fin, d.ctrl, st));
         }
+        true_res(0, 0);                      // the clock is 0: iterate 1
         if (p == 1 && max_iter >= 1) {       // iteration 1 is never an Anderson step (AAR.c:109)
             rec(1);
             hipLaunchKernelGGL(bset_kernel, dim3(1), dim3(64), 0, st, clock, 1);
@@ -583,8 +593,10 @@ done:
     if (exec) (void)hipGraphExecDestroy(exec);
     if (graph) (void)hipGraphDestroy(graph);
     (void)hipStreamSynchronize(st);
-    for (void *q : owned) (void)hipFree(q);
-    if (ndone_h) (void)hipHostFree(ndone_h);
+    if (C.batch.bytes > BATCH_KEEP) {
+        (void)hipFree(C.batch.p);
+        C.batch = DevBuf();
+    }
     if (ev_in) (void)hipEventDestroy(ev_in);
     if (ev_out) (void)hipEventDestroy(ev_out);
     return rc;
