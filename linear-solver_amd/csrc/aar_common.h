@@ -13,6 +13,7 @@ namespace aar {
 
 constexpr int R = 6;                 // stencil radius: FD12 (FDn = 6, MPI_REAL/main.c:35)
 constexpr int TX = 64;               // tile width in x: one wavefront
+constexpr long CHUNK_V = 2048;         // elements of a streaming chunk (aar_device.h)
 constexpr int BLOCK = 256;           // threads per block of the streaming (history/dot) kernels
 constexpr int MAXM = 32;             // largest Anderson history m of the real solvers (m x m LS)
 constexpr int MAXM_MID = 16;         // histories up to this run the single-pass Gram and the middle update forms

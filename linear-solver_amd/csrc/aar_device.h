@@ -44,15 +44,15 @@ __device__ inline void block_reduce_to(const double (&acc)[NACC], double *dst, d
 // memory (a grid stride of one element per thread measured 10-13% slower
 // at 512^3 for the many-stream history sweeps).  The element-to-thread
 // assignment is fixed, so reductions over it keep a fixed order.
-constexpr long CHUNK_V = 2048;
 static_assert(CHUNK_V % BLOCK == 0, "a chunk is a whole number of block steps");
-__device__ __forceinline__ long chunk_first()
+__device__ __forceinline__ long chunk_first(long chunk = CHUNK_V)
 {
-    return (long)blockIdx.x * CHUNK_V + threadIdx.x;
+    return (long)blockIdx.x * chunk + threadIdx.x;
 }
-__device__ __forceinline__ long chunk_next(long i)
+// chunk: a power of two times BLOCK
+__device__ __forceinline__ long chunk_next(long i, long chunk = CHUNK_V)
 {
-    return ((i + BLOCK) % CHUNK_V) >= BLOCK ? i + BLOCK : i + BLOCK + (long)(gridDim.x - 1) * CHUNK_V;
+    return ((i + BLOCK) & (chunk - 1)) >= BLOCK ? i + BLOCK : i + BLOCK + (long)(gridDim.x - 1) * chunk;
 }
 
 // Value-major form of block_reduce_to: thread k < NACC writes the block's

@@ -97,6 +97,7 @@ struct GramArgs {
     int fslot = 0;            // slot of f (kind 0) or of A x (kinds 1/2)
     int nvalid = 0;
     int it = 0;
+    long chunk = CHUNK_V;     // vectors a block walks at a time (m <= 8)
     int nblocks = 0;
     double *partials = nullptr;
     unsigned *counter = nullptr;

@@ -92,7 +92,8 @@ int auto_lz(const Op &op, int wy, int py, size_t es);
 long ring_ld(long n, size_t es);
 int nblocks_for(long n);
 // grid of the register Gram (m <= 8) on n points
-int gram_blocks(long n, int m);
+template <typename T>
+int gram_blocks(long n, int m, long *chunk);
 template <typename T>
 SArgs<T> base_sargs(const Op &op);
 template <typename T>

@@ -133,7 +133,7 @@ __global__ __launch_bounds__(BLOCK) void gram_kernel(const GramArgs<T> a)
     const bool vec_ok = (n % VW) == 0 && (KIND == 0 || ((uintptr_t)a.b % 16) == 0);
     if (vec_ok) {
         const long nq = n / VW;
-        for (long iq = chunk_first(); iq < nq; iq = chunk_next(iq)) {
+        for (long iq = chunk_first(a.chunk); iq < nq; iq = chunk_next(iq, a.chunk)) {
             const long i = VW * iq;
             VT vd[NS], vx[NS];
 #pragma unroll

@@ -1,0 +1,39 @@
+"""The Gram's grid where its chunks change: a vector a thread, 2 to 8, odd point
+counts, fewer points than a block; real (FP64, mixed) and complex."""
+import numpy as np
+import pytest
+import torch
+
+from aar_hip import problems as P
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("shape", [(8, 8, 7), (8, 8, 8), (8, 8, 9), (15, 13, 13), (48, 48, 48), (64, 64, 64),
+                                   (64, 64, 65), (128, 64, 65), (101, 99, 95), (128, 128, 129)])
+@pytest.mark.parametrize("solver", ["aar", "mixed", "pgr", "helm"])
+def test_gram_grid(gpu, oracle, solver, shape):
+    if solver == "helm" and min(shape) < 12:
+        pytest.skip("complex grids have sides of 12 and more")
+    print("gram grid", solver, shape, flush=True)
+    a, n, its = P.poisson_a(0.5), int(np.prod(shape)), 13
+    if solver == "helm":
+        b, c = P.rhs_complex_normal(shape, 3), P.helmholtz_coefficient(shape, 7)
+        xd = torch.zeros(n, dtype=torch.complex128, device="cuda")
+        gpu.helm_aar(xd, torch.from_numpy(b).cuda(), shape, a, torch.from_numpy(c).cuda(), 0.3, 0.5, 0.6, 0.6, 7, 6,
+                     its, 1e-30)
+        xo, _ = oracle.aar_complex(np.zeros_like(b), b, shape, a, c, 0.3, 0.5, 0.6, 0.6, 7, 6, its, 1e-30)
+    else:
+        b = np.random.default_rng(9).standard_normal(n)
+        xd, bd = torch.zeros(n, dtype=torch.float64, device="cuda"), torch.from_numpy(b).cuda()
+        if solver == "pgr":
+            gpu.PGR(xd, bd, shape, a, 0.6, 7, 6, its, 1e-30, sigma=0.5)
+            xo, _ = oracle.pgr(np.zeros(n), b, shape, a, 0.6, 7, 6, its, 1e-30, sigma=0.5)
+        else:
+            (gpu.AAR_mixed if solver == "mixed" else gpu.AAR)(xd, bd, shape, a, 0.6, 0.6, 7, 6, its, 1e-30, sigma=0.5)
+            xo, _ = oracle.aar(np.zeros(n), b, shape, a, 0.6, 0.6, 7, 6, its, 1e-30, sigma=0.5)
+    # two least-squares steps: a lost or doubled chunk moves the coefficients by
+    # its share of the points (above 1e-3); rounding moves them by the seven
+    # columns' conditioning, FP32 history by that of its own rounding
+    tol = 1e-3 if solver == "mixed" else 1e-6
+    assert np.linalg.norm(xd.cpu().numpy() - xo) <= tol * np.linalg.norm(xo)
