@@ -328,8 +328,10 @@ int aar_hip_set_tuning(int lz, int wy, int py);
  * nz grid (fp32 = 1: the FP32 sweep of the mixed solver) over the launch
  * shapes (wy, py) and z-slab depths lz and keeps the fastest for that grid;
  * later solves on the grid use it.  batch_shape = 1 tunes only lz for the
- * batched launch (aar_hip_aar_batch).  Returns the shape and its time per
- * sweep in us.  Allocates two temporary vectors of the grid. */
+ * batched launch (aar_hip_aar_batch).  Up to 8.5 million points the one-shot
+ * boxes are timed too and used when they are faster; the shape returned stays
+ * the best z-march.  Returns the shape and its time per sweep in us.
+ * Allocates two temporary vectors of the grid. */
 int aar_hip_autotune(int nx, int ny, int nz, int fp32, int batch_shape, int *lz, int *wy, int *py, double *us);
 
 /* Tuning options of the history sweeps (apply to subsequent solves):
@@ -337,8 +339,9 @@ int aar_hip_autotune(int nx, int ny, int nz, int fp32, int batch_shape, int *lz,
  *                 512), so that slots whose size is a large power of two
  *                 do not alias onto the same HBM channels;
  *   "hist_blocks" grid of the reducing sweeps (0 = automatic, <= 2048);
- *   "two_pass"    1 (default): reductions finish in a one-block second
- *                 kernel; 0: in the last block of the reducing kernel;
+ *   "two_pass"    1 (default): the history reductions finish in a one-block
+ *                 second kernel; 0: in the last block of the reducing
+ *                 kernel (the stencil sweeps' sums always in a second);
  *   "autotune"    1: a grid's stencil shape is tuned on its first solve
  *                 (aar_hip_autotune); 0 (default): automatic shapes;
  *   "complex_pinv_reference_order"  1: the complex solver's m x m SVD runs
