@@ -49,6 +49,8 @@ struct Shape {
     double us = 0.0;          // measured time of one recurrence sweep (tuned shapes)
 };
 
+// (a plane beyond the sweeps' 32-bit offsets always marches 64 x WIDE_ROWS columns)
+constexpr int WIDE_ROWS = 32;
 template <typename T>
 hipError_t launch_stencil(SMode m, const SArgs<T> &a, const Shape &sh, hipStream_t st);
 // blocks (= partials per sum) of the sweep

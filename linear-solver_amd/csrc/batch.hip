@@ -31,6 +31,7 @@ namespace aar {
 namespace {
 
 constexpr int BWY = 8, BPY = 4;        // launch shape of the batched stencils (64 x 32 columns)
+static_assert(BWY * BPY == WIDE_ROWS, "wide planes keep the batch's columns");
 constexpr int CHUNK = 4096;            // elements per block of the streaming kernels
 
 template <typename Tx, typename Tg>
@@ -65,7 +66,7 @@ struct BShared {               // batch-wide values
 // stencils: REC (g_{it+1} from g_it) and TRUE (g_{it+1} from x, after the
 // Anderson step at it), it = *clock + jrel
 // -------------------------------------------------------------------------
-template <typename T, typename Tx, typename Tg, SMode MODE>
+template <typename T, typename Tx, typename Tg, SMode MODE, bool WIDE>
 __global__ __launch_bounds__(64 * BWY) void bstencil_kernel(const BInst<Tx, Tg> *inst, const WorkItem *work,
                                                             int nwork, const int *clock, int jrel)
 {
@@ -91,7 +92,7 @@ __global__ __launch_bounds__(64 * BWY) void bstencil_kernel(const BInst<Tx, Tg> 
         }
     }
     __syncthreads();
-    stencil_body<T, BWY, BPY / Lane<T>::RPW, MODE>(sa, wi.idx);
+    stencil_body<T, BWY, BPY / Lane<T>::RPW, MODE, false, WIDE>(sa, wi.idx);
 }
 
 // per-instance finish of the true residual: relres check (or, at the start, the
@@ -476,9 +477,21 @@ int batch_solve(const aar_hip_instance *ins, int count, double omega, double bet
         const BInst<float, Tg> *IF = nullptr;
         if constexpr (sizeof(Tx) == 8) ID = (const BInst<double, Tg> *)dI;
         else IF = (const BInst<float, Tg> *)dI;
+        // one system with a plane beyond 32-bit offsets takes the whole batch
+        // to the sweeps with 64-bit ones
+        bool wide_tr = false, wide_rc = false;
+        for (const Op &o : ops) {
+            wide_tr |= wide_plane<Tx>(o.nx, o.ny);
+            wide_rc |= wide_plane<Tg>(o.nx, o.ny);
+        }
         auto rec = [&](int jrel) {
-            hipLaunchKernelGGL((bstencil_kernel<Tg, Tx, Tg, SMode::AAR_REC>), dim3((unsigned)wrc.size()),
-                               dim3(64 * BWY), 0, st, dI, drc, (int)wrc.size(), clock, jrel);
+            auto go = [&](auto w) {
+                hipLaunchKernelGGL((bstencil_kernel<Tg, Tx, Tg, SMode::AAR_REC, decltype(w)::value>),
+                                   dim3((unsigned)wrc.size()), dim3(64 * BWY), 0, st, dI, drc, (int)wrc.size(), clock,
+                                   jrel);
+            };
+            if (wide_rc) go(std::true_type{});
+            else go(std::false_type{});
             // p > m+1: the residual of iteration base + jrel is read by no
             // Anderson window (AAR.c:97-102 keeps the last m columns)
             if (p > m + 1 && jrel < p - m)
@@ -486,8 +499,13 @@ int batch_solve(const aar_hip_instance *ins, int count, double omega, double bet
                                    clock, jrel, 2, sh);
         };
         auto true_res = [&](int jrel, int check) {
-            hipLaunchKernelGGL((bstencil_kernel<Tx, Tx, Tg, SMode::AAR_TRUE>), dim3((unsigned)wtr.size()),
-                               dim3(64 * BWY), 0, st, dI, dtr, (int)wtr.size(), clock, jrel);
+            auto go = [&](auto w) {
+                hipLaunchKernelGGL((bstencil_kernel<Tx, Tx, Tg, SMode::AAR_TRUE, decltype(w)::value>),
+                                   dim3((unsigned)wtr.size()), dim3(64 * BWY), 0, st, dI, dtr, (int)wtr.size(), clock,
+                                   jrel);
+            };
+            if (wide_tr) go(std::true_type{});
+            else go(std::false_type{});
             hipLaunchKernelGGL((bfinish_kernel<Tx, Tg>), dim3(count), dim3(BLOCK), 0, st, dI, clock, jrel, check,
                                max_iter, ndone);
         };

@@ -71,7 +71,8 @@ int stencil_tile_planes(int nx, int ny, int nz)
 template <typename T>
 void stencil_geometry(SArgs<T> &a, const Shape &sh)
 {
-    const int tx = sh.tile ? tile_x<T>(sh.tile) : TX, ty = sh.tile ? tile_rows<T>(sh.tile) : sh.wy * sh.py;
+    const int tx = sh.tile ? tile_x<T>(sh.tile) : TX;
+    const int ty = wide_plane<T>(a.nx, a.ny) ? WIDE_ROWS : (sh.tile ? tile_rows<T>(sh.tile) : sh.wy * sh.py);
     a.nxy = a.nx * a.ny;
     a.ntx = (a.nx + tx - 1) / tx;
     a.nty = (a.ny + ty - 1) / ty;

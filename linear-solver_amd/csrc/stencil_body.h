@@ -34,14 +34,14 @@ template <typename T, int WY, int PY> struct March {
 // below and the batched kernel of batch.hip.  WY wavefronts, PY rows per
 // thread.  VC: the variable-coefficient operator a*Lap + c(x), with a
 // pointwise field a.vf read in the epilogue.
-template <typename T, int WY, int PY, SMode MODE, bool VC, bool EDGE>
+template <typename T, int WY, int PY, SMode MODE, bool VC, int XM>
 __device__ __forceinline__ void stencil_march(const SArgs<T> &a, const int item, typename March<T, WY, PY>::Lds &S)
 {
     static_assert(!VC || MODE != SMode::RESID, "no variable-coefficient RESID sweep");
     using M = March<T, WY, PY>;
     using L = Lane<T>;
     using Vec = typename L::Vec;
-    using Off = VOff<T, EDGE>;
+    using Off = VOff<T, XM>;
     constexpr int V = L::V, LPR = L::LPR, HXV = L::HXV;
     constexpr int NT = M::NT, TY = M::TY, NHC = M::NHC, NH = M::NH, HR = M::HR;
     constexpr int NE = ModeInfo<MODE>::NE;
@@ -117,11 +117,11 @@ __device__ __forceinline__ void stencil_march(const SArgs<T> &a, const int item,
             const size_t zo = (size_t)z * nxy;
             z = z + 1 == nz ? 0 : z + 1;
 #pragma unroll
-            for (int p = 0; p < PY; p++) q[p][s] = ld_vec<T, EDGE>(a.in0 + zo, c_off[p]);
+            for (int p = 0; p < PY; p++) q[p][s] = ld_vec<T, XM>(a.in0 + zo, c_off[p]);
             if (s >= R) {
 #pragma unroll
                 for (int j = 0; j < NH; j++) {
-                    const Vec f = ld_vec<T, EDGE>(a.in0 + zo, h_off[j]);
+                    const Vec f = ld_vec<T, XM>(a.in0 + zo, h_off[j]);
                     if (h_ok[j]) S.ring[s - R][tid + NT * j] = f;
                 }
             }
@@ -136,16 +136,16 @@ __device__ __forceinline__ void stencil_march(const SArgs<T> &a, const int item,
         zq = zq + 1 == nz ? 0 : zq + 1;
         zc = zc + 1 == nz ? 0 : zc + 1;
 #pragma unroll
-        for (int p = 0; p < PY; p++) st.qn[p] = ld_vec<T, EDGE>(a.in0 + oq, c_off[p]);
+        for (int p = 0; p < PY; p++) st.qn[p] = ld_vec<T, XM>(a.in0 + oq, c_off[p]);
 #pragma unroll
-        for (int j = 0; j < NH; j++) st.h[j] = ld_vec<T, EDGE>(a.in0 + oq, h_off[j]);
+        for (int j = 0; j < NH; j++) st.h[j] = ld_vec<T, XM>(a.in0 + oq, h_off[j]);
         if constexpr (NE > 0) {
 #pragma unroll
-            for (int p = 0; p < PY; p++) st.en[p] = ld_vec<T, EDGE>(a.bvec + oc, c_off[p]);
+            for (int p = 0; p < PY; p++) st.en[p] = ld_vec<T, XM>(a.bvec + oc, c_off[p]);
         }
         if constexpr (VC) {
 #pragma unroll
-            for (int p = 0; p < PY; p++) st.vv[p] = ld_vec<T, EDGE>(a.vf + oc, c_off[p]);
+            for (int p = 0; p < PY; p++) st.vv[p] = ld_vec<T, XM>(a.vf + oc, c_off[p]);
         }
     };
 
@@ -202,9 +202,9 @@ __device__ __forceinline__ void stencil_march(const SArgs<T> &a, const int item,
             // outputs are next read a whole sweep later (beyond the caches
             // at the sizes where the march runs): non-temporal stores
             auto put = [&](auto *base, const auto &o) {
-                st_vec<std::remove_pointer_t<decltype(base)>, true, T, EDGE>(base + zoff, c_off[p], o, c_ok[p], false);
+                st_vec<std::remove_pointer_t<decltype(base)>, true, T, XM>(base + zoff, c_off[p], o, c_ok[p], false);
             };
-            stencil_epilogue<T, MODE, VC, EDGE>(a, k, y, u, cur.en[p], cur.vv[p], c_ok[p], put, acc);
+            stencil_epilogue<T, MODE, VC, XM>(a, k, y, u, cur.en[p], cur.vv[p], c_ok[p], put, acc);
         }
         // shift the queue one plane
 #pragma unroll
@@ -228,19 +228,20 @@ __device__ __forceinline__ void stencil_march(const SArgs<T> &a, const int item,
     if (a.partials) block_reduce_to<NACC, NT>(acc, a.partials + (size_t)item * NACC, S.red);
 }
 
-template <typename T, int WY, int PY, SMode MODE, bool VC = false>
+template <typename T, int WY, int PY, SMode MODE, bool VC = false, bool WIDE = false>
 __device__ __forceinline__ void stencil_body(const SArgs<T> &a, const int item)
 {
     __shared__ typename March<T, WY, PY>::Lds S;
-    if (edge_tile(a, item)) stencil_march<T, WY, PY, MODE, VC, true>(a, item, S);
-    else stencil_march<T, WY, PY, MODE, VC, false>(a, item, S);
+    if constexpr (WIDE) stencil_march<T, WY, PY, MODE, VC, XWIDE>(a, item, S);
+    else if (edge_tile(a, item)) stencil_march<T, WY, PY, MODE, VC, XPOINT>(a, item, S);
+    else stencil_march<T, WY, PY, MODE, VC, XVEC>(a, item, S);
 }
 
-template <typename T, int WY, int PY, SMode MODE, bool VC = false>
+template <typename T, int WY, int PY, SMode MODE, bool VC = false, bool WIDE = false>
 __global__ __launch_bounds__(64 * WY) void stencil_kernel(const SArgs<T> a)
 {
     if (a.ctrl && a.ctrl->done) return;
-    stencil_body<T, WY, PY, MODE, VC>(a, xcd_item(blockIdx.x, a.nitems));
+    stencil_body<T, WY, PY, MODE, VC, WIDE>(a, xcd_item(blockIdx.x, a.nitems));
 }
 
 }  // namespace aar

@@ -9,14 +9,14 @@ namespace aar {
 // A column of 64 x (wy*py) points.  A wavefront covers RPW rows of the tile
 // (2 in FP64, 4 in FP32), so wy*py rows are wy wavefronts with wy*py/(RPW wy)
 // rows per thread, or fewer wavefronts where that is below one row.
-template <typename T, SMode M, bool VC, int WY, int ROWS>
+template <typename T, SMode M, bool VC, int WY, int ROWS, bool WIDE = false>
 hipError_t launch_march(const SArgs<T> &a, hipStream_t st)
 {
     constexpr int RPW = Lane<T>::RPW;
     constexpr int W = WY * RPW <= ROWS ? WY : ROWS / RPW;
     constexpr int PY = ROWS / (W * RPW);
     static_assert(W * RPW * PY == ROWS, "whole rows");
-    hipLaunchKernelGGL((stencil_kernel<T, W, PY, M, VC>), dim3(a.nitems), dim3(64 * W), 0, st, a);
+    hipLaunchKernelGGL((stencil_kernel<T, W, PY, M, VC, WIDE>), dim3(a.nitems), dim3(64 * W), 0, st, a);
     return hipGetLastError();
 }
 
@@ -24,6 +24,7 @@ template <typename T, SMode M, bool VC>
 hipError_t launch_sweep(SArgs<T> a, const Shape &sh, hipStream_t st)
 {
     stencil_geometry(a, sh);
+    if (wide_plane<T>(a.nx, a.ny)) return launch_march<T, M, VC, 8, WIDE_ROWS, true>(a, st);
     if (sh.tile) {
         const dim3 grid(a.nitems), block(256);
         switch (sh.tile) {

@@ -62,25 +62,40 @@ template <typename T> struct Lane {
 // 16 (32 x 32: 200 x 161 x 150 32.1 -> 32.9 us, 96^3 14.4 -> 13.7).
 template <typename T> __host__ __device__ constexpr int tile_x(int lz) { return sizeof(T) == 8 && lz > 1 ? 32 : 64; }
 
-// base[off] with a uniform (per-plane) base pointer and a 32-bit in-plane
-// offset: the access compiles to the scalar-base + vector-offset form, with
-// no per-access 64-bit address arithmetic (in-plane byte offsets are below
-// 2^32 for any plane the host accepts)
-template <typename T> __device__ __forceinline__ T ld_at(const T *base, unsigned eoff)
+// How a tile takes its vectors of V points along x.
+// * XVEC: the V points are consecutive in memory: one access, one offset.
+// * XPOINT (a tile whose window reaches past nx when nx is not a multiple of
+//   V): point by point, a wrapped offset each.
+// * XWIDE: the same with 64-bit byte offsets, for the planes of wide_plane().
+enum : int { XVEC = 0, XPOINT = 1, XWIDE = 2 };
+
+// Byte offsets in a plane are 32 bits wide.  A plane of more than 2^32 bytes
+// (2^29 points FP64, 2^30 FP32) takes the XWIDE sweep.
+template <typename T> __host__ __device__ inline bool wide_plane(int nx, int ny)
 {
-    return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + (size_t)(eoff * (unsigned)sizeof(T)));
-}
-template <typename T> __device__ __forceinline__ void st_at(T *base, unsigned eoff, T v)
-{
-    *reinterpret_cast<T *>(reinterpret_cast<char *>(base) + (size_t)(eoff * (unsigned)sizeof(T))) = v;
+    return (unsigned long long)nx * (unsigned long long)ny * sizeof(T) > 1ull << 32;
 }
 
-// In-plane element offsets of one vector of points.  EDGE false: the V
-// points are consecutive in memory (NO = 1 offset).  EDGE true (a tile whose
-// window reaches past nx when nx is not a multiple of V): one wrapped offset
-// each.
-template <typename T, bool EDGE> struct VOff {
-    static constexpr int NO = EDGE ? Lane<T>::V : 1;
+// base[off] with a uniform (per-plane) base pointer and a 32-bit in-plane
+// offset: the access compiles to the scalar-base + vector-offset form, with
+// no per-access 64-bit address arithmetic
+template <typename T, bool WIDE> __device__ __forceinline__ size_t byte_off(unsigned eoff)
+{
+    if constexpr (WIDE) return (size_t)eoff * sizeof(T);
+    else return (size_t)(eoff * (unsigned)sizeof(T));
+}
+template <bool WIDE, typename T> __device__ __forceinline__ T ld_at(const T *base, unsigned eoff)
+{
+    return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + byte_off<T, WIDE>(eoff));
+}
+template <bool WIDE, typename T> __device__ __forceinline__ void st_at(T *base, unsigned eoff, T v)
+{
+    *reinterpret_cast<T *>(reinterpret_cast<char *>(base) + byte_off<T, WIDE>(eoff)) = v;
+}
+
+// in-plane element offsets of one vector of points
+template <typename T, int XM> struct VOff {
+    static constexpr int NO = XM == XVEC ? 1 : Lane<T>::V;
     unsigned o[NO];
     __device__ __forceinline__ void set(int gx, int gy, int nx, int ny)
     {
@@ -90,17 +105,17 @@ template <typename T, bool EDGE> struct VOff {
     }
 };
 
-template <typename T, bool EDGE>
-__device__ __forceinline__ typename Lane<T>::Vec ld_vec(const T *base, const VOff<T, EDGE> &f)
+template <typename T, int XM>
+__device__ __forceinline__ typename Lane<T>::Vec ld_vec(const T *base, const VOff<T, XM> &f)
 {
     using L = Lane<T>;
     typename L::Vec r;
-    if constexpr (!EDGE) {
+    if constexpr (XM == XVEC) {
         r = *reinterpret_cast<const typename L::VecU *>(reinterpret_cast<const char *>(base) +
                                                         (size_t)(f.o[0] * (unsigned)sizeof(T)));
     } else {
 #pragma unroll
-        for (int v = 0; v < L::V; v++) r[v] = ld_at(base, f.o[v]);
+        for (int v = 0; v < L::V; v++) r[v] = ld_at<XM == XWIDE>(base, f.o[v]);
     }
     return r;
 }
@@ -114,12 +129,12 @@ template <typename T, int W = TX> __device__ __forceinline__ bool edge_tile(cons
 }
 
 // S: the stored type (T, or float for the FP32 copy of an FP64 sweep).
-// NT: non-temporal.  ok: masks of the V points (EDGE) or of the vector (ok[0]).
-template <typename S, bool NT, typename T, bool EDGE, int NV>
-__device__ __forceinline__ void st_vec(S *base, const VOff<T, EDGE> &f, const S (&v)[NV], const bool (&ok)[NV],
+// NT: non-temporal.  ok: masks of the V points, or of the vector (XVEC: ok[0]).
+template <typename S, bool NT, typename T, int XM, int NV>
+__device__ __forceinline__ void st_vec(S *base, const VOff<T, XM> &f, const S (&v)[NV], const bool (&ok)[NV],
                                        bool masked)
 {
-    if constexpr (!EDGE) {
+    if constexpr (XM == XVEC) {
         typedef S SV __attribute__((ext_vector_type(NV), aligned(sizeof(S))));
         SV r;
 #pragma unroll
@@ -132,7 +147,7 @@ __device__ __forceinline__ void st_vec(S *base, const VOff<T, EDGE> &f, const S 
     } else {
 #pragma unroll
         for (int i = 0; i < NV; i++)
-            if (!masked || ok[i]) st_at(base, f.o[i], v[i]);
+            if (!masked || ok[i]) st_at<XM == XWIDE>(base, f.o[i], v[i]);
     }
 }
 
@@ -264,7 +279,7 @@ __device__ __forceinline__ typename Lane<T>::Vec stencil_value(const SArgs<T> &a
 // so it may store the same bits to the same address: put may store
 // unconditionally (no branch per point) or masked.  Norm terms are always
 // masked, per point in an edge tile, else per vector.
-template <typename T, SMode MODE, bool VC, bool EDGE, int NACC, typename Put>
+template <typename T, SMode MODE, bool VC, int XM, int NACC, typename Put>
 __device__ __forceinline__ void stencil_epilogue(const SArgs<T> &a, const PointK<T> &k,
                                                  const typename Lane<T>::Vec y, const typename Lane<T>::Vec u,
                                                  const typename Lane<T>::Vec en, const typename Lane<T>::Vec vv,
@@ -278,7 +293,7 @@ __device__ __forceinline__ void stencil_epilogue(const SArgs<T> &a, const PointK
 #pragma unroll
     for (int j = 0; j < NACC; j++) t[j] = 0.0;
     auto m = [&](int v, double x) -> double {
-        if constexpr (EDGE) return ok[v] ? x : 0.0;
+        if constexpr (XM != XVEC) return ok[v] ? x : 0.0;
         else return x;
     };
     if constexpr (MODE == SMode::MATVEC) {
@@ -379,7 +394,7 @@ __device__ __forceinline__ void stencil_epilogue(const SArgs<T> &a, const PointK
         if (a.out1) put(a.out1, o1);
     }
 #pragma unroll
-    for (int j = 0; j < NACC; j++) acc[j] += EDGE || ok[0] ? t[j] : 0.0;
+    for (int j = 0; j < NACC; j++) acc[j] += XM != XVEC || ok[0] ? t[j] : 0.0;
 }
 
 }  // namespace aar

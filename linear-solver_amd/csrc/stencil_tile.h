@@ -32,13 +32,13 @@ template <typename T, int WY, int PY, int LZ> struct Tile {
     };
 };
 
-template <typename T, int WY, int PY, int LZ, SMode MODE, bool VC, bool EDGE>
+template <typename T, int WY, int PY, int LZ, SMode MODE, bool VC, int XM>
 __device__ __forceinline__ void stencil_box(const SArgs<T> &a, const int item, typename Tile<T, WY, PY, LZ>::Lds &S)
 {
     using B = Tile<T, WY, PY, LZ>;
     using L = Lane<T>;
     using Vec = typename L::Vec;
-    using Off = VOff<T, EDGE>;
+    using Off = VOff<T, XM>;
     constexpr int V = L::V, LPR = B::LPR, HXV = L::HXV, BX = B::BX;
     constexpr int NT = B::NT, TY = B::TY, NHC = B::NHC, NH = B::NH;
     constexpr int NE = ModeInfo<MODE>::NE;
@@ -79,7 +79,7 @@ __device__ __forceinline__ void stencil_box(const SArgs<T> &a, const int item, t
 #pragma unroll
     for (int s = 0; s < NQ; s++)
 #pragma unroll
-        for (int p = 0; p < PY; p++) q[p][s] = ld_vec<T, EDGE>(a.in0 + zo[s], c_off[p]);
+        for (int p = 0; p < PY; p++) q[p][s] = ld_vec<T, XM>(a.in0 + zo[s], c_off[p]);
     // halo vector c of the box: plane, then 2R rows of LPR and TY rows of
     // HXV left and HXV right
     Vec h[NH];
@@ -105,20 +105,20 @@ __device__ __forceinline__ void stencil_box(const SArgs<T> &a, const int item, t
         const unsigned zs = (unsigned)modp(z0 + s, nz) * (unsigned)nxy;
 #pragma unroll
         for (int v = 0; v < Off::NO; v++) off.o[v] += zs;
-        h[j] = ld_vec<T, EDGE>(a.in0, off);
+        h[j] = ld_vec<T, XM>(a.in0, off);
     }
     Vec en[PY][LZ], vv[PY][LZ];
     if constexpr (NE > 0) {
 #pragma unroll
         for (int s = 0; s < LZ; s++)
 #pragma unroll
-            for (int p = 0; p < PY; p++) en[p][s] = ld_vec<T, EDGE>(a.bvec + zo[R + s], c_off[p]);
+            for (int p = 0; p < PY; p++) en[p][s] = ld_vec<T, XM>(a.bvec + zo[R + s], c_off[p]);
     }
     if constexpr (VC) {
 #pragma unroll
         for (int s = 0; s < LZ; s++)
 #pragma unroll
-            for (int p = 0; p < PY; p++) vv[p][s] = ld_vec<T, EDGE>(a.vf + zo[R + s], c_off[p]);
+            for (int p = 0; p < PY; p++) vv[p][s] = ld_vec<T, XM>(a.vf + zo[R + s], c_off[p]);
     }
 
 #pragma unroll
@@ -160,10 +160,10 @@ __device__ __forceinline__ void stencil_box(const SArgs<T> &a, const int item, t
                 // is the next sweep's input, and they lose 0.3%)
                 constexpr bool NT_OUT = MODE == SMode::PGR_STEP;
                 auto put = [&](auto *base, const auto &o) {
-                    st_vec<std::remove_pointer_t<decltype(base)>, NT_OUT, T, EDGE>(base + zo[R + s], c_off[p], o,
+                    st_vec<std::remove_pointer_t<decltype(base)>, NT_OUT, T, XM>(base + zo[R + s], c_off[p], o,
                                                                                   c_ok[p], true);
                 };
-                stencil_epilogue<T, MODE, VC, EDGE>(a, k, y, u, en[p][s], vv[p][s], c_ok[p], put, acc);
+                stencil_epilogue<T, MODE, VC, XM>(a, k, y, u, en[p][s], vv[p][s], c_ok[p], put, acc);
             }
         }
     }
@@ -174,8 +174,8 @@ template <typename T, int WY, int PY, int LZ, SMode MODE, bool VC = false>
 __device__ __forceinline__ void stencil_tile_body(const SArgs<T> &a, const int item)
 {
     __shared__ typename Tile<T, WY, PY, LZ>::Lds S;
-    if (edge_tile<T, tile_x<T>(LZ)>(a, item)) stencil_box<T, WY, PY, LZ, MODE, VC, true>(a, item, S);
-    else stencil_box<T, WY, PY, LZ, MODE, VC, false>(a, item, S);
+    if (edge_tile<T, tile_x<T>(LZ)>(a, item)) stencil_box<T, WY, PY, LZ, MODE, VC, XPOINT>(a, item, S);
+    else stencil_box<T, WY, PY, LZ, MODE, VC, XVEC>(a, item, S);
 }
 
 template <typename T, int WY, int PY, int LZ, SMode MODE, bool VC = false>
