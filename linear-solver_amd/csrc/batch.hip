@@ -46,6 +46,7 @@ struct BInst {
     Ctrl *ctrl = nullptr;
     double *hist = nullptr;
     int hist_cap = 0;
+    int *counted = nullptr;    // 1: ndone holds this system
     double *spart = nullptr;   // stencil partials
     double *gpart = nullptr;   // Gram partials [NA][nchunks]
     int nchunks = 0;
@@ -96,7 +97,9 @@ __global__ __launch_bounds__(64 * BWY) void bstencil_kernel(const BInst<Tx, Tg> 
 }
 
 // per-instance finish of the true residual: relres check (or, at the start, the
-// record alone) at the Anderson iteration it = *clock + jrel (FIN_AAR_RES of iterate it+1)
+// record alone) at the Anderson iteration it = *clock + jrel (FIN_AAR_RES of iterate it+1).
+// Counts a stopped system into ndone, once and whatever stopped it: this check,
+// the start's tolerance rule or a least-squares solve that did not converge.
 template <typename Tx, typename Tg>
 __global__ __launch_bounds__(BLOCK) void bfinish_kernel(const BInst<Tx, Tg> *inst, const int *clock, int jrel,
                                                         int check, int max_iter, int *ndone)
@@ -104,18 +107,23 @@ __global__ __launch_bounds__(BLOCK) void bfinish_kernel(const BInst<Tx, Tg> *ins
     __shared__ double scratch[BLOCK / 64];
     __shared__ double out[1];
     const BInst<Tx, Tg> &I = inst[blockIdx.x];
-    if (I.ctrl->done) return;
-    final_sum(I.spart, I.tr_items, 1, out, scratch);
+    const bool running = !I.ctrl->done;
+    if (running) final_sum(I.spart, I.tr_items, 1, out, scratch);
     if (threadIdx.x == 0) {
-        FinArgs f = {};
-        f.fin = FIN_AAR_RES;
-        f.it = *clock + jrel + 1;
-        f.check = check;
-        f.max_iter = max_iter;
-        f.hist = I.hist;
-        f.hist_cap = I.hist_cap;
-        finalize(f, I.ctrl, out, 1);
-        if (I.ctrl->done) atomicAdd(ndone, 1);
+        if (running) {
+            FinArgs f = {};
+            f.fin = FIN_AAR_RES;
+            f.it = *clock + jrel + 1;
+            f.check = check;
+            f.max_iter = max_iter;
+            f.hist = I.hist;
+            f.hist_cap = I.hist_cap;
+            finalize(f, I.ctrl, out, 1);
+        }
+        if (I.ctrl->done && !*I.counted) {
+            *I.counted = 1;
+            atomicAdd(ndone, 1);
+        }
     }
 }
 
@@ -320,7 +328,7 @@ __global__ __launch_bounds__(BLOCK) void banchor_kernel(const BInst<Tx, Tg> *ins
 }
 
 __global__ void bclock_kernel(int *clock, int p) { if (threadIdx.x == 0 && blockIdx.x == 0) *clock += p; }
-__global__ void bset_kernel(int *v, int value) { if (threadIdx.x == 0 && blockIdx.x == 0) *v = value; }
+__global__ void bset_kernel(int *v, int value, int n) { for (int i = threadIdx.x; i < n; i += blockDim.x) v[i] = value; }
 
 // A batch's buffers are cut from one allocation, laid out twice: first from
 // address zero for its size, then in place.
@@ -396,8 +404,8 @@ int batch_solve(const aar_hip_instance *ins, int count, double omega, double bet
         Arena ar;
         if (pass == 1) ar.base = (char *)C.batch.p;
         ctrls = ar.take<Ctrl>(count);
-        clock = ar.take<int>(1);
-        ndone = ar.take<int>(1);
+        clock = ar.take<int>(2 + count);     // the clock, ndone and the systems' counted flags
+        ndone = clock + 1;
         wtr.clear();
         wrc.clear();
         wch.clear();
@@ -416,6 +424,7 @@ int batch_solve(const aar_hip_instance *ins, int count, double omega, double bet
             I.NC = NC;
             I.x = (Tx *)ins[i].x;
             I.ctrl = ctrls + i;
+            I.counted = ndone + 1 + i;
             I.hist_cap = max_iter + 4;
             I.G = ar.take<Tg>((size_t)I.ld * S);
             if (NC > 0) I.C = ar.take<Tg>((size_t)I.ld * NC);
@@ -528,8 +537,7 @@ int batch_solve(const aar_hip_instance *ins, int count, double omega, double bet
         // prologue: ||b|| and the tolerance rule of AAR.c:76-79 per instance
         // (single-solve kernels), then the true residual of x0
         for (int i = 0; i < count; i++) BHC(launch_zero_ctrl(ctrls + i, st));
-        hipLaunchKernelGGL(bset_kernel, dim3(1), dim3(64), 0, st, ndone, 0);
-        hipLaunchKernelGGL(bset_kernel, dim3(1), dim3(64), 0, st, clock, 0);
+        hipLaunchKernelGGL(bset_kernel, dim3(1), dim3(64), 0, st, clock, 0, 2 + count);
         BHC(hipEventRecord(C.t0, st));
         for (int i = 0; i < count; i++) {
             const BInst<Tx, Tg> &I = hI[i];
@@ -549,7 +557,7 @@ int batch_solve(const aar_hip_instance *ins, int count, double omega, double bet
         true_res(0, 0);                      // the clock is 0: iterate 1
         if (p == 1 && max_iter >= 1) {       // iteration 1 is never an Anderson step (AAR.c:109)
             rec(1);
-            hipLaunchKernelGGL(bset_kernel, dim3(1), dim3(64), 0, st, clock, 1);
+            hipLaunchKernelGGL(bset_kernel, dim3(1), dim3(64), 0, st, clock, 1, 1);
         }
         BHC(hipGetLastError());
 
