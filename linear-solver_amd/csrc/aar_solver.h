@@ -49,7 +49,6 @@ struct Context {
     DevBuf hist0, hist1, part0, part1;
     DevBuf vec32a, vec32b, vec64a, vec64b;
     DevBuf ringc, corrc;         // complex Helmholtz g ring and corrections
-    DevBuf batch;                // buffers of the batched solver (kept up to a bound)
     DevBuf vch;                  // variable coefficient: the recurrence field h(x)
     DevBuf kctl, kvec, kilu;     // Krylov comparators: control block, basis / work vectors, ILU(0) factors
     std::string err;

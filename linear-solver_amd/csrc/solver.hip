@@ -45,13 +45,6 @@ hipError_t ensure(DevBuf &b, size_t bytes)
     }
     if (bytes == 0) bytes = 256;
     hipError_t e = hipMalloc(&b.p, bytes);
-    DevBuf &kept = ctx().batch;
-    if (e == hipErrorOutOfMemory && kept.p && &b != &kept) {      // idle between batches
-        (void)hipGetLastError();
-        (void)hipFree(kept.p);
-        kept = DevBuf();
-        e = hipMalloc(&b.p, bytes);
-    }
     if (e == hipSuccess) b.bytes = bytes;
     return e;
 }
@@ -1606,7 +1599,7 @@ void release_all()
     Context &C = ctx();
     DevBuf *bufs[] = {&C.ring64x, &C.ring64f, &C.ring32x, &C.ring32f, &C.hist0, &C.hist1,
                       &C.part0, &C.part1, &C.vec32a, &C.vec32b, &C.vec64a, &C.vec64b,
-                      &C.ringc, &C.corrc, &C.batch, &C.vch, &C.kctl, &C.kvec, &C.kilu};
+                      &C.ringc, &C.corrc, &C.vch, &C.kctl, &C.kvec, &C.kilu};
     for (DevBuf *b : bufs) {
         if (b->p) (void)hipFree(b->p);
         b->p = nullptr;

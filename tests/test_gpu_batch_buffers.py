@@ -1,5 +1,6 @@
-"""The batch's buffers are kept between calls: a batch run again after a larger
-and a smaller one, and after solves of its own, gives the same bits."""
+"""The batch's buffers are one allocation of its own: a batch run again after a
+larger and a smaller one, and after solves of its own, gives the same bits, and
+its memory is the caller's again when it returns."""
 import numpy as np
 import pytest
 import torch
@@ -29,3 +30,15 @@ def test_kept_buffers(gpu, mixed):
     x1, it1 = run(gpu, [13, 24, 18], mixed)
     assert it0 == it1
     assert all(np.array_equal(a, b) for a, b in zip(x0, x1))
+
+
+def test_buffers_are_given_back(gpu):
+    print("batch memory", flush=True)
+    run(gpu, [13], False)                       # the library's own context
+    torch.cuda.synchronize()
+    b = torch.zeros(96 * 97 * 98, dtype=torch.float64, device="cuda")
+    args = [(torch.zeros_like(b), b + 1.0, (96, 97, 98), P.poisson_a(0.5), 0.5) for _ in range(4)]
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    gpu.AAR_batch(args, 0.6, 0.6, 7, 6, 12, 1e-8)      # 4 rings of 9 fields: 263 MB
+    assert torch.cuda.mem_get_info()[0] >= before - (32 << 20)
