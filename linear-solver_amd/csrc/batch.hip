@@ -93,7 +93,7 @@ __global__ __launch_bounds__(64 * BWY) void bstencil_kernel(const BInst<Tx, Tg> 
         }
     }
     __syncthreads();
-    stencil_body<T, BWY, BPY / Lane<T>::RPW, MODE, false, WIDE>(sa, wi.idx);
+    stencil_any<T, BWY, BPY / Lane<T>::RPW, MODE, WIDE>(sa, wi.idx);
 }
 
 // per-instance finish of the true residual: relres check (or, at the start, the

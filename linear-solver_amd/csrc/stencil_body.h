@@ -8,8 +8,7 @@
 namespace aar {
 
 // LDS of one march block: the double-buffered plane tile with its x/y halos
-// and the halo ring.  Shared by the two instantiations (interior and edge
-// tiles) of a kernel.
+// and the halo ring.  Shared by the forms of a kernel that holds two of them.
 template <typename T, int WY, int PY> struct March {
     using L = Lane<T>;
     static constexpr int NT = 64 * WY;                       // threads: WY wavefronts stacked in y
@@ -52,7 +51,9 @@ __device__ __forceinline__ void stencil_march(const SArgs<T> &a, const int item,
     const int rest = item / a.ntx;
     const int ity = rest % a.nty;
     const int izc = rest / a.nty;
-    const int x0 = itx * TX, y0 = ity * TY;
+    int x0, own;
+    tile_x0<T, TX, XM>(itx, a.nx, x0, own);
+    const int y0 = ity * TY;
     const int z0 = izc * a.lz;
     const int z1 = min(z0 + a.lz, a.nz);
     const int tid = threadIdx.x, lane = tid & 63;
@@ -66,7 +67,7 @@ __device__ __forceinline__ void stencil_march(const SArgs<T> &a, const int item,
     for (int p = 0; p < PY; p++) {
         c_off[p].set(x0 + xv * V, y0 + r0 + p, nx, ny);
 #pragma unroll
-        for (int v = 0; v < V; v++) c_ok[p][v] = (x0 + xv * V + v < nx) && (y0 + r0 + p < ny);
+        for (int v = 0; v < V; v++) c_ok[p][v] = (x0 + xv * V + v >= own) && (x0 + xv * V + v < nx) && (y0 + r0 + p < ny);
     }
     // halo vectors: 2R rows of LPR, then TY rows of HXV left and HXV right;
     // cells past the halo load a valid (unused) address so that every load is
@@ -228,20 +229,22 @@ __device__ __forceinline__ void stencil_march(const SArgs<T> &a, const int item,
     if (a.partials) block_reduce_to<NACC, NT>(acc, a.partials + (size_t)item * NACC, S.red);
 }
 
-template <typename T, int WY, int PY, SMode MODE, bool VC = false, bool WIDE = false>
-__device__ __forceinline__ void stencil_body(const SArgs<T> &a, const int item)
+// the batch: systems of any sides in one launch
+template <typename T, int WY, int PY, SMode MODE, bool WIDE>
+__device__ __forceinline__ void stencil_any(const SArgs<T> &a, const int item)
 {
     __shared__ typename March<T, WY, PY>::Lds S;
-    if constexpr (WIDE) stencil_march<T, WY, PY, MODE, VC, XWIDE>(a, item, S);
-    else if (edge_tile(a, item)) stencil_march<T, WY, PY, MODE, VC, XPOINT>(a, item, S);
-    else stencil_march<T, WY, PY, MODE, VC, XVEC>(a, item, S);
+    if constexpr (WIDE) stencil_march<T, WY, PY, MODE, false, XWIDE>(a, item, S);
+    else if (x_mode<T>(a.nx, a.ny, TX) == XPOINT) stencil_march<T, WY, PY, MODE, false, XPOINT>(a, item, S);
+    else stencil_march<T, WY, PY, MODE, false, XSHIFT>(a, item, S);
 }
 
-template <typename T, int WY, int PY, SMode MODE, bool VC = false, bool WIDE = false>
+template <typename T, int WY, int PY, SMode MODE, bool VC, int XM>
 __global__ __launch_bounds__(64 * WY) void stencil_kernel(const SArgs<T> a)
 {
+    __shared__ typename March<T, WY, PY>::Lds S;
     if (a.ctrl && a.ctrl->done) return;
-    stencil_body<T, WY, PY, MODE, VC, WIDE>(a, xcd_item(blockIdx.x, a.nitems));
+    stencil_march<T, WY, PY, MODE, VC, XM>(a, xcd_item(blockIdx.x, a.nitems), S);
 }
 
 }  // namespace aar

@@ -62,12 +62,21 @@ template <typename T> struct Lane {
 // 16 (32 x 32: 200 x 161 x 150 32.1 -> 32.9 us, 96^3 14.4 -> 13.7).
 template <typename T> __host__ __device__ constexpr int tile_x(int lz) { return sizeof(T) == 8 && lz > 1 ? 32 : 64; }
 
-// How a tile takes its vectors of V points along x.
-// * XVEC: the V points are consecutive in memory: one access, one offset.
-// * XPOINT (a tile whose window reaches past nx when nx is not a multiple of
-//   V): point by point, a wrapped offset each.
+// How the tiles of a grid take their vectors of V points along x, chosen at
+// launch (x_mode), a kernel each, so that no grid pays for the registers of
+// another's form.
+// * XVEC (nx a multiple of V): the V points are consecutive in memory, one
+//   access and one offset.
+// * XSHIFT (any other nx from a tile and its halo up): tiles that would reach
+//   past nx, or whose halo would, start earlier instead (tile_x0), so that no
+//   vector wraps inside: the same accesses, at any alignment of a row.  Points
+//   covered by two tiles are computed twice, by the same operations; the norms
+//   take them once.  With the tiles at the end of a row point by point (20
+//   accesses for 5), an iteration of the mixed solve took 84 us at 193 x 189 x 196
+//   against 57, the FP32 operator 454 against 274 at 449 x 445 x 452.
+// * XPOINT (narrower grids): point by point, a wrapped offset each.
 // * XWIDE: the same with 64-bit byte offsets, for the planes of wide_plane().
-enum : int { XVEC = 0, XPOINT = 1, XWIDE = 2 };
+enum : int { XVEC = 0, XSHIFT = 1, XPOINT = 2, XWIDE = 3 };
 
 // Byte offsets in a plane are 32 bits wide.  A plane of more than 2^32 bytes
 // (2^29 points FP64, 2^30 FP32) takes the XWIDE sweep.
@@ -95,7 +104,7 @@ template <bool WIDE, typename T> __device__ __forceinline__ void st_at(T *base, 
 
 // in-plane element offsets of one vector of points
 template <typename T, int XM> struct VOff {
-    static constexpr int NO = XM == XVEC ? 1 : Lane<T>::V;
+    static constexpr int NO = XM <= XSHIFT ? 1 : Lane<T>::V;
     unsigned o[NO];
     __device__ __forceinline__ void set(int gx, int gy, int nx, int ny)
     {
@@ -110,7 +119,7 @@ __device__ __forceinline__ typename Lane<T>::Vec ld_vec(const T *base, const VOf
 {
     using L = Lane<T>;
     typename L::Vec r;
-    if constexpr (XM == XVEC) {
+    if constexpr (XM <= XSHIFT) {
         r = *reinterpret_cast<const typename L::VecU *>(reinterpret_cast<const char *>(base) +
                                                         (size_t)(f.o[0] * (unsigned)sizeof(T)));
     } else {
@@ -120,21 +129,40 @@ __device__ __forceinline__ typename Lane<T>::Vec ld_vec(const T *base, const VOf
     return r;
 }
 
-// An edge tile's x-window reaches past nx while nx is not a whole number of
-// vectors: its vectors may wrap inside and are accessed point by point.
-template <typename T, int W = TX> __device__ __forceinline__ bool edge_tile(const SArgs<T> &a, int item)
+template <typename T> __host__ __device__ inline int x_mode(int nx, int ny, int w)
 {
     using L = Lane<T>;
-    return a.nx % L::V != 0 && (item % a.ntx) * W + W + L::HXV * L::V > a.nx;
+    if (wide_plane<T>(nx, ny)) return XWIDE;
+    if (nx % L::V == 0) return XVEC;
+    return nx >= w + L::HXV * L::V ? XSHIFT : XPOINT;
+}
+
+// First point x0 of the W-wide tile itx, and the first one whose norm terms are
+// its own.  XSHIFT: the last tile ends at nx, and the one before it a halo short
+// of nx where its halo would wrap inside a vector.
+template <typename T, int W, int XM>
+__device__ __forceinline__ void tile_x0(int itx, int nx, int &x0, int &own)
+{
+    constexpr int HX = Lane<T>::HXV * Lane<T>::V;
+    x0 = own = itx * W;
+    if constexpr (XM == XSHIFT) {
+        if (nx % Lane<T>::V == 0) return;
+        if (x0 + W >= nx) {
+            own = x0 + HX > nx ? nx - HX : x0;        // where the tile before it ends
+            x0 = nx - W;
+        } else if (x0 + W + HX > nx) {
+            x0 = nx - HX - W;
+        }
+    }
 }
 
 // S: the stored type (T, or float for the FP32 copy of an FP64 sweep).
-// NT: non-temporal.  ok: masks of the V points, or of the vector (XVEC: ok[0]).
+// NT: non-temporal.  ok: masks of the V points, or of the vector (ok[0]).
 template <typename S, bool NT, typename T, int XM, int NV>
 __device__ __forceinline__ void st_vec(S *base, const VOff<T, XM> &f, const S (&v)[NV], const bool (&ok)[NV],
                                        bool masked)
 {
-    if constexpr (XM == XVEC) {
+    if constexpr (XM <= XSHIFT) {
         typedef S SV __attribute__((ext_vector_type(NV), aligned(sizeof(S))));
         SV r;
 #pragma unroll
@@ -278,7 +306,7 @@ __device__ __forceinline__ typename Lane<T>::Vec stencil_value(const SArgs<T> &a
 // what the lane owning the wrapped point reads, through the same operations,
 // so it may store the same bits to the same address: put may store
 // unconditionally (no branch per point) or masked.  Norm terms are always
-// masked, per point in an edge tile, else per vector.
+// masked, per vector in XVEC, else per point.
 template <typename T, SMode MODE, bool VC, int XM, int NACC, typename Put>
 __device__ __forceinline__ void stencil_epilogue(const SArgs<T> &a, const PointK<T> &k,
                                                  const typename Lane<T>::Vec y, const typename Lane<T>::Vec u,

@@ -49,7 +49,9 @@ __device__ __forceinline__ void stencil_box(const SArgs<T> &a, const int item, t
     const int rest = item / a.ntx;
     const int ity = rest % a.nty;
     const int izc = rest / a.nty;
-    const int x0 = itx * BX, y0 = ity * TY, z0 = izc * LZ;
+    int x0, own;
+    tile_x0<T, BX, XM>(itx, a.nx, x0, own);
+    const int y0 = ity * TY, z0 = izc * LZ;
     const int tid = threadIdx.x, lane = tid & 63;
     const int xv = lane % LPR;
     const int r0 = ((tid >> 6) * B::RPW + lane / LPR) * PY;
@@ -58,12 +60,16 @@ __device__ __forceinline__ void stencil_box(const SArgs<T> &a, const int item, t
     const PointK<T> k(a);
 
     Off c_off[PY];
-    bool c_ok[PY][V];
+    bool c_ok[PY][V], s_ok[PY][V];                                 // norm terms; stores
 #pragma unroll
     for (int p = 0; p < PY; p++) {
         c_off[p].set(x0 + xv * V, y0 + r0 + p, nx, ny);
 #pragma unroll
-        for (int v = 0; v < V; v++) c_ok[p][v] = (x0 + xv * V + v < nx) && (y0 + r0 + p < ny);
+        for (int v = 0; v < V; v++) {
+            const int gx = x0 + xv * V + v;
+            s_ok[p][v] = gx < nx && y0 + r0 + p < ny;
+            c_ok[p][v] = s_ok[p][v] && gx >= own;
+        }
     }
     // element offsets of the planes z0-R .. z0+LZ-1+R (wrapped; uniform)
     size_t zo[NQ];
@@ -161,7 +167,7 @@ __device__ __forceinline__ void stencil_box(const SArgs<T> &a, const int item, t
                 constexpr bool NT_OUT = MODE == SMode::PGR_STEP;
                 auto put = [&](auto *base, const auto &o) {
                     st_vec<std::remove_pointer_t<decltype(base)>, NT_OUT, T, XM>(base + zo[R + s], c_off[p], o,
-                                                                                  c_ok[p], true);
+                                                                                  s_ok[p], true);
                 };
                 stencil_epilogue<T, MODE, VC, XM>(a, k, y, u, en[p][s], vv[p][s], c_ok[p], put, acc);
             }
@@ -170,19 +176,12 @@ __device__ __forceinline__ void stencil_box(const SArgs<T> &a, const int item, t
     if (a.partials) block_reduce_to<NACC, NT>(acc, a.partials + (size_t)item * NACC, S.red);
 }
 
-template <typename T, int WY, int PY, int LZ, SMode MODE, bool VC = false>
-__device__ __forceinline__ void stencil_tile_body(const SArgs<T> &a, const int item)
-{
-    __shared__ typename Tile<T, WY, PY, LZ>::Lds S;
-    if (edge_tile<T, tile_x<T>(LZ)>(a, item)) stencil_box<T, WY, PY, LZ, MODE, VC, XPOINT>(a, item, S);
-    else stencil_box<T, WY, PY, LZ, MODE, VC, XVEC>(a, item, S);
-}
-
-template <typename T, int WY, int PY, int LZ, SMode MODE, bool VC = false>
+template <typename T, int WY, int PY, int LZ, SMode MODE, bool VC, int XM>
 __global__ __launch_bounds__(64 * WY) void stencil_tile_kernel(const SArgs<T> a)
 {
+    __shared__ typename Tile<T, WY, PY, LZ>::Lds S;
     if (a.ctrl && a.ctrl->done) return;
-    stencil_tile_body<T, WY, PY, LZ, MODE, VC>(a, xcd_item(blockIdx.x, a.nitems));
+    stencil_box<T, WY, PY, LZ, MODE, VC, XM>(a, xcd_item(blockIdx.x, a.nitems), S);
 }
 
 }  // namespace aar
