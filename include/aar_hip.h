@@ -375,7 +375,10 @@ int aar_hip_last_system(int n, double *G, double *w);
  * its write) / time, in 1e9 B/s. */
 int aar_hip_stream_bandwidth(int kind, void *dst, const void *src, long bytes, int reps, double *gbps);
 
-/* Release cached device workspace. */
+/* Release cached device workspace: the single solves' rings and vectors (kept
+ * at the largest size used) and up to 1 GiB of the batched solver's.  The
+ * library's own allocations drop the batch's block when memory runs out; a
+ * caller that needs it for allocations of its own calls this. */
 int aar_hip_release(void);
 
 const char *aar_hip_last_error(void);

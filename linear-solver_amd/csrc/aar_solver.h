@@ -49,6 +49,7 @@ struct Context {
     DevBuf hist0, hist1, part0, part1;
     DevBuf vec32a, vec32b, vec64a, vec64b;
     DevBuf ringc, corrc;         // complex Helmholtz g ring and corrections
+    DevBuf batch;                // buffers of the batched solver (kept up to a bound)
     DevBuf vch;                  // variable coefficient: the recurrence field h(x)
     DevBuf kctl, kvec, kilu;     // Krylov comparators: control block, basis / work vectors, ILU(0) factors
     std::string err;
@@ -86,6 +87,9 @@ struct Op {
 
 Context &ctx();
 int context_init();
+// every device allocation of the library: one that finds no memory drops the
+// block that the last batch kept, and tries again
+hipError_t dev_alloc(void **p, size_t bytes);
 hipError_t ensure(DevBuf &b, size_t bytes);
 int auto_lz(const Op &op, int wy, int py, size_t es);
 long ring_ld(long n, size_t es);

@@ -331,9 +331,7 @@ __global__ void bclock_kernel(int *clock, int p) { if (threadIdx.x == 0 && block
 __global__ void bset_kernel(int *v, int value, int n) { for (int i = threadIdx.x; i < n; i += blockDim.x) v[i] = value; }
 
 // A batch's buffers are cut from one allocation, laid out twice: first from
-// address zero for its size, then in place.  It is given back when the batch
-// returns, so that the caller's own allocator finds the memory: at 1.4 GB (40
-// systems of sides 24 to 128) that costs 0.7 of 47.5 ms, 240 buffers took 15.
+// address zero for its size, then in place.
 struct Arena {
     char *base = nullptr;
     size_t used = 0;
@@ -344,6 +342,14 @@ struct Arena {
         return p;
     }
 };
+
+// The allocation is kept for the next batch up to this size, where it counts: a
+// batch of 16 cycles on 40 systems of sides 24 to 48 (0.2 GB) takes 7.2 ms, 7.8
+// with a fresh one.  A larger one is given back when the batch returns (40 of
+// sides 24 to 128, 1.4 GB: 47.5 ms, kept 46.9).  The kept block is dropped when
+// any other allocation of the library needs the memory (dev_alloc) and by
+// aar_hip_release().
+constexpr size_t BATCH_KEEP = (size_t)1 << 30;
 
 }  // namespace
 
@@ -375,7 +381,6 @@ int batch_solve(const aar_hip_instance *ins, int count, double omega, double bet
     WorkItem *dtr = nullptr, *drc = nullptr, *dch = nullptr;
     Ctrl *ctrls = nullptr;
     int *clock = nullptr, *ndone = nullptr, *const ndone_h = C.poll_h;
-    DevBuf buf;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     const int S = m + 2;
@@ -400,7 +405,7 @@ int batch_solve(const aar_hip_instance *ins, int count, double omega, double bet
     BHC(hipStreamWaitEvent(st, ev_in, 0));
     for (int pass = 0; pass < 2; pass++) {
         Arena ar;
-        if (pass == 1) ar.base = (char *)buf.p;
+        if (pass == 1) ar.base = (char *)C.batch.p;
         ctrls = ar.take<Ctrl>(count);
         clock = ar.take<int>(2 + count);     // the clock, ndone and the systems' counted flags
         ndone = clock + 1;
@@ -471,7 +476,7 @@ int batch_solve(const aar_hip_instance *ins, int count, double omega, double bet
         dtr = ar.take<WorkItem>(wtr.size());
         drc = ar.take<WorkItem>(wrc.size());
         dch = ar.take<WorkItem>(wch.size());
-        if (pass == 0) BHC(ensure(buf, ar.used));
+        if (pass == 0) BHC(ensure(C.batch, ar.used));
     }
     BHC(hipMemcpy(dI, hI.data(), sizeof(BInst<Tx, Tg>) * count, hipMemcpyHostToDevice));
     BHC(hipMemcpy(dtr, wtr.data(), sizeof(WorkItem) * wtr.size(), hipMemcpyHostToDevice));
@@ -617,7 +622,10 @@ done:
     if (exec) (void)hipGraphExecDestroy(exec);
     if (graph) (void)hipGraphDestroy(graph);
     (void)hipStreamSynchronize(st);
-    if (buf.p) (void)hipFree(buf.p);
+    if (C.batch.bytes > BATCH_KEEP) {
+        (void)hipFree(C.batch.p);
+        C.batch = DevBuf();
+    }
     if (ev_in) (void)hipEventDestroy(ev_in);
     if (ev_out) (void)hipEventDestroy(ev_out);
     return rc;

@@ -58,8 +58,8 @@ int stage(long n)
     if (g_stage.b) (void)hipFree(g_stage.b);
     g_stage.x = g_stage.b = nullptr;
     g_stage.cap = 0;
-    HCR(hipMalloc(&g_stage.x, bytes), AAR_HIP_ERR_HIP);
-    HCR(hipMalloc(&g_stage.b, bytes), AAR_HIP_ERR_HIP);
+    HCR(dev_alloc((void **)&g_stage.x, bytes), AAR_HIP_ERR_HIP);
+    HCR(dev_alloc((void **)&g_stage.b, bytes), AAR_HIP_ERR_HIP);
     g_stage.cap = bytes;
     return 0;
 }
@@ -251,7 +251,7 @@ int step_upload(double **DX, double **DF, const double *f, int m, int n, StepBuf
         if (b.p) (void)hipFree(b.p);
         b.p = nullptr;
         b.bytes = 0;
-        HCR(hipMalloc(&b.p, need), AAR_HIP_ERR_HIP);
+        HCR(dev_alloc(&b.p, need), AAR_HIP_ERR_HIP);
         b.bytes = need;
         return 0;
     };
@@ -281,7 +281,7 @@ int step_gram_ls(int kind, const StepBufs &sb, int m, int n)
         if (part.p) (void)hipFree(part.p);
         part.p = nullptr;
         part.bytes = 0;
-        HCR(hipMalloc(&part.p, sizeof(double) * nb * GRAM_NA_MAX), AAR_HIP_ERR_HIP);
+        HCR(dev_alloc(&part.p, sizeof(double) * nb * GRAM_NA_MAX), AAR_HIP_ERR_HIP);
         part.bytes = sizeof(double) * nb * GRAM_NA_MAX;
     }
     HCR(launch_zero_ctrl(dc, C.stream), AAR_HIP_ERR_HIP);

@@ -34,6 +34,21 @@ namespace aar {
 static Context g_ctx;
 Context &ctx() { return g_ctx; }
 
+hipError_t dev_alloc(void **p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    DevBuf &kept = ctx().batch;
+    if (e == hipErrorOutOfMemory && kept.p) {      // idle between batches
+        (void)hipGetLastError();
+        (void)hipFree(kept.p);
+        kept = DevBuf();
+        e = hipMalloc(p, bytes);
+    }
+    // the caller has the error: not for the next launch's check
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
+}
+
 hipError_t ensure(DevBuf &b, size_t bytes)
 {
     if (b.p && b.bytes >= bytes) return hipSuccess;
@@ -44,8 +59,9 @@ hipError_t ensure(DevBuf &b, size_t bytes)
         if (e != hipSuccess) return e;
     }
     if (bytes == 0) bytes = 256;
-    hipError_t e = hipMalloc(&b.p, bytes);
+    hipError_t e = dev_alloc(&b.p, bytes);
     if (e == hipSuccess) b.bytes = bytes;
+    else b.p = nullptr;
     return e;
 }
 
@@ -70,10 +86,10 @@ int context_init()
     // which is where framework callers (torch's default stream) put inputs
     HC(hipStreamCreateWithFlags(&C.own, hipStreamDefault));
     if (!C.stream_set) C.stream = C.own;
-    HC(hipMalloc((void **)&C.ctrl, 2 * sizeof(Ctrl)));
+    HC(dev_alloc((void **)&C.ctrl, 2 * sizeof(Ctrl)));
     HC(hipHostMalloc((void **)&C.ctrl_h, 2 * sizeof(Ctrl), hipHostMallocDefault));
     HC(hipHostMalloc((void **)&C.poll_h, NPOLL * sizeof(int), hipHostMallocDefault));
-    HC(hipMalloc((void **)&C.counters, 64 * sizeof(unsigned)));
+    HC(dev_alloc((void **)&C.counters, 64 * sizeof(unsigned)));
     HC(hipMemset(C.counters, 0, 64 * sizeof(unsigned)));
     for (int i = 0; i < NPOLL; i++) HC(hipEventCreateWithFlags(&C.poll_ev[i], hipEventDisableTiming));
     HC(hipEventCreate(&C.t0));
@@ -419,8 +435,8 @@ static int autotune_t(int nx, int ny, int nz, bool batch_shape, Shape *out)
     Op op;
     if (int rc = make_op(&g, nullptr, op)) return rc;
     T *in = nullptr, *o = nullptr;
-    HC(hipMalloc((void **)&in, sizeof(T) * op.n));
-    if (hipMalloc((void **)&o, sizeof(T) * op.n) != hipSuccess) {
+    HC(dev_alloc((void **)&in, sizeof(T) * op.n));
+    if (dev_alloc((void **)&o, sizeof(T) * op.n) != hipSuccess) {
         (void)hipFree(in);
         return fail(AAR_HIP_ERR_HIP, "autotune: out of device memory");
     }
@@ -1599,7 +1615,7 @@ void release_all()
     Context &C = ctx();
     DevBuf *bufs[] = {&C.ring64x, &C.ring64f, &C.ring32x, &C.ring32f, &C.hist0, &C.hist1,
                       &C.part0, &C.part1, &C.vec32a, &C.vec32b, &C.vec64a, &C.vec64b,
-                      &C.ringc, &C.corrc, &C.vch, &C.kctl, &C.kvec, &C.kilu};
+                      &C.ringc, &C.corrc, &C.batch, &C.vch, &C.kctl, &C.kvec, &C.kilu};
     for (DevBuf *b : bufs) {
         if (b->p) (void)hipFree(b->p);
         b->p = nullptr;

@@ -1,6 +1,6 @@
-"""The batch's buffers are one allocation of its own: a batch run again after a
-larger and a smaller one, and after solves of its own, gives the same bits, and
-its memory is the caller's again when it returns."""
+"""The batch's buffers are one allocation, kept up to a bound: a batch run again
+after a larger and a smaller one, and after solves of its own, gives the same
+bits."""
 import numpy as np
 import pytest
 import torch
@@ -32,13 +32,39 @@ def test_kept_buffers(gpu, mixed):
     assert all(np.array_equal(a, b) for a, b in zip(x0, x1))
 
 
-def test_buffers_are_given_back(gpu):
+def free_memory():
+    torch.cuda.synchronize()
+    return torch.cuda.mem_get_info()[0]
+
+
+def batch(gpu, side, count):
+    b = torch.ones(side ** 3, dtype=torch.float64, device="cuda")
+    args = [(torch.zeros_like(b), b, (side, side, side), P.poisson_a(0.5), 0.5) for _ in range(count)]
+    before = free_memory()
+    gpu.AAR_batch(args, 0.6, 0.6, 7, 6, 12, 1e-8)
+    return before
+
+
+def test_what_is_kept_and_given_back(gpu):
+    """Above 1 GiB nothing is kept; below, the block goes when another allocation
+    of the library finds no memory, and with release()."""
     print("batch memory", flush=True)
     run(gpu, [13], False)                       # the library's own context
-    torch.cuda.synchronize()
-    b = torch.zeros(96 * 97 * 98, dtype=torch.float64, device="cuda")
-    args = [(torch.zeros_like(b), b + 1.0, (96, 97, 98), P.poisson_a(0.5), 0.5) for _ in range(4)]
-    torch.cuda.synchronize()
-    before = torch.cuda.mem_get_info()[0]
-    gpu.AAR_batch(args, 0.6, 0.6, 7, 6, 12, 1e-8)      # 4 rings of 9 fields: 263 MB
-    assert torch.cuda.mem_get_info()[0] >= before - (32 << 20)
+    gpu.release()
+    slack = 32 << 20
+    before = batch(gpu, 128, 9)                 # 9 rings of 9 fields and 2 more each: 1.6 GB
+    assert free_memory() >= before - slack
+    before = batch(gpu, 96, 8)                  # 0.6 GB
+    assert before - (1 << 30) <= free_memory() <= before - (400 << 20)
+    # a history of 34 fields of 17 GB: more than any card holds, refused by the host
+    x = torch.empty(1290 ** 3, dtype=torch.float64, device="cuda")
+    b = torch.empty_like(x)
+    with pytest.raises(Exception, match="memory"):
+        gpu.AAR(x, b, (1290, 1290, 1290), P.poisson_a(0.5), 0.6, 0.6, 32, 6, 12, 1e-8)
+    del x, b
+    torch.cuda.empty_cache()
+    assert free_memory() >= before - slack
+    before = batch(gpu, 96, 8)
+    gpu.release()
+    assert free_memory() >= before - slack
+    run(gpu, [14], False)                       # nothing left over from the refusal
