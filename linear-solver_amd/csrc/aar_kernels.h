@@ -42,15 +42,21 @@ struct SArgs {
 
 // Launch shape of the sweeps: tile = 0: the z-march (stencil_body.h), a block
 // owning a 64 x (wy*py) column over lz planes; tile > 0: the one-shot boxes of
-// stencil_tile.h, `tile` (1, 2 or 4) planes deep.
+// stencil_tile.h, `tile` (1, 2 or 4) planes deep.  w < 64: columns w wide and
+// narrow_rows() * 64/w high, whatever wy and py.
 struct Shape {
     int lz = 0, wy = 8, py = 4;
     int tile = 0;
+    int w = TX;               // width of the march's columns (march_width)
     double us = 0.0;          // measured time of one recurrence sweep (tuned shapes)
 };
 
 // (a plane beyond the sweeps' 32-bit offsets always marches 64 x WIDE_ROWS columns)
 constexpr int WIDE_ROWS = 32;
+template <typename T> constexpr int narrow_rows() { return sizeof(T) == 8 ? 32 : 16; }
+// width of the march's columns on this grid
+template <typename T>
+int march_width(int nx, int ny);
 template <typename T>
 hipError_t launch_stencil(SMode m, const SArgs<T> &a, const Shape &sh, hipStream_t st);
 // blocks (= partials per sum) of the sweep

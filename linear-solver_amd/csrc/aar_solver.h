@@ -91,7 +91,7 @@ int context_init();
 // block that the last batch kept, and tries again
 hipError_t dev_alloc(void **p, size_t bytes);
 hipError_t ensure(DevBuf &b, size_t bytes);
-int auto_lz(const Op &op, int wy, int py, size_t es);
+int auto_lz(const Op &op, int wy, int py, size_t es, int w = TX);
 long ring_ld(long n, size_t es);
 int nblocks_for(long n);
 // grid of the register Gram (m <= 8) on n points

@@ -158,9 +158,10 @@ int make_op(const aar_hip_grid *g, const double *coeff, Op &op)
 // ---------------------------------------------------------------------------
 // launch helpers
 // ---------------------------------------------------------------------------
-int auto_lz(const Op &op, int wy, int py, size_t es)
+int auto_lz(const Op &op, int wy, int py, size_t es, int w)
 {
-    const int ntx = (op.nx + TX - 1) / TX, nty = (op.ny + wy * py - 1) / (wy * py);
+    const int rows = wy * py * TX / w;
+    const int ntx = (op.nx + w - 1) / w, nty = (op.ny + rows - 1) / rows;
     const int cols = ntx * nty;
     // long z-marches amortise the 2R-plane warm-up: about one block per CU
     // for FP64 (its plane tile and halo ring take most of the LDS, so only
@@ -198,7 +199,8 @@ Shape stencil_shape(int nx, int ny, int nz, size_t es)
         // (512^3 recurrence 230 us; 64 x 32 of eight 246, 64 x 64 233)
         if (es == 4) sh.wy = 4;
     }
-    sh.lz = C.lz > 0 ? C.lz : auto_lz(op, sh.wy, sh.py, es);
+    sh.w = es == 4 ? march_width<float>(nx, ny) : march_width<double>(nx, ny);
+    sh.lz = C.lz > 0 ? C.lz : auto_lz(op, sh.wy, sh.py, es, sh.w);
     return sh;
 }
 
@@ -443,7 +445,8 @@ static int autotune_t(int nx, int ny, int nz, bool batch_shape, Shape *out)
     if (sizeof(T) == 8) (void)launch_fill_f64((double *)in, 1.0, op.n, C.stream);
     else (void)launch_fill_f32((float *)in, 1.0f, op.n, C.stream);
     const int shapes[5][2] = {{8, 4}, {4, 8}, {8, 2}, {4, 4}, {4, 2}};
-    const int nshape = batch_shape ? 1 : 5;
+    const int width = batch_shape ? TX : march_width<T>(nx, ny);      // the batch marches 64 wide
+    const int nshape = batch_shape || width < TX ? 1 : 5;
     Shape best;
     best.us = 1e300;
     hipEvent_t e0, e1;
@@ -476,13 +479,14 @@ static int autotune_t(int nx, int ny, int nz, bool batch_shape, Shape *out)
     };
     for (int si = 0; si < nshape && !rc; si++) {
         const int wy = shapes[si][0], py = shapes[si][1];
-        std::vector<int> lzs = {auto_lz(op, wy, py, sizeof(T)), nz, (nz + 1) / 2, (nz + 3) / 4, (nz + 7) / 8};
+        std::vector<int> lzs = {auto_lz(op, wy, py, sizeof(T), width), nz, (nz + 1) / 2, (nz + 3) / 4, (nz + 7) / 8};
         std::sort(lzs.begin(), lzs.end());
         lzs.erase(std::unique(lzs.begin(), lzs.end()), lzs.end());
         for (int lz : lzs) {
             if (lz < std::min(nz, 16)) continue;
             Shape sh;
             sh.lz = lz;
+            sh.w = width;
             sh.wy = wy;
             sh.py = py;
             if ((rc = time_shape(sh))) break;

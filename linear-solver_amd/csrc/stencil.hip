@@ -27,6 +27,8 @@
 // at 512^3: FP64 487 -> 436 us (4.9 TB/s of the two vectors), FP32 285 -> 230
 // us; the true residual 680 -> 580 us.
 //
+// Rows that are no multiple of 16 bytes keep 16-byte accesses (x_mode).
+//
 // The one-shot boxes (stencil_tile.h), for the smaller grids.
 //
 // The epilogue of each mode fuses the pointwise work of the solver step
@@ -44,13 +46,35 @@ namespace aar {
 // Rows of a one-shot box: four wavefronts, one vector per thread.
 template <typename T> static int tile_rows(int lz) { return 256 * Lane<T>::V / tile_x<T>(lz); }
 
+// 64, but where rows are no multiple of a vector and too narrow for tiles of 64
+// that start early (XSHIFT) the widest of 32 and 16 that leaves room for them.
+// FP32 operator, 64 wide point by point / this: 65 x 600 x 500 136 / 88 us, 61 wide
+// 80 / 64, 37 wide 74 / 59, 29 wide 72 / 47.  FP64 loses less by points (8 bytes
+// each), so only where fewer lanes are left idle: 65 wide 165 / 127, 29 wide 86 /
+// 66, but an AAR iteration at 45 wide (32 as idle as 64) 144 / 155 and at 37 (16) 130 /
+// 141.
+template <typename T>
+int march_width(int nx, int ny)
+{
+    auto lanes = [&](int w) { return (nx + w - 1) / w * w; };
+    if (x_mode<T>(nx, ny, TX) != XPOINT) return TX;
+    for (int w : {32, 16})
+        if (x_mode<T>(nx, ny, w) == XSHIFT && (sizeof(T) == 4 || 4 * lanes(w) <= (w == 32 ? 3 : 2) * lanes(TX))) return w;
+    return TX;
+}
+
 // Where the boxes are faster than the march (recurrence sweep; FP64 with a
 // one-vector update, microseconds, march of 64 x 16 columns against boxes):
 // FP64 48^3 20.1 / 9.5, 96^3 24.4 / 15.4, 128^3 30.3 / 26.3, 160^3 43.9 / 44.3,
 // 200 x 161 x 150 56.2 / 57.4, 200^3 86.3 / 88.6, 256^3 (sweep alone) 67 / 103;
 // FP32 (sweep alone) 48^3 7.9 / 4.9, 96^3 9.5 / 8.3, 160^3 17.4 / 16.3, 200^3
 // 29.6 / 28.8, 256^3 41 / 50.  The two meet at about 8 million points; near the
-// tie the boxes need no depth chosen to fit.  Boxes of 4 planes read (4 + 12)/4
+// tie the boxes need no depth chosen to fit.  FP32 boxes that go point
+// by point (x_mode) give way to the march in narrow columns earlier: from 2.4
+// million lanes of their 64-wide tiles (61 x 200 x 200, 2.6 million lanes, 20.5 /
+// 22.4; 65 x 140 x 140, 2.5, 20.5 / 22.2; 61 x 140 x 140, 1.3, 20.1 / 17.3), from 4.5
+// million against columns of 16 (25 x 200 x 200, 2.6, 22.8 / 16.5; 37 x 300 x 300,
+// 5.8, 26.6 / 28.6).  Boxes of 4 planes read (4 + 12)/4
 // values a point; while they are about one a CU or fewer, boxes of 2 planes are
 // shorter (FP32 96^3 8.7 -> 8.3 us, FP64 true residual 64^3 7.9 -> 6.2; 128^3
 // 15.8 -> 16.8), and of one plane while those leave half the CUs idle (48^3
@@ -61,6 +85,9 @@ int stencil_tile_planes(int nx, int ny, int nz)
 {
     const long n = (long)nx * ny * nz;
     if (n > 8500000L) return 0;
+    const int mw = march_width<T>(nx, ny);
+    const long lanes = (long)((nx + TX - 1) / TX * TX) * ny * nz;
+    if (sizeof(T) == 4 && mw < TX && lanes > (mw == 32 ? 2400000L : 4500000L)) return 0;
     auto cols = [&](int lz) {
         return (long)((nx + tile_x<T>(lz) - 1) / tile_x<T>(lz)) * ((ny + tile_rows<T>(lz) - 1) / tile_rows<T>(lz));
     };
@@ -71,8 +98,10 @@ int stencil_tile_planes(int nx, int ny, int nz)
 template <typename T>
 void stencil_geometry(SArgs<T> &a, const Shape &sh)
 {
-    const int tx = sh.tile ? tile_x<T>(sh.tile) : TX;
-    const int ty = wide_plane<T>(a.nx, a.ny) ? WIDE_ROWS : (sh.tile ? tile_rows<T>(sh.tile) : sh.wy * sh.py);
+    int tx = sh.w, ty = sh.wy * sh.py;
+    if (wide_plane<T>(a.nx, a.ny)) ty = WIDE_ROWS;
+    else if (sh.tile) tx = tile_x<T>(sh.tile), ty = tile_rows<T>(sh.tile);
+    else if (sh.w < TX) ty = narrow_rows<T>() * TX / sh.w;
     a.nxy = a.nx * a.ny;
     a.ntx = (a.nx + tx - 1) / tx;
     a.nty = (a.ny + ty - 1) / ty;
@@ -122,6 +151,8 @@ template int stencil_items<double>(const SArgs<double> &, const Shape &);
 template int stencil_items<float>(const SArgs<float> &, const Shape &);
 template void stencil_geometry<double>(SArgs<double> &, const Shape &);
 template void stencil_geometry<float>(SArgs<float> &, const Shape &);
+template int march_width<double>(int, int);
+template int march_width<float>(int, int);
 template int stencil_tile_planes<double>(int, int, int);
 template int stencil_tile_planes<float>(int, int, int);
 

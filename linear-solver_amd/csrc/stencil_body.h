@@ -9,16 +9,18 @@ namespace aar {
 
 // LDS of one march block: the double-buffered plane tile with its x/y halos
 // and the halo ring.  Shared by the forms of a kernel that holds two of them.
-template <typename T, int WY, int PY> struct March {
+template <typename T, int WY, int PY, int W> struct March {
     using L = Lane<T>;
     static constexpr int NT = 64 * WY;                       // threads: WY wavefronts stacked in y
-    static constexpr int TY = WY * L::RPW * PY;
+    static constexpr int LPR = W / L::V, RPW = 64 / LPR;     // lanes a row, rows a wavefront
+    static constexpr int LW = W + 2 * L::HXV * L::V;         // row pitch of the plane tile
+    static constexpr int TY = WY * RPW * PY;
     static constexpr int LH = TY + 2 * R;
-    static constexpr int NHC = 2 * R * L::LPR + TY * 2 * L::HXV;   // halo vectors of a plane
+    static constexpr int NHC = 2 * R * LPR + TY * 2 * L::HXV;      // halo vectors of a plane
     static constexpr int NH = (NHC + NT - 1) / NT;           // per thread
     static constexpr int HR = R + 1;                         // halo ring depth (planes)
     struct Lds {
-        typename L::Vec tile[2][LH][L::LW / L::V];
+        typename L::Vec tile[2][LH][LW / L::V];
         // Halo cells are fetched R planes ahead, in the same step as the
         // neighbouring blocks fetch those lines as their own queue planes, so
         // that they are served from L2; each thread parks its cells here until
@@ -28,20 +30,21 @@ template <typename T, int WY, int PY> struct March {
     };
 };
 
-// The stencil sweep of one work item (a 64 x TY column over a z-chunk) of
+// The stencil sweep of one work item (a W x TY column over a z-chunk) of
 // the operator and fields in `a`; shared by the single-operator kernel
 // below and the batched kernel of batch.hip.  WY wavefronts, PY rows per
 // thread.  VC: the variable-coefficient operator a*Lap + c(x), with a
 // pointwise field a.vf read in the epilogue.
-template <typename T, int WY, int PY, SMode MODE, bool VC, int XM>
-__device__ __forceinline__ void stencil_march(const SArgs<T> &a, const int item, typename March<T, WY, PY>::Lds &S)
+template <typename T, int WY, int PY, SMode MODE, bool VC, int XM, int W = TX>
+__device__ __forceinline__ void stencil_march(const SArgs<T> &a, const int item,
+                                              typename March<T, WY, PY, W>::Lds &S)
 {
     static_assert(!VC || MODE != SMode::RESID, "no variable-coefficient RESID sweep");
-    using M = March<T, WY, PY>;
+    using M = March<T, WY, PY, W>;
     using L = Lane<T>;
     using Vec = typename L::Vec;
     using Off = VOff<T, XM>;
-    constexpr int V = L::V, LPR = L::LPR, HXV = L::HXV;
+    constexpr int V = L::V, LPR = M::LPR, HXV = L::HXV;
     constexpr int NT = M::NT, TY = M::TY, NHC = M::NHC, NH = M::NH, HR = M::HR;
     constexpr int NE = ModeInfo<MODE>::NE;
     constexpr int NACC = ModeInfo<MODE>::NACC;
@@ -52,13 +55,13 @@ __device__ __forceinline__ void stencil_march(const SArgs<T> &a, const int item,
     const int ity = rest % a.nty;
     const int izc = rest / a.nty;
     int x0, own;
-    tile_x0<T, TX, XM>(itx, a.nx, x0, own);
+    tile_x0<T, W, XM>(itx, a.nx, x0, own);
     const int y0 = ity * TY;
     const int z0 = izc * a.lz;
     const int z1 = min(z0 + a.lz, a.nz);
     const int tid = threadIdx.x, lane = tid & 63;
     const int xv = lane % LPR;                                     // vector of the row
-    const int r0 = ((tid >> 6) * L::RPW + lane / LPR) * PY;        // first row of this thread
+    const int r0 = ((tid >> 6) * M::RPW + lane / LPR) * PY;        // first row of this thread
     const int nx = a.nx, ny = a.ny, nz = a.nz, nxy = a.nxy;
 
     Off c_off[PY];
@@ -87,7 +90,7 @@ __device__ __forceinline__ void stencil_march(const SArgs<T> &a, const int item,
             h_col[k] = HXV + w;
         } else {
             const int r = (c - 2 * R * LPR) / (2 * HXV), w = (c - 2 * R * LPR) % (2 * HXV);
-            h_off[k].set(w < HXV ? x0 - (HXV - w) * V : x0 + TX + (w - HXV) * V, y0 + r, nx, ny);
+            h_off[k].set(w < HXV ? x0 - (HXV - w) * V : x0 + W + (w - HXV) * V, y0 + r, nx, ny);
             h_row[k] = R + r;
             h_col[k] = w < HXV ? w : LPR + w;
         }
@@ -233,18 +236,18 @@ __device__ __forceinline__ void stencil_march(const SArgs<T> &a, const int item,
 template <typename T, int WY, int PY, SMode MODE, bool WIDE>
 __device__ __forceinline__ void stencil_any(const SArgs<T> &a, const int item)
 {
-    __shared__ typename March<T, WY, PY>::Lds S;
+    __shared__ typename March<T, WY, PY, TX>::Lds S;
     if constexpr (WIDE) stencil_march<T, WY, PY, MODE, false, XWIDE>(a, item, S);
     else if (x_mode<T>(a.nx, a.ny, TX) == XPOINT) stencil_march<T, WY, PY, MODE, false, XPOINT>(a, item, S);
     else stencil_march<T, WY, PY, MODE, false, XSHIFT>(a, item, S);
 }
 
-template <typename T, int WY, int PY, SMode MODE, bool VC, int XM>
+template <typename T, int WY, int PY, SMode MODE, bool VC, int XM, int W>
 __global__ __launch_bounds__(64 * WY) void stencil_kernel(const SArgs<T> a)
 {
-    __shared__ typename March<T, WY, PY>::Lds S;
+    __shared__ typename March<T, WY, PY, W>::Lds S;
     if (a.ctrl && a.ctrl->done) return;
-    stencil_march<T, WY, PY, MODE, VC, XM>(a, xcd_item(blockIdx.x, a.nitems), S);
+    stencil_march<T, WY, PY, MODE, VC, XM, W>(a, xcd_item(blockIdx.x, a.nitems), S);
 }
 
 }  // namespace aar

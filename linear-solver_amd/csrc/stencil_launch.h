@@ -6,17 +6,18 @@
 
 namespace aar {
 
-// A column of 64 x (wy*py) points.  A wavefront covers RPW rows of the tile
+// A column of 64 x (wy*py) points (TW x (wy*py*64/TW) on narrow grids).  A
+// wavefront covers RPW rows of the tile
 // (2 in FP64, 4 in FP32), so wy*py rows are wy wavefronts with wy*py/(RPW wy)
 // rows per thread, or fewer wavefronts where that is below one row.
-template <typename T, SMode M, bool VC, int WY, int ROWS, int XM>
+template <typename T, SMode M, bool VC, int WY, int ROWS, int XM, int TW = TX>
 hipError_t launch_march_x(const SArgs<T> &a, hipStream_t st)
 {
     constexpr int RPW = Lane<T>::RPW;
     constexpr int W = WY * RPW <= ROWS ? WY : ROWS / RPW;
     constexpr int PY = ROWS / (W * RPW);
     static_assert(W * RPW * PY == ROWS, "whole rows");
-    hipLaunchKernelGGL((stencil_kernel<T, W, PY, M, VC, XM>), dim3(a.nitems), dim3(64 * W), 0, st, a);
+    hipLaunchKernelGGL((stencil_kernel<T, W, PY, M, VC, XM, TW>), dim3(a.nitems), dim3(64 * W), 0, st, a);
     return hipGetLastError();
 }
 template <typename T, SMode M, bool VC, int WY, int ROWS>
@@ -46,6 +47,10 @@ hipError_t launch_sweep(SArgs<T> a, const Shape &sh, hipStream_t st)
 {
     stencil_geometry(a, sh);
     if (wide_plane<T>(a.nx, a.ny)) return launch_march_x<T, M, VC, 8, WIDE_ROWS, XWIDE>(a, st);
+    // narrow grids: one launch shape, the default one's wavefronts and rows
+    constexpr int NWY = sizeof(T) == 8 ? 8 : 4;
+    if (sh.tile == 0 && sh.w == 32) return launch_march_x<T, M, VC, NWY, narrow_rows<T>(), XSHIFT, 32>(a, st);
+    if (sh.tile == 0 && sh.w == 16) return launch_march_x<T, M, VC, NWY, narrow_rows<T>(), XSHIFT, 16>(a, st);
     switch (sh.tile) {
     case 0: break;
     case 1: return launch_boxes<T, M, VC, 1>(a, st);

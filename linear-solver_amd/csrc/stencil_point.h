@@ -74,7 +74,8 @@ template <typename T> __host__ __device__ constexpr int tile_x(int lz) { return 
 //   take them once.  With the tiles at the end of a row point by point (20
 //   accesses for 5), an iteration of the mixed solve took 84 us at 193 x 189 x 196
 //   against 57, the FP32 operator 454 against 274 at 449 x 445 x 452.
-// * XPOINT (narrower grids): point by point, a wrapped offset each.
+// * XPOINT (narrower grids, down to which the march narrows its columns first:
+//   march_width): point by point, a wrapped offset each.
 // * XWIDE: the same with 64-bit byte offsets, for the planes of wide_plane().
 enum : int { XVEC = 0, XSHIFT = 1, XPOINT = 2, XWIDE = 3 };
 
@@ -129,6 +130,7 @@ __device__ __forceinline__ typename Lane<T>::Vec ld_vec(const T *base, const VOf
     return r;
 }
 
+// How tiles w wide take the vectors of a grid
 template <typename T> __host__ __device__ inline int x_mode(int nx, int ny, int w)
 {
     using L = Lane<T>;

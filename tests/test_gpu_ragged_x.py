@@ -1,6 +1,7 @@
 """Sweeps on x-sides that are not a multiple of a 16-byte vector: tiles that start
 early so that no vector wraps inside (sides from a tile and its halo up), the
-tile before the last one where its halo would, and narrower grids point by point.
+tile before the last one where its halo would, and narrower grids, in FP32 vectors
+of two parts, else point by point.
 Every point is written, and the norms count it once."""
 import numpy as np
 import pytest
@@ -13,7 +14,7 @@ pytestmark = pytest.mark.gpu
 
 # around 32 + 6 and 64 + 6 (FP64 boxes and march), 64 + 8 (FP32), and every
 # distance of the last tile's end from nx at which the tile before it moves
-SIDES = [37, 39, 69, 70, 71, 73, 74, 75, 77, 97, 99, 101, 103, 129, 130, 131, 133, 135, 137, 193, 195, 199]
+SIDES = [1, 3, 5, 6, 7, 9, 37, 39, 62, 65, 67, 69, 70, 71, 73, 74, 75, 77, 97, 99, 101, 103, 129, 130, 131, 133, 135, 137, 193, 195, 199]
 # boxes of 1, 2 and 4 planes, and the march
 FORMS = [((9, 7), None), ((40, 60), None), ((70, 90), None), ((35, 19), (9, 8, 4)), ((18, 19), (5, 4, 4))]
 
@@ -37,7 +38,7 @@ def test_operator(gpu, nx):
         assert np.max(np.abs(y32 - yo)) <= 40 * 2.0 ** -23 * 4.0 * 10.0 * np.max(np.abs(x))
 
 
-@pytest.mark.parametrize("nx", [37, 69, 73, 74, 75, 99, 130, 133, 135, 199])
+@pytest.mark.parametrize("nx", [5, 7, 37, 66, 69, 73, 74, 75, 99, 130, 133, 135, 199])
 @pytest.mark.parametrize("form", range(len(FORMS)))
 def test_recurrence_and_norms(gpu, oracle, nx, form):
     """Six iterations with two Anderson steps of AAR, constant coefficient and
