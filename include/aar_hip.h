@@ -328,10 +328,11 @@ int aar_hip_set_tuning(int lz, int wy, int py);
  * nz grid (fp32 = 1: the FP32 sweep of the mixed solver) over the launch
  * shapes (wy, py) and z-slab depths lz and keeps the fastest for that grid;
  * later solves on the grid use it.  batch_shape = 1 tunes only lz for the
- * batched launch (aar_hip_aar_batch).  Up to 8.5 million points the one-shot
- * boxes are timed too and used when they are faster; the shape returned stays
- * the best z-march.  Returns the shape and its time per sweep in us.
- * Allocates two temporary vectors of the grid. */
+ * batched launch (aar_hip_aar_batch).  Where the automatic choice is the
+ * one-shot boxes (grids of up to 5.6 to 8.5 million points) they are timed too
+ * and used when they are faster; the shape returned stays the best z-march.
+ * Returns the shape and its time per sweep in us.  Allocates two temporary
+ * vectors of the grid. */
 int aar_hip_autotune(int nx, int ny, int nz, int fp32, int batch_shape, int *lz, int *wy, int *py, double *us);
 
 /* Tuning options of the history sweeps (apply to subsequent solves):

@@ -63,13 +63,27 @@ int march_width(int nx, int ny)
     return TX;
 }
 
-// Where the boxes are faster than the march (recurrence sweep; FP64 with a
-// one-vector update, microseconds, march of 64 x 16 columns against boxes):
-// FP64 48^3 20.1 / 9.5, 96^3 24.4 / 15.4, 128^3 30.3 / 26.3, 160^3 43.9 / 44.3,
-// 200 x 161 x 150 56.2 / 57.4, 200^3 86.3 / 88.6, 256^3 (sweep alone) 67 / 103;
-// FP32 (sweep alone) 48^3 7.9 / 4.9, 96^3 9.5 / 8.3, 160^3 17.4 / 16.3, 200^3
-// 29.6 / 28.8, 256^3 41 / 50.  The two meet at about 8 million points; near the
-// tie the boxes need no depth chosen to fit.  FP32 boxes that go point
+// Where the boxes are faster than the march (microseconds, march / boxes, nx a
+// multiple of 4 and one more):
+//                   recurrence                   true residual  PGR step
+//   FP64 114^3      34.1 / 16.6   34.2 / 16.9    40.7 / 17.8    41.6 / 18.4
+//        160^3      35.0 / 25.8   36.3 / 30.6    40.9 / 29.2    43.4 / 31.2
+//        200x161x150 37.4 / 35.3                 43.6 / 40.0    47.7 / 44.4
+//        172x171x171 38.0 / 34.7  (171) 38.5 / 35.4  44.5 / 41.5  48.1 / 44.2
+//        182^3      38.3 / 40.1   38.1 / 40.9    47.3 / 48.9    49.8 / 55.1
+//        192^3      39.8 / 44.5   44.1 / 48.7    47.5 / 50.9    51.0 / 56.7
+//        204x203x204 47.7 / 55.7  48.9 / 56.6    60.4 / 66.3    67.3 / 76.2
+//   FP32 160^3      22.9 / 17.2   24.1 / 18.2
+//        192^3      25.1 / 22.5   28.8 / 26.5
+//        204x203x204 31.8 / 28.9  32.4 / 29.1
+// The operator alone, CG's sweeps and the ones with c(x) cross at the same
+// sizes: FP64 between 5.5 and 6.0 million points (CG at 176^3, 5.5 million, 99 us an
+// iteration with the boxes, 103 with the march), FP32 above 8.4 million (256^3,
+// sweep alone, 41 / 50).  FP64 grids whose sides leave more than a quarter more
+// of the march's 64 x 32 columns idle than of the 32 x 16 boxes keep the boxes
+// up to there (recurrence: 1.33 times the lanes 300 x 40 x 520 43.6 / 40.3, 80 x
+// 300 x 300 49.7 / 43.1, twice 28 x 500 x 500 56.7 / 40.5; 1.28 times 130 x 230 x
+// 230 47.6 / 46.2; 1.2 times 160 x 214 x 214 41.6 / 44.9).  FP32 boxes that go point
 // by point (x_mode) give way to the march in narrow columns earlier: from 2.4
 // million lanes of their 64-wide tiles (61 x 200 x 200, 2.6 million lanes, 20.5 /
 // 22.4; 65 x 140 x 140, 2.5, 20.5 / 22.2; 61 x 140 x 140, 1.3, 20.1 / 17.3), from 4.5
@@ -85,9 +99,11 @@ int stencil_tile_planes(int nx, int ny, int nz)
 {
     const long n = (long)nx * ny * nz;
     if (n > 8500000L) return 0;
+    auto lanes = [&](int w, int rows) { return (long)((nx + w - 1) / w * w) * ((ny + rows - 1) / rows * rows); };
     const int mw = march_width<T>(nx, ny);
-    const long lanes = (long)((nx + TX - 1) / TX * TX) * ny * nz;
-    if (sizeof(T) == 4 && mw < TX && lanes > (mw == 32 ? 2400000L : 4500000L)) return 0;
+    const bool idle = 4 * lanes(mw, narrow_rows<T>() * TX / mw) > 5 * lanes(tile_x<T>(4), tile_rows<T>(4));
+    if (sizeof(T) == 8 && !idle && n > 5600000L) return 0;
+    if (sizeof(T) == 4 && mw < TX && lanes(TX, 1) * nz > (mw == 32 ? 2400000L : 4500000L)) return 0;
     auto cols = [&](int lz) {
         return (long)((nx + tile_x<T>(lz) - 1) / tile_x<T>(lz)) * ((ny + tile_rows<T>(lz) - 1) / tile_rows<T>(lz));
     };
