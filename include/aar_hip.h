@@ -354,7 +354,10 @@ int aar_hip_set_option(const char *name, long value);
 /* Per-kernel GPU timing with hipEvents (off by default).  Kernel names:
  * "stencil_matvec", "stencil_aar_true", "stencil_aar_rec", "stencil_resid",
  * "stencil_pgr_rich", "stencil_cg_q", "stencil_cg_resid",
- * "gram", "ls", "anchor_update", "fold", "dot", "pgr_update", "cg_dir", "cg_update". */
+ * "gram", "ls", "anchor_update", "fold", "dot", "pgr_update", "cg_dir", "cg_update".
+ * "ls" covers the final sum of the Gram's block partials and the m x m solve
+ * (one launch); "gram" the products alone.  A sweep's norm is finished outside
+ * its entry. */
 int aar_hip_profile(int enable);
 int aar_hip_profile_reset(void);
 int aar_hip_profile_query(const char *name, int *count, double *total_ms, double *bytes);

@@ -329,8 +329,9 @@ hipError_t launch_helm_grad_c(long n, const double2 *lambda, const double2 *u, d
 
 // Reducing kernels run the finaliser in their last block when given a
 // counter, or only write per-block partials when counter == nullptr; then
-// launch_finish (or, for the Gram, launch_gram itself) runs a one-block
-// second pass.
+// launch_finish runs a one-block second pass.  The Gram's second pass is
+// launch_gram_solve (ctrl->G holds nothing before it), the complex Gram's
+// launch_hgram_solve.
 //
 // A residual norm that is only recorded needs no finish of its own: the sweeps
 // between two checks leave their partials in consecutive sets, and the finish

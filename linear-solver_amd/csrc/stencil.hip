@@ -10,7 +10,8 @@
 // Two forms of the sweep share the point formulas (stencil_point.h):
 //
 // The march (stencil_body.h), for grids that fill the chip: a block of WY
-// wavefronts owns a 64 x TY column of the grid over a z-chunk of `lz` planes
+// wavefronts owns a column of 64 (narrow grids 32 or 16: march_width) x TY
+// points over a z-chunk of `lz` planes
 // and marches it in z.
 // * z-neighbours come from a per-thread register queue of 13 planes, so
 //   every plane of the column is read from HBM once per chunk;
